@@ -483,6 +483,52 @@ int wbfmm_hip_hel_shift_mfma(int mode, const uint32_t *parents, unsigned npar,
                              const uint32_t *cflag, int N, const double *in, double *out,
                              const void *plan_dev, const double *A, const double *A2,
                              const double *CS, const wbfmm_m2l_plan_t *plan_host);
+/* The same translations with the order as a run-time value, for orders the
+   kernels above do not serve and for levels of two different orders: N =
+   max(Nin, Nout) in 2..40.  P (part 0: rows m = 0..n) and Q (part 1: m =
+   1..n) are apart; the blocks of a part have the sizes 1..N+1 (part 0) or
+   1..N (part 1), one of each size, in the rotations (degree n) as in the
+   coaxial stage (order m), and the block of a size has the same slots in
+   both.  Row tiles t of a part: tile[t] = first input slot, k-steps, first
+   k-step in the tables; wavefront w of 16 runs wbeg[w]..wbeg[w+1].  map1,
+   map2, map3: slot of a tile's row after stages 1, 2 and 3 (after stage 3
+   the unit n(n+1)/2 + nu), -1 for an unused row; s1: slots of a unit as
+   the input of stage 1. */
+#define WBFMM_HEL_WIDE_MAXN 40
+#define WBFMM_HEL_WIDE_MAXT 80
+#define WBFMM_HEL_WIDE_MAXU 861
+typedef struct {
+  int N, NU, KT, NTH, NR;
+  int nt[2], wbeg[2][17];
+  int tile[2][WBFMM_HEL_WIDE_MAXT][4];
+  int map1[2][16 * WBFMM_HEL_WIDE_MAXT], map2[2][16 * WBFMM_HEL_WIDE_MAXT],
+      map3[2][16 * WBFMM_HEL_WIDE_MAXT];
+  int s1[2][WBFMM_HEL_WIDE_MAXU];
+  int th[343], rix[343];
+  double chi[343], rr[32];
+} wbfmm_hel_wide_plan_t;
+/* host: the plan of order N; the rotation tiles at nth polar angles (A: nth
+   x KT x 64 doubles; ths NULL: the plan's NTH offset angles); the coaxial
+   tiles of nr tables E of order L >= N (A2: nr x 2 x KT x 64, real and
+   imaginary part of each) */
+int wbfmm_hip_hel_wide_plan(int N, wbfmm_hel_wide_plan_t *plan);
+int wbfmm_hip_hel_wide_rot(const wbfmm_hel_wide_plan_t *plan, int nth, const double *ths,
+                           double *A);
+int wbfmm_hip_hel_wide_coax(const wbfmm_hel_wide_plan_t *plan, int L, int nr, const double *E,
+                            double *A2);
+/* M2L (as wbfmm_hip_hel_m2l_mfma; CS: 343 x (N+1) x 2, cos and sin of m
+   chi) and M2M / L2L (as wbfmm_hip_hel_shift_mfma; CS: 8 x (N+1) x 2) */
+int wbfmm_hip_hel_wide_m2l(const uint32_t *cls, const unsigned *cstart, const unsigned *ccount,
+                           const uint32_t *sstart, const uint32_t *send, unsigned level, int Ns,
+                           int Nr, const double *mps, double *mpr, const void *plan_dev,
+                           const double *A, const double *A2, const double *CS,
+                           const wbfmm_hel_wide_plan_t *plan_host);
+int wbfmm_hip_hel_wide_shift(int mode, const uint32_t *parents, unsigned npar,
+                             const uint32_t *cstart, const uint32_t *cend,
+                             const uint32_t *cflag, int Nin, int Nout, const double *in,
+                             double *out, const void *plan_dev, const double *A,
+                             const double *A2, const double *CS,
+                             const wbfmm_hel_wide_plan_t *plan_host);
 /* M2L for the listed target boxes, accumulating into mpr; Hth: H tables
    of the offset polar angles; th_idx/chi/rix: per-slot geometry (device);
    SR: one S|R table of ne complex entries per offset length

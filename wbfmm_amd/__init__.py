@@ -156,6 +156,9 @@ _SIGS = {
     "wbfmm_hip_hel_m2l_rot_tiles": (_i, [_vp, _vp]),
     "wbfmm_hip_hel_rot_tiles": (_i, [_vp, _i, _vp, _vp]),
     "wbfmm_hip_hel_m2l_coax_tiles": (_i, [_vp, _i, _i, _vp, _vp]),
+    "wbfmm_hip_hel_wide_plan": (_i, [_i, _vp]),
+    "wbfmm_hip_hel_wide_rot": (_i, [_vp, _i, _vp, _vp]),
+    "wbfmm_hip_hel_wide_coax": (_i, [_vp, _i, _i, _vp, _vp]),
     "wbfmm_tree_coefficient_init": (_i, [_vp, _u, _u, _u]),
     "wbfmm_tree_leaf_expansions": (_i, [_vp, _d, _vp, _i, _vp, _i, _i, _vp]),
     "wbfmm_shift_operators_coaxial_SR_init": (_i, [_vp, _d, _u, _u, _d, _vp]),

@@ -21,7 +21,7 @@ LIB = os.path.join(HERE, "libwbfmm.so")
 HIP_SOURCES = [
     # the Helmholtz and Laplace matrix-core kernels, one range of orders per unit
     "hel_m2l_o26_27.hip", "hel_m2l_o24_25.hip", "hel_m2l_o22_23.hip", "hel_m2l_o19_21.hip",
-    "m2l_lap_o22_24.hip", "m2l_lap_o19_21.hip", "m2l_lap_o16_18.hip", "hel_m2l_o15_18.hip",
+    "hel_wide.hip", "m2l_lap_o22_24.hip", "m2l_lap_o19_21.hip", "m2l_lap_o16_18.hip", "hel_m2l_o15_18.hip",
     "m2l_lap_o13_15.hip", "m2l_lap_o11_12.hip", "m2l_lap_o08_10.hip", "hel_m2l_o10_14.hip",
     "m2l_lap_o02_07.hip", "hel_m2l_o02_09.hip",
     "helmholtz.hip", "laplace.hip", "m2l_mfma.hip", "hel_m2l_mfma.hip", "runtime.hip",

@@ -211,6 +211,17 @@ typedef struct {
   double *ss_host[WBFMM_TREE_MAX_DEPTH + 1];
   double *hel_SS2[WBFMM_TREE_MAX_DEPTH + 1];
   int hel_SS2_N[WBFMM_TREE_MAX_DEPTH + 1];
+  /* Helmholtz passes with run-time orders (wbfmm_hip_hel_wide_*): plan,
+     rotation tiles of the offset and child angles and phases per order
+     (shared by the process), coaxial tiles per level with the order they
+     were made for */
+  wbfmm_hel_wide_plan_t *wide_plan[WBFMM_HIP_MAX_ORDER + 1];
+  void *wide_plan_dev[WBFMM_HIP_MAX_ORDER + 1];
+  double *wide_A[WBFMM_HIP_MAX_ORDER + 1], *wide_shA[WBFMM_HIP_MAX_ORDER + 1];
+  double *wide_CS[WBFMM_HIP_MAX_ORDER + 1], *wide_CSup[WBFMM_HIP_MAX_ORDER + 1],
+      *wide_CSdn[WBFMM_HIP_MAX_ORDER + 1];
+  double *wide_SR[WBFMM_TREE_MAX_DEPTH + 1], *wide_SS[WBFMM_TREE_MAX_DEPTH + 1];
+  int wide_SR_N[WBFMM_TREE_MAX_DEPTH + 1], wide_SS_N[WBFMM_TREE_MAX_DEPTH + 1];
   /* mixed-precision Helmholtz: FP32 rotation tiles and phases per order,
      and per level the scaled FP32 coaxial tiles of the M2L and of the
      M2M into / L2L from the level above, with the order and wavenumber
@@ -1012,6 +1023,8 @@ gint wbfmm_shift_operators_free(wbfmm_shift_operators_t *op)
     free(od->sr_host[n]);
     wbfmm_hip_free(od->hel_SS2[n]);
     free(od->ss_host[n]);
+    wbfmm_hip_free(od->wide_SR[n]);
+    wbfmm_hip_free(od->wide_SS[n]);
     wbfmm_hip_free(od->f_hA2[n]);
     wbfmm_hip_free(od->f_hUp[n]);
     wbfmm_hip_free(od->f_hDn[n]);
@@ -2132,6 +2145,8 @@ gint wbfmm_shift_operators_coaxial_SR_init(wbfmm_shift_operators_t *w, gdouble D
   od->sr_nr = nr;
   wbfmm_hip_free(od->hel_A2[level]);
   od->hel_A2[level] = NULL;
+  wbfmm_hip_free(od->wide_SR[level]);
+  od->wide_SR[level] = NULL;
   w->L[level] = L;
   return 0;
 }
@@ -2160,6 +2175,8 @@ gint wbfmm_shift_operators_coaxial_SS_init(wbfmm_shift_operators_t *w, gdouble D
   od->ss_host[level] = h;
   wbfmm_hip_free(od->hel_SS2[level]);
   od->hel_SS2[level] = NULL;
+  wbfmm_hip_free(od->wide_SS[level]);
+  od->wide_SS[level] = NULL;
   od->ss_L[level] = L;
   return 0;
 }
@@ -2186,6 +2203,9 @@ gint wbfmm_shift_operators_coaxial_reset(wbfmm_shift_operators_t *w)
     wbfmm_hip_free(od->f_hUp[n]);
     wbfmm_hip_free(od->f_hDn[n]);
     od->f_hA2[n] = od->f_hUp[n] = od->f_hDn[n] = NULL;
+    wbfmm_hip_free(od->wide_SR[n]);
+    wbfmm_hip_free(od->wide_SS[n]);
+    od->wide_SR[n] = od->wide_SS[n] = NULL;
   }
   od->hel_k_set = 0;
   return 0;
@@ -2246,6 +2266,9 @@ static void ensure_hel_rotations(ops_dev *od)
 }
 
 static int hel_shift_mfma(ops_dev *od, guint Nc, guint Np);
+static int hel_wide_serves(guint Na, guint Nb);
+static void ensure_wide_plan(ops_dev *od, int N);
+static const double *wide_coax(ops_dev *od, guint level, int N, int shift);
 static void ensure_hel_shift_rot_tiles(ops_dev *od, int N);
 static void ensure_hel_shift_coax_tiles(ops_dev *od, guint level, int N);
 
@@ -2265,6 +2288,16 @@ static void hel_m2m64(wbfmm_tree_t *t, ops_dev *od, guint level, const double *s
                                    td->d_start[level], td->d_end[level], NULL, N, src, dst,
                                    od->m2l_plan_dev[N], od->hel_shA[N], od->hel_SS2[level],
                                    od->sh_CSup[N], od->m2l_plan[N]));
+    return;
+  }
+  if (hel_wide_serves(Nc, Np)) {
+    int N = (int)(Nc > Np ? Nc : Np);
+    ensure_wide_plan(od, N);
+    HIPOK(wbfmm_hip_hel_wide_shift(0, td->d_occ[level - 1], td->nocc[level - 1],
+                                   td->d_start[level], td->d_end[level], NULL, (int)Nc, (int)Np,
+                                   src, dst, od->wide_plan_dev[N], od->wide_shA[N],
+                                   wide_coax(od, level, N, 1), od->wide_CSup[N],
+                                   od->wide_plan[N]));
     return;
   }
   ensure_hel_rotations(od);
@@ -2412,6 +2445,130 @@ static int hel_shift_mfma(ops_dev *od, guint Nc, guint Np)
   return Nc == Np && (int)Nc >= M2L_MFMA_MIN && (int)Nc <= HEL_MFMA_MAX && hel_mfma_enabled();
 }
 
+/* orders Na, Nb of the two sides of a translation that the run-time-order
+   matrix-core passes take: different orders, and equal ones above those of
+   the per-order kernels, which serve equal orders better where they fit
+   (M2L of a 1e5-point sphere at orders 25/23: 7.7 against 16.8 ms).  The
+   vector kernels they replace: 3e4-point cube, order 30, M2L 63.8 -> 3.6,
+   M2M 2.0 -> 0.06, L2L 2.0 -> 0.07 ms; M2M 23 -> 25 and L2L 25 -> 23 on
+   the sphere 1.05 -> 0.30 and 1.08 -> 0.36 ms */
+static int hel_wide_serves(guint Na, guint Nb)
+{
+  const guint N = Na > Nb ? Na : Nb;
+  return (Na != Nb || (int)N > HEL_MFMA_MAX) && N >= 2 && N <= WBFMM_HEL_WIDE_MAXN &&
+         hel_mfma_enabled();
+}
+
+static double *dev_copy(const void *h, size_t bytes)
+{
+  void *d = NULL;
+  HIPOK(wbfmm_hip_malloc(&d, bytes));
+  HIPOK(wbfmm_hip_memcpy(d, h, bytes));
+  return d;
+}
+
+/* plan, child rotation tiles and phases of order N, built once per process */
+static void ensure_wide_plan(ops_dev *od, int N)
+{
+  if (od->wide_plan[N]) return;
+  mu_lock(&g_ord_mu[N]);
+  if (!g_tab.wide_plan[N]) {
+    wbfmm_hel_wide_plan_t *P = calloc(1, sizeof(*P));
+    const size_t na = (size_t)343 * (N + 1) * 2, nc = (size_t)8 * (N + 1) * 2;
+    double ths[2] = {acos(1.0 / sqrt(3.0)), acos(-1.0 / sqrt(3.0))}, *A, *CS, *up, *dn;
+    int i, m;
+    if (!P) WBFMM_FATAL("out of host memory");
+    HIPOK(wbfmm_hip_hel_wide_plan(N, P));
+    A = malloc(sizeof(double) * 2 * P->KT * 64);
+    CS = malloc(sizeof(double) * na);
+    up = malloc(sizeof(double) * nc);
+    dn = malloc(sizeof(double) * nc);
+    if (!A || !CS || !up || !dn) WBFMM_FATAL("out of host memory");
+    HIPOK(wbfmm_hip_hel_wide_rot(P, 2, ths, A));
+    for (i = 0; i < 343; i++)
+      for (m = 0; m <= N; m++) {
+        CS[((size_t)i * (N + 1) + m) * 2] = cos(m * P->chi[i]);
+        CS[((size_t)i * (N + 1) + m) * 2 + 1] = sin(m * P->chi[i]);
+      }
+    /* azimuths of child -> parent (M2M) and parent -> child (L2L) */
+    for (i = 0; i < 8; i++) {
+      const double ex = 0.5 - (i & 1), ey = 0.5 - ((i >> 1) & 1);
+      const double cu = atan2(ey, ex), cd = atan2(-ey, -ex);
+      for (m = 0; m <= N; m++) {
+        up[((size_t)i * (N + 1) + m) * 2] = cos(m * cu);
+        up[((size_t)i * (N + 1) + m) * 2 + 1] = sin(m * cu);
+        dn[((size_t)i * (N + 1) + m) * 2] = cos(m * cd);
+        dn[((size_t)i * (N + 1) + m) * 2 + 1] = sin(m * cd);
+      }
+    }
+    g_tab.wide_plan_dev[N] = dev_copy(P, sizeof(*P));
+    g_tab.wide_shA[N] = dev_copy(A, sizeof(double) * 2 * P->KT * 64);
+    g_tab.wide_CS[N] = dev_copy(CS, sizeof(double) * na);
+    g_tab.wide_CSup[N] = dev_copy(up, sizeof(double) * nc);
+    g_tab.wide_CSdn[N] = dev_copy(dn, sizeof(double) * nc);
+    g_tab.wide_plan[N] = P;
+    free(A);
+    free(CS);
+    free(up);
+    free(dn);
+  }
+  od->wide_plan_dev[N] = g_tab.wide_plan_dev[N];
+  od->wide_shA[N] = g_tab.wide_shA[N];
+  od->wide_CS[N] = g_tab.wide_CS[N];
+  od->wide_CSup[N] = g_tab.wide_CSup[N];
+  od->wide_CSdn[N] = g_tab.wide_CSdn[N];
+  od->wide_plan[N] = g_tab.wide_plan[N];
+  mu_unlock(&g_ord_mu[N]);
+}
+
+/* rotation tiles of the offset angles for order N, built once per process
+   (after ensure_wide_plan) */
+static void ensure_wide_rot(ops_dev *od, int N)
+{
+  if (od->wide_A[N]) return;
+  mu_lock(&g_ord_mu[N]);
+  if (!g_tab.wide_A[N]) {
+    const wbfmm_hel_wide_plan_t *P = od->wide_plan[N];
+    const size_t n = (size_t)P->NTH * P->KT * 64;
+    double *h = malloc(sizeof(double) * n);
+    if (!h) WBFMM_FATAL("out of host memory");
+    HIPOK(wbfmm_hip_hel_wide_rot(P, P->NTH, NULL, h));
+    g_tab.wide_A[N] = dev_copy(h, sizeof(double) * n);
+    free(h);
+  }
+  od->wide_A[N] = g_tab.wide_A[N];
+  mu_unlock(&g_ord_mu[N]);
+}
+
+/* coaxial tiles of `level' for order N: S|R at the offset lengths (M2L) or
+   R|R between the level and its parents (shift) */
+static const double *wide_coax(ops_dev *od, guint level, int N, int shift)
+{
+  const wbfmm_hel_wide_plan_t *P = od->wide_plan[N];
+  double **slot = shift ? &od->wide_SS[level] : &od->wide_SR[level], *h;
+  int *have = shift ? &od->wide_SS_N[level] : &od->wide_SR_N[level], i;
+  const double *E = shift ? od->ss_host[level] : od->sr_host[level];
+  const int nr = shift ? 1 : P->NR;
+  const size_t n = (size_t)nr * 2 * P->KT * 64;
+  if (*slot && *have == N) return *slot;
+  if (!E) WBFMM_FATAL("coaxial operators not initialised at level %u", level);
+  if (!shift) {
+    /* both follow wbfmm_hip_offset_geometry */
+    if (od->sr_nr != nr) WBFMM_FATAL("%d offset lengths, the plan has %d", od->sr_nr, nr);
+    for (i = 0; i < nr; i++)
+      if (od->sr_rr[i] != P->rr[i]) WBFMM_FATAL("offset length %g not in the S|R tables", P->rr[i]);
+  }
+  h = malloc(sizeof(double) * n);
+  if (!h) WBFMM_FATAL("out of host memory");
+  HIPOK(wbfmm_hip_hel_wide_coax(P, shift ? (int)od->ss_L[level] : (int)od->op.L[level], nr, E, h));
+  wbfmm_hip_free(*slot);
+  *slot = NULL;
+  *slot = dev_copy(h, sizeof(double) * n);
+  *have = N;
+  free(h);
+  return *slot;
+}
+
 /* FP64 M2L at `level' for the nt target boxes tl */
 static void hel_m2l64(wbfmm_tree_t *t, ops_dev *od, guint level, const uint32_t *tl, unsigned nt)
 {
@@ -2433,6 +2590,19 @@ static void hel_m2l64(wbfmm_tree_t *t, ops_dev *od, guint level, const uint32_t 
                                  level, N, (double *)t->mps[level], (double *)t->mpr[level],
                                  od->m2l_plan_dev[N], od->hel_A[N], od->hel_A2[level],
                                  od->m2l_CS[N], od->m2l_plan[N]));
+    wbfmm_hip_free(cls);
+  } else if (hel_wide_serves(Ns, Nr) && level <= M2L_MFMA_MAX_LEVEL) {
+    int N = (int)(Ns > Nr ? Ns : Nr);
+    unsigned cstart[8], ccount[8];
+    uint32_t *cls;
+    ensure_wide_plan(od, N);
+    ensure_wide_rot(od, N);
+    HIPOK(wbfmm_hip_malloc((void **)&cls, sizeof(uint32_t) * (nt ? nt : 1)));
+    HIPOK(wbfmm_hip_split_classes(tl, nt, cls, cstart, ccount));
+    HIPOK(wbfmm_hip_hel_wide_m2l(cls, cstart, ccount, td->d_start[level], td->d_end[level],
+                                 level, (int)Ns, (int)Nr, (double *)t->mps[level],
+                                 (double *)t->mpr[level], od->wide_plan_dev[N], od->wide_A[N],
+                                 wide_coax(od, level, N, 0), od->wide_CS[N], od->wide_plan[N]));
     wbfmm_hip_free(cls);
   } else {
     ensure_hel_rotations(od); /* the vector kernels' H tables, on first use */
@@ -2459,6 +2629,14 @@ static void hel_l2l64(wbfmm_tree_t *t, ops_dev *od, guint level, const uint32_t 
                                    td->have_targets ? td->d_flag[level + 1] : NULL, N, src, dst,
                                    od->m2l_plan_dev[N], od->hel_shA[N], od->hel_SS2[level + 1],
                                    od->sh_CSdn[N], od->m2l_plan[N]));
+  } else if (hel_wide_serves(Nr, Nc)) {
+    int N = (int)(Nr > Nc ? Nr : Nc);
+    ensure_wide_plan(od, N);
+    HIPOK(wbfmm_hip_hel_wide_shift(1, tl, nt, NULL, NULL,
+                                   td->have_targets ? td->d_flag[level + 1] : NULL, (int)Nr,
+                                   (int)Nc, src, dst, od->wide_plan_dev[N], od->wide_shA[N],
+                                   wide_coax(od, level + 1, N, 1), od->wide_CSdn[N],
+                                   od->wide_plan[N]));
   } else {
     ensure_hel_rotations(od);
     HIPOK(wbfmm_hip_hel_l2l(tl, nt, td->have_targets ? td->d_flag[level + 1] : NULL, (int)Nr,

@@ -1088,3 +1088,214 @@ int wbfmm_hip_hel_coax_tiles_scaled(const wbfmm_m2l_plan_t *P, int L, int nr, co
   free(T);
   return 0;
 }
+
+/* ------------------------------------------------------------------
+ * Plan and tiles of the run-time-order Helmholtz translations (see
+ * wbfmm_hip.h): P and Q apart, blocks without padding rows.
+ * ------------------------------------------------------------------ */
+
+/* first slot of the block of size sz of part pt, sizes descending */
+static int wide_base(int N, int pt, int sz)
+{
+  int top = pt ? N : N + 1;               /* the largest size */
+  return (top - sz) * (top + sz + 1) / 2;  /* top + (top-1) + .. + (sz+1) */
+}
+
+/* the row tiles of a part: a block of more than 16 rows in tiles of its
+   own over all its columns; the smaller blocks, consecutive ones together
+   while they fit 16 rows.  Dealt to the 16 wavefronts in order of their
+   k-steps, back and forth. */
+static int wide_tiles(int N, int pt, wbfmm_hel_wide_plan_t *P, int rowbase[], int nrow[],
+                      int klen[])
+{
+  int top = pt ? N : N + 1, sz, nt = 0, t, w, ord[WBFMM_HEL_WIDE_MAXT];
+  int kb[WBFMM_HEL_WIDE_MAXT], rb[WBFMM_HEL_WIDE_MAXT], nr[WBFMM_HEL_WIDE_MAXT],
+      kl[WBFMM_HEL_WIDE_MAXT], koff;
+  for (sz = top; sz >= 1;) {
+    const int b = wide_base(N, pt, sz);
+    if (sz > 16) {
+      for (t = 0; t < sz; t += 16) {
+        if (nt == WBFMM_HEL_WIDE_MAXT) return -1;
+        kb[nt] = b;
+        kl[nt] = sz;
+        rb[nt] = b + t;
+        nr[nt++] = sz - t < 16 ? sz - t : 16;
+      }
+      sz--;
+    } else {
+      int fill = 0;
+      while (sz >= 1 && fill + sz <= 16) fill += sz--;
+      if (nt == WBFMM_HEL_WIDE_MAXT) return -1;
+      kb[nt] = rb[nt] = b;
+      kl[nt] = nr[nt] = fill;
+      nt++;
+    }
+  }
+  /* longest first (stable) */
+  for (t = 0; t < nt; t++) {
+    int i = t;
+    for (; i > 0 && kl[ord[i - 1]] < kl[t]; i--) ord[i] = ord[i - 1];
+    ord[i] = t;
+  }
+  koff = pt ? P->KT : 0;
+  P->nt[pt] = 0;
+  for (w = 0; w < 16; w++) {
+    P->wbeg[pt][w] = P->nt[pt];
+    for (t = 0; 16 * t < nt; t++) {
+      const int i = 16 * t + ((t & 1) ? 15 - w : w), n = P->nt[pt];
+      if (i >= nt) continue;
+      P->tile[pt][n][0] = kb[ord[i]];
+      P->tile[pt][n][1] = (kl[ord[i]] + 3) / 4;
+      P->tile[pt][n][2] = koff;
+      koff += P->tile[pt][n][1];
+      rowbase[n] = rb[ord[i]];
+      nrow[n] = nr[ord[i]];
+      klen[n] = kl[ord[i]];
+      P->nt[pt]++;
+    }
+  }
+  P->wbeg[pt][16] = P->nt[pt];
+  P->KT = koff;
+  return 0;
+}
+
+/* block size and index within the block of a slot of part pt */
+static void wide_slot(int N, int pt, int slot, int *sz, int *idx)
+{
+  int s = pt ? N : N + 1;
+  while (slot >= s) slot -= s--;
+  *sz = s;
+  *idx = slot;
+}
+
+int wbfmm_hip_hel_wide_plan(int N, wbfmm_hel_wide_plan_t *P)
+{
+  int pt, t, r, n, m, rowbase[WBFMM_HEL_WIDE_MAXT], nrow[WBFMM_HEL_WIDE_MAXT],
+      klen[WBFMM_HEL_WIDE_MAXT];
+  double ths[64];
+  if (N < 2 || N > WBFMM_HEL_WIDE_MAXN) return WBFMM_HIP_ERR_ORDER;
+  memset(P, 0, sizeof(*P));
+  P->N = N;
+  P->NU = (N + 1) * (N + 2) / 2;
+  for (pt = 0; pt < 2; pt++) {
+    if (wide_tiles(N, pt, P, rowbase, nrow, klen)) return WBFMM_HIP_ERR_ORDER;
+    for (t = 0; t < P->nt[pt]; t++)
+      for (r = 0; r < 16; r++) {
+        int sz, idx, nn, nu, mm;
+        P->map1[pt][16 * t + r] = P->map2[pt][16 * t + r] = P->map3[pt][16 * t + r] = -1;
+        if (r >= nrow[t]) continue;
+        wide_slot(N, pt, rowbase[t] + r, &sz, &idx);
+        /* as a row of a rotation: degree nn, order nu */
+        nn = pt ? sz : sz - 1;
+        nu = idx + pt;
+        P->map1[pt][16 * t + r] = wide_base(N, pt, N + 1 - nu) + nn - nu;
+        P->map3[pt][16 * t + r] = nn * (nn + 1) / 2 + nu;
+        /* as a row of the coaxial stage: order mm, degree mm + idx */
+        mm = N + 1 - sz;
+        nn = mm + idx;
+        P->map2[pt][16 * t + r] = wide_base(N, pt, pt ? nn : nn + 1) + mm - pt;
+      }
+  }
+  for (n = 0; n <= N; n++)
+    for (m = 0; m <= n; m++) {
+      P->s1[0][n * (n + 1) / 2 + m] = wide_base(N, 0, n + 1) + m;
+      P->s1[1][n * (n + 1) / 2 + m] = m ? wide_base(N, 1, n) + m - 1 : 0;
+    }
+  return wbfmm_hip_offset_geometry(ths, &P->NTH, P->th, P->chi, P->rr, &P->NR, P->rix);
+}
+
+/* the tiles of part pt with entry val(ctx, pt, size, row, column) */
+typedef double (*wide_entry)(const void *ctx, int pt, int sz, int row, int col);
+static void wide_fill(const wbfmm_hel_wide_plan_t *Q, wide_entry val, const void *ctx, double *A)
+{
+  wbfmm_hel_wide_plan_t P;
+  int pt, t, j, l, rowbase[WBFMM_HEL_WIDE_MAXT], nrow[WBFMM_HEL_WIDE_MAXT],
+      klen[WBFMM_HEL_WIDE_MAXT];
+  P.KT = 0;
+  for (pt = 0; pt < 2; pt++) {
+    wide_tiles(Q->N, pt, &P, rowbase, nrow, klen);
+    for (t = 0; t < P.nt[pt]; t++)
+      for (l = 0; l < 64; l++) {
+        int r = l % 16, sr = 0, ir = 0;
+        if (r < nrow[t]) wide_slot(Q->N, pt, rowbase[t] + r, &sr, &ir);
+        for (j = 0; j < P.tile[pt][t][1]; j++) {
+          int k = 4 * j + l / 16, sc = 0, ic = 0;
+          double v = 0.0;
+          if (r < nrow[t] && k < klen[t]) {
+            wide_slot(Q->N, pt, P.tile[pt][t][0] + k, &sc, &ic);
+            if (sc == sr) v = val(ctx, pt, sr, ir, ic);
+          }
+          A[((size_t)P.tile[pt][t][2] + j) * 64 + l] = v;
+        }
+      }
+  }
+}
+
+static double wide_rot_entry(const void *ctx, int pt, int sz, int row, int col)
+{
+  const double *H = ctx;
+  const int n = pt ? sz : sz - 1, nu = row + pt, m = col + pt;
+  if (pt) return H[RIDX(nu, m, n)] - H[RIDX(-nu, m, n)];
+  return m == 0 ? H[RIDX(nu, 0, n)] : H[RIDX(nu, m, n)] + H[RIDX(-nu, m, n)];
+}
+
+typedef struct {
+  const wbfmm_hel_wide_plan_t *P;
+  const double *ths;
+  double *A;
+  int rc;
+} wide_rot_job;
+
+static void wide_rot_one(int k, void *c)
+{
+  wide_rot_job *j = c;
+  double *H = malloc(sizeof(double) * rot_size(j->P->N));
+  if (!H) {
+    j->rc = WBFMM_HIP_ERR_NOMEM;
+    return;
+  }
+  H_rotation(H, j->P->N, j->ths[k]);
+  wide_fill(j->P, wide_rot_entry, H, j->A + (size_t)k * j->P->KT * 64);
+  free(H);
+}
+
+int wbfmm_hip_hel_wide_rot(const wbfmm_hel_wide_plan_t *P, int nth, const double *ths, double *A)
+{
+  wide_rot_job j = {P, ths, A, 0};
+  double own[64];
+  if (!ths) {
+    if (nth != P->NTH || plan_thetas(own) != nth) return WBFMM_HIP_ERR_ARG;
+    j.ths = own;
+  }
+  if (nth < 1) return WBFMM_HIP_ERR_ARG;
+  par_for(nth, wide_rot_one, &j);
+  return j.rc;
+}
+
+typedef struct {
+  int N;
+  const double *E; /* the table, offset to the wanted part */
+} wide_coax_ctx;
+
+static double wide_coax_entry(const void *ctx, int pt, int sz, int row, int col)
+{
+  const wide_coax_ctx *x = ctx;
+  const int m = x->N + 1 - sz, n = m + row, l = m + col;
+  const double v = x->E[2 * (l >= n ? CXI(l, m, n) : CXI(n, m, l))];
+  (void)pt;
+  return l < n && ((n + l) & 1) ? -v : v;
+}
+
+int wbfmm_hip_hel_wide_coax(const wbfmm_hel_wide_plan_t *P, int L, int nr, const double *E,
+                            double *A2)
+{
+  const size_t ne = CXI(L + 1, 0, 0), per = (size_t)P->KT * 64;
+  int i, c;
+  if (L < P->N) return WBFMM_HIP_ERR_ORDER;
+  for (i = 0; i < nr; i++)
+    for (c = 0; c < 2; c++) {
+      wide_coax_ctx x = {P->N, E + (size_t)i * 2 * ne + c};
+      wide_fill(P, wide_coax_entry, &x, A2 + (size_t)(2 * i + c) * per);
+    }
+  return 0;
+}
