@@ -154,7 +154,8 @@ struct RecTab {
   double rb[kRT][2 * kRT + 1];  // rec_b(i, m - kRT)
   double pa[kRT];               // sqrt(2 i + 1)
   double pb[kRT][kRT];          // sqrt((i^2 - m^2) / (2 i - 1))
-  double pd[kRT][kRT];          // sqrt(((i + 1)^2 - m^2) / (2 i + 3))
+  double pd[kRT][kRT];          // 1 / sqrt(((i + 1)^2 - m^2) / (2 i + 3))
+  double pc[kRT];               // sqrt((2 i + 1) / (2 i))
 };
 
 __global__ void k_rec_tab(RecTab *T) {
@@ -163,13 +164,16 @@ __global__ void k_rec_tab(RecTab *T) {
     const int i = t / kRT, m = t % kRT;
     T->ra[i][m] = rec_a(i - 1, m);
     T->pb[i][m] = sqrt((double)(i * i - m * m) / (2 * i - 1));
-    T->pd[i][m] = sqrt((double)((i + 1) * (i + 1) - m * m) / (2 * i + 3));
+    T->pd[i][m] = 1.0 / sqrt((double)((i + 1) * (i + 1) - m * m) / (2 * i + 3));
   }
   if (t < kRT * (2 * kRT + 1)) {
     const int i = t / (2 * kRT + 1), m = t % (2 * kRT + 1) - kRT;
     T->rb[i][m + kRT] = rec_b(i, m);
   }
-  if (t < kRT) T->pa[t] = sqrt(2.0 * t + 1);
+  if (t < kRT) {
+    T->pa[t] = sqrt(2.0 * t + 1);
+    T->pc[t] = t ? sqrt((2.0 * t + 1) / (2.0 * t)) : 1.0;
+  }
 }
 
 // rec_a(n, m) for n >= -1, |m| <= n + 1 <= WBFMM_HIP_MAX_ORDER + 1
@@ -184,7 +188,7 @@ __device__ __forceinline__ double tab_b(const RecTab *__restrict__ T, int n, int
 __device__ __forceinline__ double tab_pbar_up(const RecTab *__restrict__ T, int n, int m, double C,
                                               double pn, double pnm1) {
   const double v = C * T->pa[n] * pn - T->pb[n][m] * pnm1;
-  return v / T->pd[n][m];
+  return v * T->pd[n][m];
 }
 
 // ---------------------------------------------------------------------
@@ -520,6 +524,48 @@ __global__ __launch_bounds__(64) void k_hel_m2l(
   for (int r = lane; r < (Nr + 1) * (Nr + 1); r += kWave) out[r] = cadd(out[r], acc[r]);
 }
 
+// Shared by the two thread kernels.  G lanes per target: the columns m of the
+// local expansion dealt back and forth, the neighbours' sources as in
+// NearSplit, the lanes' sums added at the end; with several lanes the
+// Bessel functions are computed side by side, an order a lane, through LDS.
+template <int NMAX, int G>
+struct HelFieldJ {
+  static constexpr int n = G > 1 ? (128 / G) * (NMAX + 2) : 1;
+};
+template <int NMAX, int G>
+__device__ __forceinline__ const double *hel_field_bessel(int N, double x, int g, double *lds,
+                                                          double *own) {
+  if constexpr (G > 1) {
+    double *J = lds + (threadIdx.x / G) * (NMAX + 2);
+    for (int nn = g; nn <= N + 1; nn += G) J[nn] = bessel_j_one(nn, x);
+    __syncthreads();
+    return J;
+  } else {
+    bessel_j(N + 1, x, own);
+    return own;
+  }
+}
+#define HEL_FIELD_BESSEL                                                        \
+  __shared__ double jlds[HelFieldJ<NMAX, G>::n];                                \
+  double jown[G > 1 ? 1 : NMAX + 2];                                            \
+  const double *jn = hel_field_bessel<NMAX, G>(N, k * r, g, jlds, jown);
+#define HEL_FIELD_STORE                                                         \
+  const double2 v[4] = {pot, gx, gy, gz};                                       \
+  double sum[8];                                                                \
+  _Pragma("unroll") for (int c = 0; c < 4; c++) {                               \
+    sum[2 * c] = group_sum<G>(v[c].x);                                          \
+    sum[2 * c + 1] = group_sum<G>(v[c].y);                                      \
+  }                                                                             \
+  if (!valid || g) return;                                                      \
+  double *o = f + (size_t)tid[i] * fstr;                                        \
+  if (field & 1) {                                                              \
+    o[0] += sum[0];                                                             \
+    o[1] += sum[1];                                                             \
+    o += 2;                                                                     \
+  }                                                                             \
+  if (field & 2)                                                                \
+    for (int c = 0; c < 6; c++) o[c] += sum[2 + c];
+
 // ---------------------------------------------------------------------
 // L2P + near field (src/local.c:32-310, src/expansions.c:275-344,
 // src/gradient.c:282-399), one thread per target.  With
@@ -535,7 +581,7 @@ __global__ __launch_bounds__(64) void k_hel_m2l(
 // f[tid*fstr + ...]: potential (2 doubles) then gradient (6) when both
 // are asked, accumulated.
 // ---------------------------------------------------------------------
-template <int NMAX>
+template <int NMAX, int G>
 __global__ __launch_bounds__(128) void k_hel_field(
     const double *__restrict__ xt, const uint32_t *__restrict__ tid, unsigned n,
     const uint32_t *__restrict__ start, const uint32_t *__restrict__ end,
@@ -544,8 +590,10 @@ __global__ __launch_bounds__(128) void k_hel_field(
     unsigned level, double x0, double y0, double z0, double D, int N, double k,
     const double2 *__restrict__ mpr, int field, double *__restrict__ f, int fstr,
     const RecTab *__restrict__ RT) {
-  const unsigned i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
+  const unsigned id = blockIdx.x * blockDim.x + threadIdx.x;
+  const int g = (int)(id % G);
+  const bool valid = id / G < n;
+  const unsigned i = valid ? id / G : n - 1;
   const double x = xt[4 * i], y = xt[4 * i + 1], z = xt[4 * i + 2];
   const uint64_t code = point_code(x, y, z, x0, y0, z0, D);
   const uint64_t b = code >> (3 * (20 - level));
@@ -559,13 +607,16 @@ __global__ __launch_bounds__(128) void k_hel_field(
     return Lc[hidx(nn, mm)];
   };
   {
-    double r, C, S, cp, sp, jn[NMAX + 2];
+    double r, C, S, cp, sp;
     sph(x - xc, y - yc, z - zc, r, C, S, cp, sp);
-    bessel_j(N + 1, k * r, jn);
+    HEL_FIELD_BESSEL
     const double phi = atan2(sp, cp);
     double pmm = 1.0 / sqrt(4.0 * kPi);
-    for (int m = 0; m <= N + 1; m++) {
-      if (m > 0) pmm *= sqrt((2.0 * m + 1) / (2.0 * m)) * S;
+    int m0 = 0;
+    for (int mb = 0; mb <= N + 1; mb += G) {
+      const int m = (mb / G) & 1 ? mb + G - 1 - g : mb + g;
+      if (m > N + 1) continue;
+      for (; m0 < m; m0++) pmm *= RT->pc[m0 + 1] * S;
       double sn, cs;
       sincos((double)m * phi, &sn, &cs);
       double p = pmm, pprev = 0.0;
@@ -599,61 +650,45 @@ __global__ __launch_bounds__(128) void k_hel_field(
   double2 gy = make_double2(dd.y, -dd.x);
   gz = cscale(gz, k);
   // near field: the 27 neighbours of the target's box
-  const int bi = compact3(b), bj = compact3(b >> 1), bk = compact3(b >> 2), nb = 1 << level;
-  for (int a = -1; a <= 1; a++)
-    for (int bb = -1; bb <= 1; bb++)
-      for (int c = -1; c <= 1; c++) {
-        const int si = bi + a, sj = bj + bb, sk = bk + c;
-        if (si < 0 || si >= nb || sj < 0 || sj >= nb || sk < 0 || sk >= nb) continue;
-        const uint64_t sb = spread3(si) | (spread3(sj) << 1) | (spread3(sk) << 2);
-        for (uint32_t s = start[sb]; s < end[sb]; s++) {
-          const double rx = x - xyz[4 * s], ry = y - xyz[4 * s + 1], rz = z - xyz[4 * s + 2];
-          const double r = sqrt(rx * rx + ry * ry + rz * rz);
-          if (r <= 1e-6) continue;
-          double sn, cs;
-          sincos(k * r, &sn, &cs);
-          // G = e^{ikr} / (4 pi i k r) = (sin - i cos) / (4 pi k r)
-          const double g0 = 1.0 / (4.0 * kPi * k * r);
-          const double2 G = make_double2(sn * g0, -cs * g0);
-          const double2 dG = cmul(G, make_double2(-1.0 / r, k));  // G (ik - 1/r)
-          const double2 G2 = cmul(G, cadd(cmul(make_double2(-1.0 / r, k), make_double2(-1.0 / r, k)),
-                                          make_double2(1.0 / (r * r), 0.0)));
-          const double ux = rx / r, uy = ry / r, uz = rz / r;
-          if (q) {
-            const double2 qq = q[s];
-            const double2 qG = cmul(qq, G), qd = cmul(qq, dG);
-            pot = cadd(pot, qG);
-            gx = cadd(gx, cscale(qd, ux));
-            gy = cadd(gy, cscale(qd, uy));
-            gz = cadd(gz, cscale(qd, uz));
-          }
-          if (dip) {
-            const double2 dq = dip[s];
-            const double nx = nrm[4 * s], ny = nrm[4 * s + 1], nz = nrm[4 * s + 2];
-            const double nr = nx * ux + ny * uy + nz * uz;
-            pot = cadd(pot, cscale(cmul(dq, dG), nr));
-            const double2 t1 = cscale(cmul(dq, G2), nr), t2 = cscale(cmul(dq, dG), 1.0 / r);
-            gx = cadd(gx, cadd(cscale(t1, ux), cscale(t2, nx - nr * ux)));
-            gy = cadd(gy, cadd(cscale(t1, uy), cscale(t2, ny - nr * uy)));
-            gz = cadd(gz, cadd(cscale(t1, uz), cscale(t2, nz - nr * uz)));
-          }
-        }
-      }
-  double *o = f + (size_t)tid[i] * fstr;
-  int at = 0;
-  if (field & 1) {
-    o[0] += pot.x;
-    o[1] += pot.y;
-    at = 2;
-  }
-  if (field & 2) {
-    o[at + 0] += gx.x;
-    o[at + 1] += gx.y;
-    o[at + 2] += gy.x;
-    o[at + 3] += gy.y;
-    o[at + 4] += gz.x;
-    o[at + 5] += gz.y;
-  }
+  near_sources<G>(g, compact3(b), compact3(b >> 1), compact3(b >> 2), (int)level, start, end,
+                  [&](uint32_t s) {
+    const double rx = x - xyz[4 * (size_t)s], ry = y - xyz[4 * (size_t)s + 1],
+                 rz = z - xyz[4 * (size_t)s + 2];
+    const double r = sqrt(rx * rx + ry * ry + rz * rz);
+    if (r <= 1e-6) return;
+    const double ir = 1.0 / r;
+    double sn, cs;
+    sincos(k * r, &sn, &cs);
+    // G = e^{ikr} / (4 pi i k r) = (sin - i cos) / (4 pi k r)
+    const double g0 = ir * (1.0 / (4.0 * kPi * k));
+    const double2 Gr = make_double2(sn * g0, -cs * g0);
+    const double2 dG = cmul(Gr, make_double2(-ir, k));  // G (ik - 1/r)
+    const double ux = rx * ir, uy = ry * ir, uz = rz * ir;
+    // a source without a strength of a kind adds nothing of that kind
+    const double2 qq = q ? q[s] : make_double2(0.0, 0.0);
+    if (qq.x != 0.0 || qq.y != 0.0) {
+      const double2 qG = cmul(qq, Gr), qd = cmul(qq, dG);
+      pot = cadd(pot, qG);
+      gx = cadd(gx, cscale(qd, ux));
+      gy = cadd(gy, cscale(qd, uy));
+      gz = cadd(gz, cscale(qd, uz));
+    }
+    const double2 dq = dip ? dip[s] : make_double2(0.0, 0.0);
+    if (dq.x != 0.0 || dq.y != 0.0) {
+      // G ((ik - 1/r)^2 + 1/r^2)
+      const double2 G2 = cmul(Gr, cadd(cmul(make_double2(-ir, k), make_double2(-ir, k)),
+                                       make_double2(ir * ir, 0.0)));
+      const double nx = nrm[4 * (size_t)s], ny = nrm[4 * (size_t)s + 1],
+                   nz = nrm[4 * (size_t)s + 2];
+      const double nr = nx * ux + ny * uy + nz * uz;
+      pot = cadd(pot, cscale(cmul(dq, dG), nr));
+      const double2 t1 = cscale(cmul(dq, G2), nr), t2 = cscale(cmul(dq, dG), ir);
+      gx = cadd(gx, cadd(cscale(t1, ux), cscale(t2, nx - nr * ux)));
+      gy = cadd(gy, cadd(cscale(t1, uy), cscale(t2, ny - nr * uy)));
+      gz = cadd(gz, cadd(cscale(t1, uz), cscale(t2, nz - nr * uz)));
+    }
+  });
+  HEL_FIELD_STORE
 }
 
 // ---------------------------------------------------------------------
@@ -875,7 +910,7 @@ __global__ __launch_bounds__(64) void k_hel_field_box(
 // On leaves of a few to a few tens of targets this keeps every lane busy,
 // where one wavefront per target box leaves most of its lanes idle.
 // ---------------------------------------------------------------------
-template <int NMAX>
+template <int NMAX, int G>
 __global__ __launch_bounds__(128) void k_hel_field_mixed(
     const double *__restrict__ xt, const uint32_t *__restrict__ tid, unsigned n,
     const uint32_t *__restrict__ start, const uint32_t *__restrict__ end,
@@ -887,8 +922,10 @@ __global__ __launch_bounds__(128) void k_hel_field_mixed(
   __shared__ double sinv[NMAX + 2];
   for (int t = threadIdx.x; t <= N + 1; t += blockDim.x) sinv[t] = 1.0 / sc[t];
   __syncthreads();
-  const unsigned i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
+  const unsigned id = blockIdx.x * blockDim.x + threadIdx.x;
+  const int g = (int)(id % G);
+  const bool valid = id / G < n;
+  const unsigned i = valid ? id / G : n - 1;
   const double x = xt[4 * i], y = xt[4 * i + 1], z = xt[4 * i + 2];
   const uint64_t code = point_code(x, y, z, x0, y0, z0, D);
   const uint64_t b = code >> (3 * (20 - level));
@@ -908,13 +945,16 @@ __global__ __launch_bounds__(128) void k_hel_field_mixed(
     return make_double2((double)v.x * w, (double)v.y * w);
   };
   {
-    double r, C, S, cp, sp, jn[NMAX + 2];
+    double r, C, S, cp, sp;
     sph(x - xc, y - yc, z - zc, r, C, S, cp, sp);
-    bessel_j(N + 1, k * r, jn);
+    HEL_FIELD_BESSEL
     const double phi = atan2(sp, cp);
     double pmm = 1.0 / sqrt(4.0 * kPi);
-    for (int m = 0; m <= N + 1; m++) {
-      if (m > 0) pmm *= sqrt((2.0 * m + 1) / (2.0 * m)) * S;
+    int m0 = 0;
+    for (int mb = 0; mb <= N + 1; mb += G) {
+      const int m = (mb / G) & 1 ? mb + G - 1 - g : mb + g;
+      if (m > N + 1) continue;
+      for (; m0 < m; m0++) pmm *= RT->pc[m0 + 1] * S;
       double sn, cs;
       sincos((double)m * phi, &sn, &cs);
       double p = pmm, pprev = 0.0;
@@ -954,72 +994,54 @@ __global__ __launch_bounds__(128) void k_hel_field_mixed(
   agy.zero();
   agz.zero();
   const float kk = (float)k, c4 = (float)(1.0 / (4.0 * kPi * k));
-  const int bi = compact3(b), bj = compact3(b >> 1), bk = compact3(b >> 2), nb = 1 << level;
-  for (int a = -1; a <= 1; a++)
-    for (int bb = -1; bb <= 1; bb++)
-      for (int c = -1; c <= 1; c++) {
-        const int si = bi + a, sj = bj + bb, sk = bk + c;
-        if (si < 0 || si >= nb || sj < 0 || sj >= nb || sk < 0 || sk >= nb) continue;
-        const uint64_t sb = spread3(si) | (spread3(sj) << 1) | (spread3(sk) << 2);
-        for (uint32_t s = start[sb]; s < end[sb]; s++) {
-          const double rxd = x - xyz[4 * s], ryd = y - xyz[4 * s + 1], rzd = z - xyz[4 * s + 2];
-          const double r2 = rxd * rxd + ryd * ryd + rzd * rzd;
-          if (r2 <= 1e-12) continue;
-          const float rx = (float)rxd, ry = (float)ryd, rz = (float)rzd;
-          const float r = sqrtf((float)r2), ir = 1.0f / r;
-          float sn, cs;
-          sincosf(kk * r, &sn, &cs);
-          // G = (sin - i cos) / (4 pi k r), G (ik - 1/r), G ((ik - 1/r)^2 + 1/r^2)
-          const float g0 = c4 * ir;
-          const float Gr = sn * g0, Gi = -cs * g0;
-          const float dGr = -Gr * ir - Gi * kk, dGi = Gr * kk - Gi * ir;
-          const float ux = rx * ir, uy = ry * ir, uz = rz * ir;
-          if (q) {
-            const float qr = (float)q[s].x, qi = (float)q[s].y;
-            apot.add(qr * Gr - qi * Gi, qr * Gi + qi * Gr);
-            const float qdr = qr * dGr - qi * dGi, qdi = qr * dGi + qi * dGr;
-            agx.add(qdr * ux, qdi * ux);
-            agy.add(qdr * uy, qdi * uy);
-            agz.add(qdr * uz, qdi * uz);
-          }
-          if (dip) {
-            const float dr = (float)dip[s].x, di = (float)dip[s].y;
-            const double nxd = nrm[4 * s], nyd = nrm[4 * s + 1], nzd = nrm[4 * s + 2];
-            const float nx = (float)nxd, ny = (float)nyd, nz = (float)nzd;
-            // n.(x-y) in FP64 (close points on a surface: n nearly orthogonal)
-            const float nr = (float)(nxd * rxd + nyd * ryd + nzd * rzd) * ir;
-            const float ddr = dr * dGr - di * dGi, ddi = dr * dGi + di * dGr;
-            apot.add(ddr * nr, ddi * nr);
-            // (ik - 1/r)^2 + 1/r^2 = 2/r^2 - k^2 - 2ik/r
-            const float e2r = 2.0f * ir * ir - kk * kk, e2i = -2.0f * kk * ir;
-            const float g2r = Gr * e2r - Gi * e2i, g2i = Gr * e2i + Gi * e2r;
-            const float t1r = (dr * g2r - di * g2i) * nr, t1i = (dr * g2i + di * g2r) * nr;
-            const float t2r = ddr * ir, t2i = ddi * ir;
-            agx.add(t1r * ux + t2r * (nx - nr * ux), t1i * ux + t2i * (nx - nr * ux));
-            agy.add(t1r * uy + t2r * (ny - nr * uy), t1i * uy + t2i * (ny - nr * uy));
-            agz.add(t1r * uz + t2r * (nz - nr * uz), t1i * uz + t2i * (nz - nr * uz));
-          }
-        }
-      }
+  near_sources<G>(g, compact3(b), compact3(b >> 1), compact3(b >> 2), (int)level, start, end,
+                  [&](uint32_t s) {
+    const double rxd = x - xyz[4 * (size_t)s], ryd = y - xyz[4 * (size_t)s + 1], rzd = z - xyz[4 * (size_t)s + 2];
+    const double r2 = rxd * rxd + ryd * ryd + rzd * rzd;
+    if (r2 <= 1e-12) return;
+    const float rx = (float)rxd, ry = (float)ryd, rz = (float)rzd;
+    const float r = sqrtf((float)r2), ir = 1.0f / r;
+    float sn, cs;
+    sincosf(kk * r, &sn, &cs);
+    // G = (sin - i cos) / (4 pi k r), G (ik - 1/r), G ((ik - 1/r)^2 + 1/r^2)
+    const float g0 = c4 * ir;
+    const float Gr = sn * g0, Gi = -cs * g0;
+    const float dGr = -Gr * ir - Gi * kk, dGi = Gr * kk - Gi * ir;
+    const float ux = rx * ir, uy = ry * ir, uz = rz * ir;
+    // a source without a strength of a kind adds nothing of that kind
+    const double2 qq = q ? q[s] : make_double2(0.0, 0.0);
+    if (qq.x != 0.0 || qq.y != 0.0) {
+      const float qr = (float)qq.x, qi = (float)qq.y;
+      apot.add(qr * Gr - qi * Gi, qr * Gi + qi * Gr);
+      const float qdr = qr * dGr - qi * dGi, qdi = qr * dGi + qi * dGr;
+      agx.add(qdr * ux, qdi * ux);
+      agy.add(qdr * uy, qdi * uy);
+      agz.add(qdr * uz, qdi * uz);
+    }
+    const double2 dq = dip ? dip[s] : make_double2(0.0, 0.0);
+    if (dq.x != 0.0 || dq.y != 0.0) {
+      const float dr = (float)dq.x, di = (float)dq.y;
+      const double nxd = nrm[4 * (size_t)s], nyd = nrm[4 * (size_t)s + 1], nzd = nrm[4 * (size_t)s + 2];
+      const float nx = (float)nxd, ny = (float)nyd, nz = (float)nzd;
+      // n.(x-y) in FP64 (close points on a surface: n nearly orthogonal)
+      const float nr = (float)(nxd * rxd + nyd * ryd + nzd * rzd) * ir;
+      const float ddr = dr * dGr - di * dGi, ddi = dr * dGi + di * dGr;
+      apot.add(ddr * nr, ddi * nr);
+      // (ik - 1/r)^2 + 1/r^2 = 2/r^2 - k^2 - 2ik/r
+      const float e2r = 2.0f * ir * ir - kk * kk, e2i = -2.0f * kk * ir;
+      const float g2r = Gr * e2r - Gi * e2i, g2i = Gr * e2i + Gi * e2r;
+      const float t1r = (dr * g2r - di * g2i) * nr, t1i = (dr * g2i + di * g2r) * nr;
+      const float t2r = ddr * ir, t2i = ddi * ir;
+      agx.add(t1r * ux + t2r * (nx - nr * ux), t1i * ux + t2i * (nx - nr * ux));
+      agy.add(t1r * uy + t2r * (ny - nr * uy), t1i * uy + t2i * (ny - nr * uy));
+      agz.add(t1r * uz + t2r * (nz - nr * uz), t1i * uz + t2i * (nz - nr * uz));
+    }
+  });
   pot = cadd(pot, apot.value());
   gx = cadd(gx, agx.value());
   gy = cadd(gy, agy.value());
   gz = cadd(gz, agz.value());
-  double *o = f + (size_t)tid[i] * fstr;
-  int at = 0;
-  if (field & 1) {
-    o[0] += pot.x;
-    o[1] += pot.y;
-    at = 2;
-  }
-  if (field & 2) {
-    o[at + 0] += gx.x;
-    o[at + 1] += gx.y;
-    o[at + 2] += gy.x;
-    o[at + 3] += gy.y;
-    o[at + 4] += gz.x;
-    o[at + 5] += gz.y;
-  }
+  HEL_FIELD_STORE
 }
 
 // out (FP32, box-major, complex) = in (FP64) with degree n multiplied by
@@ -1324,16 +1346,35 @@ int wbfmm_hip_hel_field(const double *xt, const uint32_t *tid, unsigned n,
     const int rc = rec_tab(&RT);
     if (rc) return rc;
   }
-#define HF(NM)                                                                          \
-  WBFMM_LAUNCH("hel_l2p_p2p", k_hel_field<NM>, dim3((n + 127) / 128), dim3(128), 0, xt, \
-               tid, n, start, end, xyz, (const double2 *)q, nrm, (const double2 *)dip,  \
-               level, x0[0], x0[1], x0[2], D, N, k, (const double2 *)mpr, field, f, fstr, RT)
-  if (N <= 16) HF(16);
-  else if (N <= 24) HF(24);
-  else if (N <= 32) HF(32);
-  else if (N <= WBFMM_HIP_MAX_ORDER) HF(WBFMM_HIP_MAX_ORDER);
-  else return WBFMM_HIP_ERR_ORDER;
+  const int lanes = n > (1u << 26) ? 1 : field_lanes(n);
+#define HF_G(NM, G)                                                                          \
+  case G:                                                                                    \
+    WBFMM_LAUNCH("hel_l2p_p2p", (k_hel_field<NM, G>),                                   \
+                 dim3((unsigned)(((size_t)n * G + 127) / 128)), dim3(128), 0, xt, tid, n, start, \
+                 end, xyz, (const double2 *)q, nrm, (const double2 *)dip, level, x0[0],      \
+                 x0[1], x0[2], D, N, k, (const double2 *)mpr, field, f, fstr, RT);           \
+    break;
+#define HF(NM)       \
+  switch (lanes) {   \
+    HF_G(NM, 1)      \
+    HF_G(NM, 2)      \
+    HF_G(NM, 4)      \
+    HF_G(NM, 8)      \
+    HF_G(NM, 16)     \
+  }
+  if (N <= 16) {
+    HF(16)
+  } else if (N <= 24) {
+    HF(24)
+  } else if (N <= 32) {
+    HF(32)
+  } else if (N <= WBFMM_HIP_MAX_ORDER) {
+    HF(WBFMM_HIP_MAX_ORDER)
+  } else {
+    return WBFMM_HIP_ERR_ORDER;
+  }
 #undef HF
+#undef HF_G
   return 0;
 }
 
@@ -1350,17 +1391,35 @@ int wbfmm_hip_hel_field_f32(const double *xt, const uint32_t *tid, unsigned n,
     const int rc = rec_tab(&RT);
     if (rc) return rc;
   }
-#define HF(NM)                                                                              \
-  WBFMM_LAUNCH("hel_l2p_p2p_f32", k_hel_field_mixed<NM>, dim3((n + 127) / 128), dim3(128), 0, \
-               xt, tid, n, start, end, xyz, (const double2 *)q, nrm, (const double2 *)dip,   \
-               level, x0[0], x0[1], x0[2], D, N, k, (const float2 *)mpr, scale, field, f,    \
-               fstr, RT)
-  if (N <= 16) HF(16);
-  else if (N <= 24) HF(24);
-  else if (N <= 32) HF(32);
-  else if (N <= WBFMM_HIP_MAX_ORDER) HF(WBFMM_HIP_MAX_ORDER);
-  else return WBFMM_HIP_ERR_ORDER;
+  const int lanes = n > (1u << 26) ? 1 : field_lanes(n);
+#define HF_G(NM, G)                                                                          \
+  case G:                                                                                    \
+    WBFMM_LAUNCH("hel_l2p_p2p_f32", (k_hel_field_mixed<NM, G>),                                   \
+                 dim3((unsigned)(((size_t)n * G + 127) / 128)), dim3(128), 0, xt, tid, n, start, \
+                 end, xyz, (const double2 *)q, nrm, (const double2 *)dip, level, x0[0],      \
+                 x0[1], x0[2], D, N, k, (const float2 *)mpr, scale, field, f, fstr, RT);     \
+    break;
+#define HF(NM)       \
+  switch (lanes) {   \
+    HF_G(NM, 1)      \
+    HF_G(NM, 2)      \
+    HF_G(NM, 4)      \
+    HF_G(NM, 8)      \
+    HF_G(NM, 16)     \
+  }
+  if (N <= 16) {
+    HF(16)
+  } else if (N <= 24) {
+    HF(24)
+  } else if (N <= 32) {
+    HF(32)
+  } else if (N <= WBFMM_HIP_MAX_ORDER) {
+    HF(WBFMM_HIP_MAX_ORDER)
+  } else {
+    return WBFMM_HIP_ERR_ORDER;
+  }
 #undef HF
+#undef HF_G
   return 0;
 }
 

@@ -116,4 +116,48 @@ __device__ __forceinline__ int isqrt_deg(int r) {
 constexpr double kPi = 3.14159265358979323846;
 constexpr int kWave = 64;
 
+// ---- several lanes per target (field kernels) ------------------------------
+
+// Lanes per target for n targets: enough that they fill the chip's 1024 SIMDs
+// twice, at most 16.  Measured (L2P + P2P, ms): 1000 targets 0.228 -> 0.021
+// and 13337 0.55 -> 0.080 with 16 lanes (32 lanes: 0.098), 10000 (Helmholtz)
+// 0.285 -> 0.067, 31013 on a sphere 0.52 -> 0.116 with 8, 100003
+// (Helmholtz) 1.83 -> 1.53 with 2 (4 lanes 1.56); more lanes than that only
+// repeat each target's preparation (3e5 targets: 0.39 with 1 lane, 0.44
+// with 4).
+inline int field_lanes(unsigned n) {
+  int g = 1;
+  while (g < 16 && (uint64_t)n * g < 131072u) g *= 2;
+  return g;
+}
+
+// sum over the G consecutive lanes of a group, the same in each
+template <int G>
+__device__ __forceinline__ double group_sum(double v) {
+#pragma unroll
+  for (int h = 1; h < G; h *= 2) v += __shfl_xor(v, h);
+  return v;
+}
+
+// The 27 neighbour boxes' sources of a target, dealt to its G lanes: GB of
+// them take every GB-th box, and the G / GB lanes of a box every
+// (G / GB)-th source
+template <int G>
+struct NearSplit {
+  static constexpr int GB = G >= 4 ? 4 : G, GS = G / GB;
+};
+template <int G, typename F>
+__device__ __forceinline__ void near_sources(int g, int bi, int bj, int bk, int level,
+                                             const uint32_t *start, const uint32_t *end, F f) {
+  constexpr int GB = NearSplit<G>::GB, GS = NearSplit<G>::GS;
+  const int nbox = 1 << level;
+  for (int c = g / GS; c < 27; c += GB) {
+    const int ii = bi + c / 9 - 1, jj = bj + (c / 3) % 3 - 1, kk = bk + c % 3 - 1;
+    if (ii < 0 || ii >= nbox || jj < 0 || jj >= nbox || kk < 0 || kk >= nbox) continue;
+    const uint64_t nb = spread3(ii) | (spread3(jj) << 1) | (spread3(kk) << 2);
+    const uint32_t e = end[nb];
+    for (uint32_t s = start[nb] + g % GS; s < e; s += GS) f(s);
+  }
+}
+
 }  // namespace wbfmm

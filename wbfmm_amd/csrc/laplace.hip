@@ -19,6 +19,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <mutex>
+
 #include "hip_common.h"
 
 namespace wbfmm {
@@ -570,19 +572,79 @@ __device__ __forceinline__ void lcoef_nb(const T *mpr, uint64_t b, int C, int n,
   im = m ? v : 0.0;
 }
 
+// The factors of the regular functions' recurrences and of the gradient per
+// (j, k), 0 <= k <= j, and the ladder factors of the second derivatives:
+// one table per process, built once on the device, read instead of several
+// square roots and divisions per step.
+struct LapCol {
+  double al, be;      // P_j^k = Cth al P_{j-1}^k - be P_{j-2}^k (j > k)
+  double f0, f1, f2;  // d/dz, and D+ from L_{j+1}^{k-1} and L_{j+1}^{k+1}
+  double dg;          // P_k^k = dg Sth P_{k-1}^{k-1} (at j = k > 0)
+};
+constexpr int kLapTabN = WBFMM_HIP_MAX_ORDER + 3;
+struct LapTab {
+  LapCol c[(WBFMM_HIP_MAX_ORDER + 1) * (WBFMM_HIP_MAX_ORDER + 2) / 2];
+  double la[kLapTabN][kLapTabN];          // lad_a(n, m)
+  double lb[kLapTabN][2 * kLapTabN + 1];  // lad_s(mu) lad_b(n, mu), mu - kLapTabN
+};
+
+__device__ __forceinline__ double lad_kn(int n) { return (2.0 * n + 1) / (2.0 * n - 1); }
+__device__ __forceinline__ double lad_a(int n, int m) {
+  return n >= 1 && m <= n ? sqrt(lad_kn(n) * (double)(n - m) * (double)(n + m)) : 0.0;
+}
+__device__ __forceinline__ double lad_b(int n, int mu) {
+  const double v = (double)(n - mu) * (double)(n - mu - 1);
+  return (n >= 1 && v > 0.0) ? sqrt(lad_kn(n) * v) : 0.0;
+}
+__device__ __forceinline__ double lad_s(int mu) { return mu >= 0 ? -1.0 : 1.0; }
+
+__global__ void k_lap_tab(LapTab *T) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < (WBFMM_HIP_MAX_ORDER + 1) * (WBFMM_HIP_MAX_ORDER + 2) / 2) {
+    int j = 0;
+    while ((j + 1) * (j + 2) / 2 <= t) j++;
+    const int k = t - j * (j + 1) / 2, n1 = j + 1;
+    LapCol c = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    if (j > k) {
+      const double h = sqrt((2.0 * j + 1) / (double)(j * j - k * k));
+      c.al = sqrt(2.0 * j - 1) * h;
+      c.be = j - 1 > k ? sqrt((double)((j - 1) * (j - 1) - k * k) / (2 * j - 3)) * h : 0.0;
+    } else if (k > 0) {
+      c.dg = sqrt((2.0 * k + 1) / (2.0 * k));
+    }
+    const double fc = sqrt((2.0 * n1 + 1) / (2.0 * n1 - 1));
+    c.f0 = fc * sqrt((double)(n1 - k) * (n1 + k));
+    c.f1 = k >= 1 ? fc * sqrt((double)(n1 - k + 1) * (n1 - k)) : 0.0;
+    c.f2 = fc * sqrt((double)(n1 + k + 1) * (n1 + k));
+    T->c[t] = c;
+  }
+  if (t < kLapTabN * kLapTabN) T->la[t / kLapTabN][t % kLapTabN] = lad_a(t / kLapTabN, t % kLapTabN);
+  if (t < kLapTabN * (2 * kLapTabN + 1)) {
+    const int n = t / (2 * kLapTabN + 1), mu = t % (2 * kLapTabN + 1) - kLapTabN;
+    T->lb[n][mu + kLapTabN] = (mu < 0 ? -mu : mu) <= n ? lad_s(mu) * lad_b(n, mu) : 0.0;
+  }
+}
+
+// G lanes per target (G a power of two): the columns k of the local
+// expansion dealt back and forth (lane g takes g, 2G-1-g, 2G+g, ..: near
+// equal numbers of steps), the neighbours' sources as in NearSplit, and the
+// lanes' sums added at the end.  One lane per target leaves most of the
+// chip idle below a few hundred thousand targets: 13337 targets, order 13,
+// 39 points a leaf, are 209 wavefronts, each a chain of 105 expansion steps
+// and 1050 pairs (0.55 ms); see field_lanes for the figures.
 // T: coefficient type; rs as in k_lap_p2m (1/w for coefficients scaled by
 // the box width, L_n w^(n+1): the expansion then gives phi w and grad w^2)
-template <typename T>
-__global__ void k_lap_field(const double *xt, const uint32_t *tid,
-                            unsigned ntgt, const uint32_t *start,
-                            const uint32_t *end, const double *xyz,
-                            const double *q, const double *nrm,
-                            const double *dip, int level, double x0,
-                            double y0, double z0, double D, int N,
-                            double rs, const T *mpr, int field, double *f,
-                            int fstr) {
-  unsigned t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= ntgt) return;
+template <typename T, int G>
+__global__ __launch_bounds__(128) void k_lap_field(
+    const double *__restrict__ xt, const uint32_t *__restrict__ tid, unsigned ntgt,
+    const uint32_t *__restrict__ start, const uint32_t *__restrict__ end,
+    const double *__restrict__ xyz, const double *__restrict__ q,
+    const double *__restrict__ nrm, const double *__restrict__ dip, int level, double x0,
+    double y0, double z0, double D, int N, double rs, const T *__restrict__ mpr, int field,
+    double *__restrict__ f, int fstr, const LapTab *__restrict__ tab) {
+  const unsigned id = blockIdx.x * blockDim.x + threadIdx.x, t = id / G;
+  const int g = (int)(id % G);
+  if (t >= ntgt) return;  // the same in a group's lanes
   double px = xt[4 * (size_t)t], py = xt[4 * (size_t)t + 1],
          pz = xt[4 * (size_t)t + 2];
   uint64_t code = point_code(px, py, pz, x0, y0, z0, D);
@@ -601,9 +663,13 @@ __global__ void k_lap_field(const double *xt, const uint32_t *tid,
   const double rr = r * rs;
   // regular solid harmonics R_j^k column by column
   double pmm = s4pi, rm = 1.0, cm = 1.0, sm = 0.0;
-  for (int k = 0; k <= N; k++) {
-    if (k > 0) {
-      pmm *= sqrt((2.0 * k + 1) / (2.0 * k)) * Sth;
+  int k0 = 0;
+  for (int cb = 0; cb <= N; cb += G) {
+    const int k = (cb / G) & 1 ? cb + G - 1 - g : cb + g;
+    if (k > N) continue;
+    for (; k0 < k; k0++) {
+      const int kk = k0 + 1;
+      pmm *= tab->c[kk * (kk + 1) / 2 + kk].dg * Sth;
       rm *= rr;
       double tcm = cm * cp - sm * sp;
       sm = sm * cp + cm * sp;
@@ -612,10 +678,9 @@ __global__ void k_lap_field(const double *xt, const uint32_t *tid,
     double p1 = 0.0, p0 = pmm, rn = rm;
     double wk = (k == 0) ? 1.0 : 2.0;
     for (int j = k; j <= N; j++) {
+      const LapCol tc = tab->c[j * (j + 1) / 2 + k];
       if (j > k) {
-        double pn = (Cth * sqrt(2.0 * (j - 1) + 1) * p0 -
-                     sqrt((double)((j - 1) * (j - 1) - k * k) / (2 * (j - 1) - 1)) * p1) *
-                    sqrt((2.0 * (j - 1) + 3) / (double)(j * j - k * k));
+        double pn = Cth * tc.al * p0 - tc.be * p1;
         p1 = p0;
         p0 = pn;
         rn *= rr;
@@ -626,30 +691,22 @@ __global__ void k_lap_field(const double *xt, const uint32_t *tid,
       phi += wk * (lr * Rr - li * Ri);
       if (want_g && j < N) {
         int n1 = j + 1;
-        double fc = sqrt((2.0 * n1 + 1) / (2.0 * n1 - 1));
-        // the three coefficients of degree j + 1 read without branches
-        // (the conditions are the same in every lane), so that their
-        // loads issue together: L^k, L^{k-1} (weight 0 at k = 0, read at
-        // order 0 there), L^{k+1} (k + 1 <= j + 1 always)
+        // the three coefficients of degree j + 1 read without branches, so
+        // that their loads issue together: L^k, L^{k-1} (weight 0 at k = 0,
+        // read at order 0 there), L^{k+1} (k + 1 <= j + 1 always)
         double l0r, l0i, lmr, lmi, lpr, lpi;
         const int mm = k >= 1 ? k - 1 : 0, mp = k + 1;
         lcoef_nb(mpr, b, C, n1, k, l0r, l0i);
         lcoef_nb(mpr, b, C, n1, mm, lmr, lmi);
         lcoef_nb(mpr, b, C, n1, mp, lpr, lpi);
         // dz: a_{j+1}^k L_{j+1}^k R_j^k
-        gz += wk * fc * sqrt((double)(n1 - k) * (n1 + k)) * (l0r * Rr - l0i * Ri);
+        gz += wk * tc.f0 * (l0r * Rr - l0i * Ri);
         // D+: -b1_{j+1}^{k-1} L_{j+1}^{k-1} R_j^k
-        {
-          double b1 = k >= 1 ? fc * sqrt((double)(n1 - mm) * (n1 - mm - 1)) : 0.0;
-          gpr -= b1 * (lmr * Rr - lmi * Ri);
-          gpi -= b1 * (lmr * Ri + lmi * Rr);
-        }
+        gpr -= tc.f1 * (lmr * Rr - lmi * Ri);
+        gpi -= tc.f1 * (lmr * Ri + lmi * Rr);
         // D+: b2_{j+1}^{k+1} conj(L_{j+1}^{k+1} R_j^k)
-        {
-          double b2 = fc * sqrt((double)(n1 + mp) * (n1 + mp - 1));
-          gpr += b2 * (lpr * Rr - lpi * Ri);
-          gpi -= b2 * (lpr * Ri + lpi * Rr);
-        }
+        gpr += tc.f2 * (lpr * Rr - lpi * Ri);
+        gpi -= tc.f2 * (lpr * Ri + lpi * Rr);
       }
     }
   }
@@ -658,41 +715,35 @@ __global__ void k_lap_field(const double *xt, const uint32_t *tid,
   double gx = gpr * (rs * rs), gy = gpi * (rs * rs);
   // near field over the 27 neighbours, cutoff |x-y| <= 1e-6
   const double c4 = 0.25 / kPi, cut2 = 1e-12;
-  int nbox = 1 << level;
-  for (int ii = bi - 1; ii <= bi + 1; ii++) {
-    if (ii < 0 || ii >= nbox) continue;
-    for (int jj = bj - 1; jj <= bj + 1; jj++) {
-      if (jj < 0 || jj >= nbox) continue;
-      for (int kk = bk - 1; kk <= bk + 1; kk++) {
-        if (kk < 0 || kk >= nbox) continue;
-        uint64_t nb = spread3(ii) | (spread3(jj) << 1) | (spread3(kk) << 2);
-        for (uint32_t s = start[nb]; s < end[nb]; s++) {
-          double rx = px - xyz[4 * (size_t)s], ry = py - xyz[4 * (size_t)s + 1],
-                 rz = pz - xyz[4 * (size_t)s + 2];
-          double r2 = rx * rx + ry * ry + rz * rz;
-          if (r2 <= cut2) continue;
-          double ir = 1.0 / sqrt(r2), ir3 = ir * ir * ir;
-          if (q) {
-            double qs = q[s] * c4;
-            phi += qs * ir;
-            gx -= qs * rx * ir3;
-            gy -= qs * ry * ir3;
-            gz -= qs * rz * ir3;
-          }
-          if (dip) {
-            double nx = nrm[4 * (size_t)s], ny = nrm[4 * (size_t)s + 1],
-                   nz = nrm[4 * (size_t)s + 2];
-            double nr = nx * rx + ny * ry + nz * rz, ds = dip[s] * c4;
-            double ir5 = ir3 * ir * ir;
-            phi += ds * nr * ir3;
-            gx += ds * (nx * ir3 - 3.0 * nr * rx * ir5);
-            gy += ds * (ny * ir3 - 3.0 * nr * ry * ir5);
-            gz += ds * (nz * ir3 - 3.0 * nr * rz * ir5);
-          }
-        }
-      }
+  near_sources<G>(g, bi, bj, bk, level, start, end, [&](uint32_t s) {
+    double rx = px - xyz[4 * (size_t)s], ry = py - xyz[4 * (size_t)s + 1],
+           rz = pz - xyz[4 * (size_t)s + 2];
+    double r2 = rx * rx + ry * ry + rz * rz;
+    if (r2 <= cut2) return;
+    double ir = rsqrt(r2), ir3 = ir * ir * ir;
+    if (q) {
+      double qs = q[s] * c4;
+      phi += qs * ir;
+      gx -= qs * rx * ir3;
+      gy -= qs * ry * ir3;
+      gz -= qs * rz * ir3;
     }
-  }
+    if (dip) {
+      double nx = nrm[4 * (size_t)s], ny = nrm[4 * (size_t)s + 1],
+             nz = nrm[4 * (size_t)s + 2];
+      double nr = nx * rx + ny * ry + nz * rz, ds = dip[s] * c4;
+      double ir5 = ir3 * ir * ir;
+      phi += ds * nr * ir3;
+      gx += ds * (nx * ir3 - 3.0 * nr * rx * ir5);
+      gy += ds * (ny * ir3 - 3.0 * nr * ry * ir5);
+      gz += ds * (nz * ir3 - 3.0 * nr * rz * ir5);
+    }
+  });
+  phi = group_sum<G>(phi);
+  gx = group_sum<G>(gx);
+  gy = group_sum<G>(gy);
+  gz = group_sum<G>(gz);
+  if (g) return;
   double *out = f + (size_t)tid[t] * fstr;
   int o = 0;
   if (field & 1) out[o++] += phi;
@@ -720,16 +771,6 @@ __global__ void k_lap_field(const double *xt, const uint32_t *tid,
 // derivative of the expansion is an expansion of lower degree whose
 // coefficient at (j, nu) is read from L at degree j+1 or j+2.
 // ---------------------------------------------------------------------
-__device__ __forceinline__ double lad_kn(int n) { return (2.0 * n + 1) / (2.0 * n - 1); }
-__device__ __forceinline__ double lad_a(int n, int m) {
-  return n >= 1 ? sqrt(lad_kn(n) * (double)(n - m) * (double)(n + m)) : 0.0;
-}
-__device__ __forceinline__ double lad_b(int n, int mu) {
-  const double v = (double)(n - mu) * (double)(n - mu - 1);
-  return (n >= 1 && v > 0.0) ? sqrt(lad_kn(n) * v) : 0.0;
-}
-__device__ __forceinline__ double lad_s(int mu) { return mu >= 0 ? -1.0 : 1.0; }
-
 // L_n^mu of one box (real-packed: n^2 for mu = 0, n^2 + 2|mu| - 1 and +1)
 __device__ __forceinline__ double2 lcoef_c(const double *L, int N, int n, int mu) {
   const int am = mu < 0 ? -mu : mu;
@@ -741,19 +782,27 @@ __device__ __forceinline__ double2 lcoef_c(const double *L, int N, int n, int mu
 
 // potential, gradient (want_g) and second derivatives (want_h: xx, yy,
 // zz, xy, yz, zx) of one local expansion L of order N at offset (dx, dy,
-// dz) from its centre
-__device__ void lap_local_derivs(const double *L, int N, double dx, double dy, double dz,
-                                 bool want_g, bool want_h, double &phi, double g[3],
-                                 double h[6]) {
+// dz) from its centre: the share of the columns k that fall to lane part of
+// parts (back and forth, as in k_lap_field)
+__device__ __forceinline__ void lap_local_derivs(const double *__restrict__ L, int N, double dx,
+                                                 double dy, double dz, bool want_g, bool want_h,
+                                                 int part, int parts,
+                                                 const LapTab *__restrict__ tab, double &phi,
+                                                 double g[3], double h[6]) {
   const double r = sqrt(dx * dx + dy * dy + dz * dz), rho = sqrt(dx * dx + dy * dy);
   const double Cth = r > 0.0 ? dz / r : 1.0, Sth = r > 0.0 ? rho / r : 0.0;
   const double cp = rho > 0.0 ? dx / rho : 1.0, sp = rho > 0.0 ? dy / rho : 0.0;
   double ph = 0.0, gz = 0.0, gpr = 0.0, gpi = 0.0, zz = 0.0, vr = 0.0, vi = 0.0, wr = 0.0,
          wi = 0.0;
   double pmm = 1.0 / sqrt(4.0 * kPi), rm = 1.0, cm = 1.0, sm = 0.0;
-  for (int k = 0; k <= N; k++) {
-    if (k > 0) {
-      pmm *= sqrt((2.0 * k + 1) / (2.0 * k)) * Sth;
+  auto lb = [&](int n, int mu) { return tab->lb[n][mu + kLapTabN]; };
+  int k0 = 0;
+  for (int cb = 0, odd = 0; cb <= N; cb += parts, odd ^= 1) {
+    const int k = odd ? cb + parts - 1 - part : cb + part;
+    if (k > N) continue;
+    for (; k0 < k; k0++) {
+      const int kk = k0 + 1;
+      pmm *= tab->c[kk * (kk + 1) / 2 + kk].dg * Sth;
       rm *= r;
       const double tcm = cm * cp - sm * sp;
       sm = sm * cp + cm * sp;
@@ -762,9 +811,8 @@ __device__ void lap_local_derivs(const double *L, int N, double dx, double dy, d
     double p1 = 0.0, p0 = pmm, rn = rm;
     for (int j = k; j <= N; j++) {
       if (j > k) {
-        const double pn = (Cth * sqrt(2.0 * (j - 1) + 1) * p0 -
-                           sqrt((double)((j - 1) * (j - 1) - k * k) / (2 * (j - 1) - 1)) * p1) *
-                          sqrt((2.0 * (j - 1) + 3) / (double)(j * j - k * k));
+        const LapCol &tc = tab->c[j * (j + 1) / 2 + k];
+        const double pn = Cth * tc.al * p0 - tc.be * p1;
         p1 = p0;
         p0 = pn;
         rn *= r;
@@ -782,23 +830,22 @@ __device__ void lap_local_derivs(const double *L, int N, double dx, double dy, d
         acc(lcoef_c(L, N, j, nu), ph, dum);
         if (want_g) {
           const double2 cz = lcoef_c(L, N, j + 1, nu);
-          const double az = lad_a(j + 1, k);
+          const double az = tab->la[j + 1][k];
           acc(make_double2(cz.x * az, cz.y * az), gz, dum);
           const double2 cpl = lcoef_c(L, N, j + 1, nu - 1);
-          const double bp = lad_s(nu - 1) * lad_b(j + 1, nu - 1);
+          const double bp = lb(j + 1, nu - 1);
           acc(make_double2(cpl.x * bp, cpl.y * bp), gpr, gpi);
         }
         if (want_h) {
           const double2 c2 = lcoef_c(L, N, j + 2, nu);
-          const double f2 = lad_a(j + 2, k) * lad_a(j + 1, k);
+          const double f2 = tab->la[j + 2][k] * tab->la[j + 1][k];
           acc(make_double2(c2.x * f2, c2.y * f2), zz, dum);
           const int m1 = nu - 1 < 0 ? 1 - nu : nu - 1;
           const double2 cv = lcoef_c(L, N, j + 2, nu - 1);
-          const double fv = lad_a(j + 2, m1) * lad_s(nu - 1) * lad_b(j + 1, nu - 1);
+          const double fv = tab->la[j + 2][m1] * lb(j + 1, nu - 1);
           acc(make_double2(cv.x * fv, cv.y * fv), vr, vi);
           const double2 cw = lcoef_c(L, N, j + 2, nu - 2);
-          const double fw =
-              lad_s(nu - 2) * lad_b(j + 2, nu - 2) * lad_s(nu - 1) * lad_b(j + 1, nu - 1);
+          const double fw = lb(j + 2, nu - 2) * lb(j + 1, nu - 1);
           acc(make_double2(cw.x * fw, cw.y * fw), wr, wi);
         }
       }
@@ -885,17 +932,23 @@ __host__ __device__ __forceinline__ int vec_width(int mode, int nq) {
   return ((mode & 1) ? nq : 0) + ((mode & 2) ? 3 * nq : 0);
 }
 
-// one thread per target: local expansions of the target's leaf box plus
-// the 27 neighbour boxes' sources (strengths nq per point, sorted order)
+// Local expansions of the target's leaf box plus the 27 neighbour boxes'
+// sources (strengths nq per point, sorted order), G = 1, 4 or 16 lanes per
+// target: of four lanes, lane c takes the components c, c + 4, .., the
+// groups of four share each component's columns, and the sources are dealt
+// as in NearSplit.  CURL apart, so that its twelve sums stay in registers.
+template <bool CURL, int G>
 __global__ __launch_bounds__(128) void k_lap_field_vec(
     const double *__restrict__ xt, const uint32_t *__restrict__ tid, unsigned ntgt,
     const uint32_t *__restrict__ start, const uint32_t *__restrict__ end,
     const double *__restrict__ xyz, const double *__restrict__ q,
     const double *__restrict__ nrm, const double *__restrict__ dip, int nq, int level,
     double x0, double y0, double z0, double D, int N, const double *__restrict__ mpr,
-    size_t pst, int mode, double *__restrict__ f, int fstr) {
-  const unsigned t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= ntgt) return;
+    size_t pst, int mode, double *__restrict__ f, int fstr, const LapTab *__restrict__ tab) {
+  constexpr int GC = G >= 4 ? 4 : 1, GP = G / GC;  // lanes over components, over columns
+  const unsigned id = blockIdx.x * blockDim.x + threadIdx.x, t = id / G;
+  const int lane = (int)(id % G);
+  if (t >= ntgt) return;  // the same in a group's lanes
   const double px = xt[4 * (size_t)t], py = xt[4 * (size_t)t + 1], pz = xt[4 * (size_t)t + 2];
   const uint64_t b = point_code(px, py, pz, x0, y0, z0, D) >> (3 * (20 - level));
   const int bi = compact3(b), bj = compact3(b >> 1), bk = compact3(b >> 2);
@@ -903,48 +956,48 @@ __global__ __launch_bounds__(128) void k_lap_field_vec(
   const double dx = px - (x0 + w * (bi + 0.5)), dy = py - (y0 + w * (bj + 0.5)),
                dz = pz - (z0 + w * (bk + 0.5));
   const size_t C = (size_t)(N + 1) * (N + 1);
-  double out[kVecMaxOut];
-  const int nout = vec_width(mode, nq);
-  for (int i = 0; i < kVecMaxOut; i++) out[i] = 0.0;
-  if (mode & 4) {
-    double J[3][3], H[3][6];
-    for (int l = 0; l < 3; l++) {
-      double phi;
-      lap_local_derivs(mpr + l * pst + b * C, N, dx, dy, dz, true, (mode & 2) != 0, phi, J[l],
-                       H[l]);
-    }
-    curl_from(J, H, (mode & 2) != 0, out);
-  } else {
-    const int go = (mode & 1) ? nq : 0;
-    for (int l = 0; l < nq; l++) {
-      double phi, g[3], h[6];
-      lap_local_derivs(mpr + l * pst + b * C, N, dx, dy, dz, (mode & 2) != 0, false, phi, g, h);
+  constexpr int NO = CURL ? 12 : kVecMaxOut;
+  double out[NO];
+#pragma unroll
+  for (int i = 0; i < NO; i++) out[i] = 0.0;
+  const int go = (mode & 1) ? nq : 0;
+  for (int l = lane % GC; l < (CURL ? 3 : nq); l += GC) {
+    double phi, g[3], h[6];
+    lap_local_derivs(mpr + l * pst + b * C, N, dx, dy, dz, CURL || (mode & 2) != 0,
+                     CURL && (mode & 2) != 0, lane / GC, GP, tab, phi, g, h);
+    if constexpr (CURL) {
+      double J[3][3], H[3][6];
+#pragma unroll
+      for (int c = 0; c < 3; c++) {
+#pragma unroll
+        for (int i = 0; i < 3; i++) J[c][i] = l == c ? g[i] : 0.0;
+#pragma unroll
+        for (int i = 0; i < 6; i++) H[c][i] = l == c ? h[i] : 0.0;
+      }
+      curl_from(J, H, (mode & 2) != 0, out);
+    } else {
       if (mode & 1) out[l] += phi;
       if (mode & 2)
         for (int j = 0; j < 3; j++) out[go + 3 * l + j] += g[j];
     }
   }
-  const int nbox = 1 << level;
-  for (int ii = bi - 1; ii <= bi + 1; ii++) {
-    if (ii < 0 || ii >= nbox) continue;
-    for (int jj = bj - 1; jj <= bj + 1; jj++) {
-      if (jj < 0 || jj >= nbox) continue;
-      for (int kk = bk - 1; kk <= bk + 1; kk++) {
-        if (kk < 0 || kk >= nbox) continue;
-        const uint64_t nb = spread3(ii) | (spread3(jj) << 1) | (spread3(kk) << 2);
-        for (uint32_t s = start[nb]; s < end[nb]; s++) {
-          const double rx = px - xyz[4 * (size_t)s], ry = py - xyz[4 * (size_t)s + 1],
-                       rz = pz - xyz[4 * (size_t)s + 2];
-          if (rx * rx + ry * ry + rz * rz <= 1e-12) continue;
-          near_vec(mode, nq, rx, ry, rz, q ? q + (size_t)s * nq : nullptr,
-                   dip ? dip + (size_t)s * nq : nullptr, dip ? nrm[4 * (size_t)s] : 0.0,
-                   dip ? nrm[4 * (size_t)s + 1] : 0.0, dip ? nrm[4 * (size_t)s + 2] : 0.0, out);
-        }
-      }
-    }
-  }
+  near_sources<G>(lane, bi, bj, bk, level, start, end, [&](uint32_t s) {
+    const double rx = px - xyz[4 * (size_t)s], ry = py - xyz[4 * (size_t)s + 1],
+                 rz = pz - xyz[4 * (size_t)s + 2];
+    if (rx * rx + ry * ry + rz * rz <= 1e-12) return;
+    near_vec(CURL ? 4 | (mode & 2) : mode & 3, nq, rx, ry, rz,
+             q ? q + (size_t)s * nq : nullptr, dip ? dip + (size_t)s * nq : nullptr,
+             dip ? nrm[4 * (size_t)s] : 0.0, dip ? nrm[4 * (size_t)s + 1] : 0.0,
+             dip ? nrm[4 * (size_t)s + 2] : 0.0, out);
+  });
   double *o = f + (size_t)tid[t] * fstr;
-  for (int i = 0; i < nout; i++) o[i] += out[i];
+  const int nout = vec_width(mode, nq);
+#pragma unroll
+  for (int i = 0; i < NO; i++) {
+    if (i >= nout) break;
+    const double v = group_sum<G>(out[i]);
+    if (lane == 0) o[i] += v;
+  }
 }
 
 // direct sums with vector sources (src/direct-laplace.c:87-198, :200-336):
@@ -1068,6 +1121,59 @@ __global__ void k_d2f(const double *in, float *out, size_t n) {
 }  // namespace wbfmm
 
 using namespace wbfmm;
+
+// the factors' table, built by the first call that needs it (finished
+// before it is published: other streams read it then)
+static LapTab *g_laptab = nullptr;
+static std::mutex g_laptab_mu;
+
+static int lap_tab(const LapTab **out) {
+  std::lock_guard<std::mutex> lk(g_laptab_mu);
+  if (!g_laptab) {
+    LapTab *t = nullptr;
+    WBFMM_CHECK(hipMalloc((void **)&t, sizeof(LapTab)));
+    WBFMM_LAUNCH("lap_tab", k_lap_tab, dim3(nblk(kLapTabN * (2 * kLapTabN + 1), 256)),
+                 dim3(256), 0, t);
+    WBFMM_CHECK(hipStreamSynchronize(stream()));
+    g_laptab = t;
+  }
+  *out = g_laptab;
+  return 0;
+}
+
+template <typename T>
+static int lap_field(const char *name, const double *xt, const uint32_t *tid, unsigned n,
+                     const uint32_t *start, const uint32_t *end, const double *xyz,
+                     const double *q, const double *nrm, const double *dip, unsigned level,
+                     const double *x0, double D, int N, double rs, const T *mpr, int field,
+                     double *f, int fstr) {
+  if (N < 0 || N > kMaxN) return WBFMM_HIP_ERR_ORDER;
+  if (n == 0) return 0;
+  const LapTab *tab = nullptr;
+  const int rc = lap_tab(&tab);
+  if (rc) return rc;
+#define LAP_FIELD(G)                                                                          \
+  case G:                                                                                     \
+    WBFMM_LAUNCH(name, (k_lap_field<T, G>), dim3(nblk((size_t)n * G, 128)), dim3(128), 0, xt, \
+                 tid, n, start, end, xyz, q, nrm, dip, (int)level, x0[0], x0[1], x0[2], D, N, \
+                 rs, mpr, field, f, fstr, tab);                                               \
+    return 0;
+  // leaves of fewer than two targets: mostly expansion steps, whose
+  // scattered coefficient reads four lanes of a target share (1e6 targets
+  // at depth 7, order 12: 2.40 ms with one lane, 1.80 with two, 1.57 with
+  // four)
+  int g = field_lanes(n);
+  if (g < 4 && n >> 1 < (uint64_t)1 << (3 * level)) g = 4;
+  switch (n > (1u << 26) ? 1 : g) {
+    LAP_FIELD(1)
+    LAP_FIELD(2)
+    LAP_FIELD(4)
+    LAP_FIELD(8)
+    LAP_FIELD(16)
+  }
+#undef LAP_FIELD
+  return WBFMM_HIP_ERR_ARG;
+}
 
 // one wavefront per box: groups of 16 lanes up to order 15, 32 up to 31,
 // 64 above; LDS holds one expansion per group
@@ -1236,12 +1342,8 @@ int wbfmm_hip_lap_field(const double *xt, const uint32_t *tid, unsigned n,
                         const double *dip, unsigned level, const double *x0,
                         double D, int N, const double *mpr, int field,
                         double *f, int fstr) {
-  if (N < 0 || N > kMaxN) return WBFMM_HIP_ERR_ORDER;
-  if (n == 0) return 0;
-  WBFMM_LAUNCH("lap_l2p_p2p", k_lap_field<double>, dim3(nblk(n, 128)), dim3(128), 0,
-               xt, tid, n, start, end, xyz, q, nrm, dip, (int)level, x0[0],
-               x0[1], x0[2], D, N, 1.0, mpr, field, f, fstr);
-  return 0;
+  return lap_field<double>("lap_l2p_p2p", xt, tid, n, start, end, xyz, q, nrm, dip, level, x0, D, N,
+                           1.0, mpr, field, f, fstr);
 }
 
 int wbfmm_hip_lap_field_f32(const double *xt, const uint32_t *tid, unsigned n,
@@ -1250,13 +1352,9 @@ int wbfmm_hip_lap_field_f32(const double *xt, const uint32_t *tid, unsigned n,
                             const double *dip, unsigned level, const double *x0,
                             double D, int N, const float *mpr, int field,
                             double *f, int fstr) {
-  if (N < 0 || N > kMaxN) return WBFMM_HIP_ERR_ORDER;
-  if (n == 0) return 0;
   const double w = D / (double)(1u << level);
-  WBFMM_LAUNCH("lap_l2p_p2p_f32", k_lap_field<float>, dim3(nblk(n, 128)), dim3(128), 0,
-               xt, tid, n, start, end, xyz, q, nrm, dip, (int)level, x0[0],
-               x0[1], x0[2], D, N, 1.0 / w, mpr, field, f, fstr);
-  return 0;
+  return lap_field<float>("lap_l2p_p2p_f32", xt, tid, n, start, end, xyz, q, nrm, dip, level, x0, D,
+                          N, 1.0 / w, mpr, field, f, fstr);
 }
 
 int wbfmm_hip_to_f32(const double *in, float *out, size_t n) {
@@ -1276,9 +1374,24 @@ int wbfmm_hip_lap_field_vec(const double *xt, const uint32_t *tid, unsigned n,
       vec_width(mode, nq) > kVecMaxOut || fstr < vec_width(mode, nq) || ((mode & 4) && dip))
     return WBFMM_HIP_ERR_ARG;
   if (n == 0) return 0;
-  WBFMM_LAUNCH("lap_l2p_p2p_vec", k_lap_field_vec, dim3(nblk(n, 128)), dim3(128), 0, xt, tid, n,
-               start, end, xyz, q, nrm, dip, nq, (int)level, x0[0], x0[1], x0[2], D, N, mpr,
-               plane_stride, mode, f, fstr);
+  const LapTab *tab = nullptr;
+  const int rc = lap_tab(&tab);
+  if (rc) return rc;
+  const int g = n > (1u << 26) ? 1 : field_lanes(n);
+#define LAP_VEC(CU, G)                                                                        \
+  WBFMM_LAUNCH("lap_l2p_p2p_vec", (k_lap_field_vec<CU, G>), dim3(nblk((size_t)n * G, 128)),   \
+               dim3(128), 0, xt, tid, n, start, end, xyz, q, nrm, dip, nq, (int)level, x0[0], \
+               x0[1], x0[2], D, N, mpr, plane_stride, mode, f, fstr, tab)
+  if (mode & 4) {
+    if (g >= 16) LAP_VEC(true, 16);
+    else if (g >= 4) LAP_VEC(true, 4);
+    else LAP_VEC(true, 1);
+  } else {
+    if (g >= 16) LAP_VEC(false, 16);
+    else if (g >= 4) LAP_VEC(false, 4);
+    else LAP_VEC(false, 1);
+  }
+#undef LAP_VEC
   return 0;
 }
 
