@@ -109,6 +109,28 @@ int wbfmm_hip_gather_strided(const double *src, int sstr, int ncomp,
    arrays 8^level, zeroed here first) */
 int wbfmm_hip_box_ranges(const uint64_t *codes, unsigned n, unsigned level,
                          uint32_t *start, uint32_t *end);
+/* points (host or device, byte stride) in Morton order: positions (4
+   doubles each), codes and caller indices; raw: scratch of 4 n doubles;
+   *nbad: points outside the domain.  Returns when the points are read and
+   *nbad is known. */
+int wbfmm_hip_points_sorted(const void *pts, size_t pstr, unsigned n, const double *x0, double D,
+                            double *raw, double *xyz, uint64_t *codes, uint32_t *idx,
+                            unsigned *nbad);
+/* dense [start, end) ranges (0, 0 where empty) and ascending lists of the
+   occupied boxes of the levels lo..hi (at most 10) over the sorted codes,
+   all levels at once; arrays by level; tot[10 l]: boxes listed (device) */
+int wbfmm_hip_tree_levels(const uint64_t *codes, unsigned n, unsigned lo, unsigned hi,
+                          uint32_t *const *start, uint32_t *const *end, uint32_t *const *occ,
+                          uint32_t *tot);
+/* with the ranges above, for the levels 0..hi: flag 1 where a box holds
+   sources or targets (their sorted codes), the flagged boxes ascending
+   (act) and grouped by child digit (cls, as wbfmm_hip_split_classes groups
+   them); tot[10 l + 1]: boxes listed, tot[10 l + 2 + c]: those of digit c */
+int wbfmm_hip_tree_targets(const uint64_t *tcodes, unsigned n, unsigned hi,
+                           uint32_t *const *start, uint32_t *const *end, uint32_t *const *flag,
+                           uint32_t *const *act, uint32_t *const *cls, uint32_t *tot);
+/* every box of a level >= 1 grouped by child digit (8^(level-1) each) */
+int wbfmm_hip_all_classes(unsigned level, uint32_t *out);
 /* compact list of the boxes with end>start (or flag!=0 when flag is not
    NULL) in Morton order; *count (host) gets the list length */
 int wbfmm_hip_compact_boxes(const uint32_t *start, const uint32_t *end,

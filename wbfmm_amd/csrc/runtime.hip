@@ -196,6 +196,196 @@ __global__ void k_mark_boxes(const uint64_t *codes, unsigned n, int shift,
   flag[codes[i] >> shift] = 1u;
 }
 
+// ---- box ranges and box lists of all levels of a tree at once ----------------
+//
+// The boxes of the levels lo..lo+n-1 form one grid of 2048-box chunks.  Three
+// launches, whatever the depth: the ranges (or flags) of every box with the
+// chunk's counts; an exclusive scan of the counts over each level's chunks,
+// one block a level, whose totals go to tot; the lists, each box placed by
+// its chunk's base and its rank in the chunk.  Counts stay on the device and
+// reach the host in one copy.  Level by level, with a library scan over a
+// flag array and the count read back at each level, a tree of depth 2 took
+// some 60 launches and copies and 7 waits for the device, twice over with a
+// target list.
+constexpr unsigned kLevChunk = 2048, kLevThreads = 256;
+constexpr int kLevMax = 17;
+struct LevelSet {
+  unsigned lo, n;
+  unsigned chunk0[kLevMax + 1];
+  uint32_t *start[kLevMax], *end[kLevMax];                 // ranges over the sources
+  uint32_t *list[kLevMax], *flag[kLevMax], *cls[kLevMax];  // lists; flags and class lists of targets
+};
+
+// first i with codes[i] >= key
+__device__ __forceinline__ unsigned code_bound(const uint64_t *__restrict__ codes, unsigned n,
+                                               uint64_t key) {
+  unsigned a = 0, b = n;
+  while (a < b) {
+    const unsigned m = a + (b - a) / 2;
+    if (codes[m] < key)
+      a = m + 1;
+    else
+      b = m;
+  }
+  return a;
+}
+
+// level index (from lo) of the block's chunk, its first box and the number
+// of boxes of the level
+__device__ __forceinline__ int chunk_level(const LevelSet &L, unsigned &box0, unsigned &nb) {
+  int l = 0;
+  while (l + 1 < (int)L.n && blockIdx.x >= L.chunk0[l + 1]) l++;
+  box0 = (blockIdx.x - L.chunk0[l]) * kLevChunk;
+  nb = 1u << (3 * (L.lo + l));
+  return l;
+}
+
+// [start, end) of every box over the sorted codes (0, 0 for an empty box)
+__global__ __launch_bounds__(kLevThreads) void k_level_ranges(const uint64_t *__restrict__ codes,
+                                                              unsigned n, LevelSet L,
+                                                              uint32_t *__restrict__ cnt) {
+  __shared__ unsigned bound[kLevThreads + 1], total;
+  unsigned box0, nb;
+  const int l = chunk_level(L, box0, nb), shift = 3 * (20 - (int)(L.lo + l));
+  if (threadIdx.x == 0) total = 0;
+  for (unsigned i = 0; i < kLevChunk; i += kLevThreads) {
+    const unsigned b = box0 + i + threadIdx.x;
+    __syncthreads();
+    if (b < nb) {
+      bound[threadIdx.x] = code_bound(codes, n, (uint64_t)b << shift);
+      if (threadIdx.x == kLevThreads - 1 || b == nb - 1)
+        bound[threadIdx.x + 1] = code_bound(codes, n, ((uint64_t)b + 1) << shift);
+    }
+    __syncthreads();
+    bool occ = false;
+    if (b < nb) {
+      const unsigned s = bound[threadIdx.x], e = bound[threadIdx.x + 1];
+      occ = e > s;
+      L.start[l][b] = occ ? s : 0u;
+      L.end[l][b] = occ ? e : 0u;
+    }
+    const unsigned c = (unsigned)__popcll(__ballot(occ));
+    if ((threadIdx.x & 63) == 0 && c) atomicAdd(&total, c);
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) cnt[blockIdx.x] = total;
+}
+
+// flag of every box: 1 where it holds sources or targets; counts of the
+// flagged boxes and of those of each child digit (9 per chunk)
+__global__ __launch_bounds__(kLevThreads) void k_level_flags(const uint64_t *__restrict__ tcodes,
+                                                             unsigned n, LevelSet L,
+                                                             uint32_t *__restrict__ cnt) {
+  __shared__ unsigned total[9];
+  unsigned box0, nb;
+  const int l = chunk_level(L, box0, nb), shift = 3 * (20 - (int)(L.lo + l));
+  if (threadIdx.x < 9) total[threadIdx.x] = 0;
+  __syncthreads();
+  for (unsigned i = 0; i < kLevChunk; i += kLevThreads) {
+    const unsigned b = box0 + i + threadIdx.x;
+    bool on = false;
+    if (b < nb) {
+      on = L.end[l][b] > L.start[l][b];
+      if (!on) {
+        const unsigned s = code_bound(tcodes, n, (uint64_t)b << shift);
+        on = s < n && (tcodes[s] >> shift) == b;
+      }
+      L.flag[l][b] = on ? 1u : 0u;
+    }
+    const unsigned long long m = __ballot(on);
+    const int lane = threadIdx.x & 63;
+    if (lane < 9 && m) {
+      const unsigned c = (unsigned)__popcll(lane ? m & (0x0101010101010101ull << (lane - 1)) : m);
+      if (c) atomicAdd(&total[lane], c);
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x < 9) cnt[9 * (size_t)blockIdx.x + threadIdx.x] = total[threadIdx.x];
+}
+
+// counts of F fields per chunk -> exclusive sums over the chunks of the
+// level; totals to tot[10 level + at + field] (block: a level)
+template <int F>
+__global__ __launch_bounds__(1024) void k_chunk_scan(LevelSet L, uint32_t *__restrict__ cnt,
+                                                     uint32_t *__restrict__ tot, int at) {
+  __shared__ unsigned wsum[16];
+  const int l = blockIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const unsigned c0 = L.chunk0[l], c1 = L.chunk0[l + 1];
+  for (int f = 0; f < F; f++) {
+    unsigned base = 0;
+    for (unsigned c = c0; c < c1; c += 1024) {
+      const unsigned k = c + threadIdx.x;
+      const unsigned v = k < c1 ? cnt[(size_t)k * F + f] : 0u;
+      unsigned x = v;
+      for (int h = 1; h < 64; h *= 2) {
+        const unsigned y = __shfl_up(x, h);
+        if (lane >= h) x += y;
+      }
+      if (lane == 63) wsum[w] = x;
+      __syncthreads();
+      unsigned before = base, all = 0;
+      for (int i = 0; i < 16; i++) {
+        if (i < w) before += wsum[i];
+        all += wsum[i];
+      }
+      if (k < c1) cnt[(size_t)k * F + f] = before + x - v;
+      base += all;
+      __syncthreads();
+    }
+    if (threadIdx.x == 0) tot[10 * (L.lo + l) + at + f] = base;
+  }
+}
+
+// boxes in ascending order where end > start (CLS 0), or the flagged boxes
+// in ascending order and grouped by child digit (CLS 1)
+template <int CLS>
+__global__ __launch_bounds__(kLevThreads) void k_level_lists(LevelSet L,
+                                                             const uint32_t *__restrict__ base,
+                                                             const uint32_t *__restrict__ tot) {
+  constexpr int F = CLS ? 9 : 1, W = kLevThreads / 64;
+  __shared__ unsigned wc[W][F];
+  unsigned box0, nb;
+  const int l = chunk_level(L, box0, nb), lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const unsigned digit = threadIdx.x & 7;
+  const unsigned long long below = (1ull << lane) - 1, mine = 0x0101010101010101ull << digit;
+  unsigned at = base[(size_t)blockIdx.x * F], cat = 0;
+  if (CLS) {
+    cat = base[(size_t)blockIdx.x * F + 1 + digit];
+    for (unsigned c = 0; c < digit; c++) cat += tot[10 * (L.lo + l) + 2 + c];
+  }
+  for (unsigned i = 0; i < kLevChunk; i += kLevThreads) {
+    const unsigned b = box0 + i + threadIdx.x;
+    bool on = false;
+    if (b < nb) on = CLS ? L.flag[l][b] != 0 : L.end[l][b] > L.start[l][b];
+    const unsigned long long m = __ballot(on);
+    __syncthreads();
+    if (lane < F)
+      wc[w][lane] = (unsigned)__popcll(lane ? m & (0x0101010101010101ull << (lane - 1)) : m);
+    __syncthreads();
+    unsigned r = (unsigned)__popcll(m & below), cr = (unsigned)__popcll(m & below & mine);
+    for (int j = 0; j < W; j++) {
+      if (j < w) {
+        r += wc[j][0];
+        if (CLS) cr += wc[j][F > 1 ? 1 + digit : 0];
+      }
+    }
+    if (on) {
+      L.list[l][at + r] = b;
+      if (CLS) L.cls[l][cat + cr] = b;
+    }
+    for (int j = 0; j < W; j++) {
+      at += wc[j][0];
+      if (CLS) cat += wc[j][F > 1 ? 1 + digit : 0];
+    }
+  }
+}
+
+// every box of a level, grouped by child digit
+__global__ void k_all_classes(unsigned nb, uint32_t *out) {
+  const unsigned i = blockIdx.x * blockDim.x + threadIdx.x, per = nb / 8;
+  if (i < nb) out[i] = 8 * (i % per) + i / per;
+}
+
 // per-block minimum and maximum of the 3 coordinates: out[6 b + 0..2] min,
 // out[6 b + 3..5] max
 __global__ void k_bounds(const char *pts, size_t pstr, unsigned n,
@@ -577,6 +767,112 @@ int wbfmm_hip_compact_boxes(const uint32_t *start, const uint32_t *end,
   dfree(pos);
   WBFMM_CHECK(hipStreamSynchronize(stream()));
   *count = lastf + lastp;
+  return 0;
+}
+
+// points in Morton order: positions (4 doubles), codes and caller indices;
+// raw: scratch of 4 n doubles; *nbad: points outside the domain
+int wbfmm_hip_points_sorted(const void *pts, size_t pstr, unsigned n, const double *x0, double D,
+                            double *raw, double *xyz, uint64_t *codes, uint32_t *idx,
+                            unsigned *nbad) {
+  *nbad = 0;
+  if (n == 0) return 0;
+  size_t sort_bytes = 0;
+  WBFMM_CHECK(rocprim::radix_sort_pairs(nullptr, sort_bytes, codes, codes, idx, idx, n, 0, 60,
+                                        stream()));
+  // one block: counter, unsorted codes and indices, the caller's strided
+  // host block as it lies, the sort's scratch
+  const bool host = !wbfmm_hip_is_device(pts);
+  auto round = [](size_t b) { return (b + 255) / 256 * 256; };
+  const size_t o_codes = 256, o_idx = o_codes + round(8 * (size_t)n),
+               o_pts = o_idx + round(4 * (size_t)n),
+               pbytes = host ? (size_t)(n - 1) * pstr + 3 * sizeof(double) : 0,
+               o_sort = o_pts + round(pbytes);
+  char *tmp = nullptr;
+  if (dmalloc((void **)&tmp, o_sort + sort_bytes)) return WBFMM_HIP_ERR_NOMEM;
+  uint64_t *tcodes = (uint64_t *)(tmp + o_codes);
+  uint32_t *tidx = (uint32_t *)(tmp + o_idx);
+  const char *dpts = (const char *)pts;
+  if (host) {
+    WBFMM_CHECK(hipMemcpyAsync(tmp + o_pts, pts, pbytes, hipMemcpyHostToDevice, stream()));
+    dpts = tmp + o_pts;
+  }
+  WBFMM_CHECK(hipMemsetAsync(tmp, 0, sizeof(unsigned), stream()));
+  WBFMM_LAUNCH("tree_morton", k_morton, dim3(nblk(n, 256)), dim3(256), 0, dpts, pstr, n, x0[0],
+               x0[1], x0[2], D, raw, tcodes, tidx, (unsigned *)tmp);
+  timing_begin("tree_sort");
+  WBFMM_CHECK(rocprim::radix_sort_pairs(tmp + o_sort, sort_bytes, tcodes, codes, tidx, idx, n, 0,
+                                        60, stream()));
+  timing_end("tree_sort");
+  WBFMM_LAUNCH("gather4", k_gather4, dim3(nblk(n, 256)), dim3(256), 0, raw, idx, n, xyz);
+  WBFMM_CHECK(hipMemcpyAsync(nbad, tmp, sizeof(unsigned), hipMemcpyDeviceToHost, stream()));
+  dfree(tmp);
+  WBFMM_CHECK(hipStreamSynchronize(stream()));
+  return 0;
+}
+
+static int level_set(LevelSet &L, unsigned lo, unsigned hi, unsigned *chunks) {
+  if (hi < lo || hi > (unsigned)kMortonAddMaxLevel) return WBFMM_HIP_ERR_ARG;
+  L.lo = lo;
+  L.n = hi - lo + 1;
+  unsigned c = 0;
+  for (unsigned i = 0; i < L.n; i++) {
+    L.chunk0[i] = c;
+    c += ((1u << (3 * (lo + i))) + kLevChunk - 1) / kLevChunk;
+  }
+  L.chunk0[L.n] = c;
+  *chunks = c;
+  return 0;
+}
+
+int wbfmm_hip_tree_levels(const uint64_t *codes, unsigned n, unsigned lo, unsigned hi,
+                          uint32_t *const *start, uint32_t *const *end, uint32_t *const *occ,
+                          uint32_t *tot) {
+  LevelSet L{};
+  unsigned chunks = 0;
+  if (level_set(L, lo, hi, &chunks)) return WBFMM_HIP_ERR_ARG;
+  for (unsigned i = 0; i < L.n; i++) {
+    L.start[i] = start[lo + i];
+    L.end[i] = end[lo + i];
+    L.list[i] = occ[lo + i];
+  }
+  uint32_t *cnt = nullptr;
+  if (dmalloc((void **)&cnt, sizeof(uint32_t) * chunks)) return WBFMM_HIP_ERR_NOMEM;
+  WBFMM_LAUNCH("tree_box_ranges", k_level_ranges, dim3(chunks), dim3(kLevThreads), 0, codes, n, L,
+               cnt);
+  WBFMM_LAUNCH("tree_box_scan", k_chunk_scan<1>, dim3(L.n), dim3(1024), 0, L, cnt, tot, 0);
+  WBFMM_LAUNCH("tree_box_lists", k_level_lists<0>, dim3(chunks), dim3(kLevThreads), 0, L, cnt, tot);
+  dfree(cnt);
+  return 0;
+}
+
+int wbfmm_hip_tree_targets(const uint64_t *tcodes, unsigned n, unsigned hi,
+                           uint32_t *const *start, uint32_t *const *end, uint32_t *const *flag,
+                           uint32_t *const *act, uint32_t *const *cls, uint32_t *tot) {
+  LevelSet L{};
+  unsigned chunks = 0;
+  if (level_set(L, 0, hi, &chunks)) return WBFMM_HIP_ERR_ARG;
+  for (unsigned i = 0; i < L.n; i++) {
+    L.start[i] = start[i];
+    L.end[i] = end[i];
+    L.flag[i] = flag[i];
+    L.list[i] = act[i];
+    L.cls[i] = cls[i];
+  }
+  uint32_t *cnt = nullptr;
+  if (dmalloc((void **)&cnt, sizeof(uint32_t) * 9 * chunks)) return WBFMM_HIP_ERR_NOMEM;
+  WBFMM_LAUNCH("tree_box_flags", k_level_flags, dim3(chunks), dim3(kLevThreads), 0, tcodes, n, L,
+               cnt);
+  WBFMM_LAUNCH("tree_box_scan", k_chunk_scan<9>, dim3(L.n), dim3(1024), 0, L, cnt, tot, 1);
+  WBFMM_LAUNCH("tree_box_lists", k_level_lists<1>, dim3(chunks), dim3(kLevThreads), 0, L, cnt, tot);
+  dfree(cnt);
+  return 0;
+}
+
+int wbfmm_hip_all_classes(unsigned level, uint32_t *out) {
+  if (level < 1 || level > (unsigned)kMortonAddMaxLevel) return WBFMM_HIP_ERR_ARG;
+  const unsigned nb = 1u << (3 * level);
+  WBFMM_LAUNCH("tree_all_classes", k_all_classes, dim3(nblk(nb, 256)), dim3(256), 0, nb, out);
   return 0;
 }
 

@@ -204,7 +204,7 @@ size_t footprint(const wbfmm_serve_request_t &r, const Plan &p) {
     // mixed-precision Helmholtz keeps the high-frequency levels in FP64
     const double ka = r.k * 0.5 * std::sqrt(3.0) * p.D / (double)(1u << l);
     const size_t es = p.precision == 32 && (cplx == 1 || ka <= 2.0) ? 4 : 8;
-    b += nb * (2 * C * es * cplx + 16);
+    b += nb * (2 * C * es * cplx + 24);
     const size_t split_targets = std::min<size_t>(nb, 16384);
     const size_t level_tr = nb / 8 + 4 * nb + 8 * split_targets * C * es * cplx;
     transient = std::max(transient, level_tr);

@@ -120,12 +120,23 @@ typedef struct {
   uint32_t *d_start[WBFMM_TREE_MAX_DEPTH + 1], *d_end[WBFMM_TREE_MAX_DEPTH + 1];
   uint32_t *d_occ[WBFMM_TREE_MAX_DEPTH + 1];
   unsigned nocc[WBFMM_TREE_MAX_DEPTH + 1];
+  /* levels 0..built-1 hold the ranges and lists of the current points
+     (refine leaves them to the first call that reads them: build_levels);
+     d_tot: box counts per level on the device (wbfmm_hip_tree_levels, _targets),
+     read into nocc, nact and cls_* by tree_counts when counts_due */
+  unsigned built;
+  uint32_t *d_tot;
+  int counts_due;
   /* boxes holding sources or registered targets; when no target list is
      registered every box is a possible target and these stay NULL */
   uint32_t *d_flag[WBFMM_TREE_MAX_DEPTH + 1];
   uint32_t *d_act[WBFMM_TREE_MAX_DEPTH + 1];
   unsigned nact[WBFMM_TREE_MAX_DEPTH + 1];
+  /* d_act grouped by child digit */
+  uint32_t *d_cls[WBFMM_TREE_MAX_DEPTH + 1];
+  unsigned cls_start[WBFMM_TREE_MAX_DEPTH + 1][8], cls_count[WBFMM_TREE_MAX_DEPTH + 1][8];
   int have_targets; /* d_flag/d_act describe the current points */
+  unsigned tgt_levels; /* the levels 0..tgt_levels-1 of them */
   size_t mps_bytes[WBFMM_TREE_MAX_DEPTH + 1], mpr_bytes[WBFMM_TREE_MAX_DEPTH + 1];
   double *d_q, *d_dip; /* strengths in sorted order */
   unsigned cap_q, cap_dip;
@@ -537,6 +548,7 @@ wbfmm_tree_t *wbfmm_tree_new(gdouble *x, gdouble D, guint maxpoints)
   HIPOK(wbfmm_hip_malloc((void **)&td->d_xyz_raw, sizeof(double) * 4 * (maxpoints ? maxpoints : 1)));
   HIPOK(wbfmm_hip_malloc((void **)&td->d_codes, sizeof(uint64_t) * (maxpoints ? maxpoints : 1)));
   HIPOK(wbfmm_hip_malloc((void **)&td->d_idx, sizeof(uint32_t) * (maxpoints ? maxpoints : 1)));
+  HIPOK(wbfmm_hip_malloc((void **)&td->d_tot, sizeof(uint32_t) * 10 * (WBFMM_TREE_MAX_DEPTH + 1)));
   return t;
 }
 
@@ -546,18 +558,49 @@ gint wbfmm_tree_host_mirror(wbfmm_tree_t *t, gboolean on)
   return 0;
 }
 
-static void level_ranges(tree_dev *td, unsigned l)
+/* box ranges and occupied lists of the levels up to the tree's depth, as far
+   as they are not built, without waiting for the device */
+static void build_levels(tree_dev *td)
 {
-  size_t nb = (size_t)1 << (3 * l);
-  if (!td->d_start[l]) {
-    HIPOK(wbfmm_hip_malloc((void **)&td->d_start[l], sizeof(uint32_t) * nb));
-    HIPOK(wbfmm_hip_malloc((void **)&td->d_end[l], sizeof(uint32_t) * nb));
-    HIPOK(wbfmm_hip_malloc((void **)&td->d_occ[l], sizeof(uint32_t) * nb));
+  const unsigned lo = td->built, hi = td->t.depth;
+  unsigned l;
+  if (lo > hi) return;
+  for (l = lo; l <= hi; l++)
+    if (!td->d_start[l]) {
+      /* start, end and list in one block */
+      const size_t nb = (size_t)1 << (3 * l);
+      HIPOK(wbfmm_hip_malloc((void **)&td->d_start[l], sizeof(uint32_t) * 3 * nb));
+      td->d_end[l] = td->d_start[l] + nb;
+      td->d_occ[l] = td->d_end[l] + nb;
+    }
+  HIPOK(wbfmm_hip_tree_levels(td->d_codes, td->t.npoints, lo, hi, td->d_start, td->d_end,
+                              td->d_occ, td->d_tot));
+  td->built = hi + 1;
+  td->counts_due = 1;
+}
+
+/* every level built and its box counts on the host (waits for the device
+   once after a change of the points or targets) */
+static void tree_counts(tree_dev *td)
+{
+  uint32_t tot[10 * (WBFMM_TREE_MAX_DEPTH + 1)];
+  unsigned l, c;
+  build_levels(td);
+  if (!td->counts_due) return;
+  HIPOK(wbfmm_hip_memcpy(tot, td->d_tot, sizeof(uint32_t) * 10 * td->built));
+  for (l = 0; l < td->built; l++) {
+    unsigned at = 0;
+    td->nocc[l] = tot[10 * l];
+    if (!td->have_targets) continue;
+    /* levels added after the targets were registered have none */
+    td->nact[l] = l < td->tgt_levels ? tot[10 * l + 1] : 0;
+    for (c = 0; c < 8; c++) {
+      td->cls_start[l][c] = at;
+      td->cls_count[l][c] = l < td->tgt_levels ? tot[10 * l + 2 + c] : 0;
+      at += td->cls_count[l][c];
+    }
   }
-  HIPOK(wbfmm_hip_box_ranges(td->d_codes, td->t.npoints, l, td->d_start[l],
-                             td->d_end[l]));
-  HIPOK(wbfmm_hip_compact_boxes(td->d_start[l], td->d_end[l], NULL, l,
-                                td->d_occ[l], &td->nocc[l]));
+  td->counts_due = 0;
 }
 
 static void mirror_level(tree_dev *td, unsigned l)
@@ -566,16 +609,16 @@ static void mirror_level(tree_dev *td, unsigned l)
   uint32_t *s, *e;
   wbfmm_box_t *boxes = td->t.boxes[l];
   if (!td->host_mirror || !boxes) return;
-  s = malloc(sizeof(uint32_t) * nb);
-  e = malloc(sizeof(uint32_t) * nb);
-  HIPOK(wbfmm_hip_memcpy(s, td->d_start[l], sizeof(uint32_t) * nb));
-  HIPOK(wbfmm_hip_memcpy(e, td->d_end[l], sizeof(uint32_t) * nb));
+  build_levels(td);
+  s = malloc(sizeof(uint32_t) * 2 * nb);
+  if (!s) WBFMM_FATAL("out of host memory");
+  e = s + nb; /* the two arrays are one block on the device */
+  HIPOK(wbfmm_hip_memcpy(s, td->d_start[l], sizeof(uint32_t) * 2 * nb));
   for (b = 0; b < nb; b++) {
     boxes[b].n = e[b] - s[b];
     boxes[b].i = boxes[b].n ? s[b] : 0;
   }
   free(s);
-  free(e);
 }
 
 static gint add_points_dbl(wbfmm_tree_t *t, gpointer pts, gsize pstr, gpointer normals,
@@ -603,19 +646,18 @@ static gint add_points_dbl(wbfmm_tree_t *t, gpointer pts, gsize pstr, gpointer n
      any registered target list must be added again */
   t->depth = 0;
   td->have_targets = 0;
+  td->built = 0;
   t->npoints = npts;
   t->points = (char *)pts;
   t->pstr = pstr;
   t->normals = (char *)normals;
   t->nstr = nstr;
   t->sorted = sorted;
-  HIPOK(wbfmm_hip_morton(pts, pstr, npts, x0, t->D, td->d_xyz_raw,
-                         td->d_codes, td->d_idx, &nbad));
+  HIPOK(wbfmm_hip_points_sorted(pts, pstr, npts, x0, t->D, td->d_xyz_raw, td->d_xyz,
+                                td->d_codes, td->d_idx, &nbad));
   if (nbad)
     WBFMM_FATAL("%u points do not lie in box of width %g at (%g,%g,%g)", nbad,
                 t->D, x0[0], x0[1], x0[2]);
-  HIPOK(wbfmm_hip_sort(td->d_codes, td->d_idx, npts));
-  HIPOK(wbfmm_hip_gather4(td->d_xyz_raw, td->d_idx, npts, td->d_xyz));
   if (normals) {
     if (!td->d_nrm)
       HIPOK(wbfmm_hip_malloc((void **)&td->d_nrm, sizeof(double) * 4 * (t->maxpoints ? t->maxpoints : 1)));
@@ -626,7 +668,6 @@ static gint add_points_dbl(wbfmm_tree_t *t, gpointer pts, gsize pstr, gpointer n
     HIPOK(wbfmm_hip_memcpy(t->ip, td->d_idx, sizeof(uint32_t) * npts));
   t->boxes[0][0].i = 0;
   t->boxes[0][0].n = npts;
-  level_ranges(td, 0);
   return 0;
 }
 
@@ -691,10 +732,11 @@ gint wbfmm_tree_refine(wbfmm_tree_t *t)
   unsigned l = t->depth + 1;
   if (l > WBFMM_TREE_MAX_DEPTH)
     WBFMM_FATAL("tree depth would exceed %d", WBFMM_TREE_MAX_DEPTH);
+  if (l > M2L_MFMA_MAX_LEVEL)
+    WBFMM_FATAL("dense levels are limited to %d", M2L_MFMA_MAX_LEVEL);
   if (td->host_mirror && !t->boxes[l])
     t->boxes[l] = calloc((size_t)1 << (3 * l), sizeof(wbfmm_box_t));
   t->depth = l;
-  level_ranges(td, l);
   mirror_level(td, l);
   return 0;
 }
@@ -912,6 +954,7 @@ gint wbfmm_tree_laplace_leaf_expansions(wbfmm_tree_t *t, gdouble *src,
     WBFMM_FATAL("tree has invalid number of components in source terms (%d)", t->nq);
   if (t->problem != WBFMM_PROBLEM_LAPLACE) WBFMM_FATAL("tree is not a Laplace tree");
   if (!t->mps[d]) WBFMM_FATAL("coefficients not initialised at level %u", d);
+  tree_counts(td);
   if (zero_expansions) HIPOK(wbfmm_hip_memset(t->mps[d], 0, td->mps_bytes[d]));
   if (src == NULL && dipoles == NULL) return 0;
   if (t->normals == NULL && dipoles != NULL)
@@ -1311,6 +1354,7 @@ gint wbfmm_laplace_upward_pass(wbfmm_tree_t *t, wbfmm_shift_operators_t *op,
   if ((int)t->order_s[level] > od->lay.L || (int)t->order_s[level - 1] > od->lay.L)
     WBFMM_FATAL("operators built to order %d, tree needs %u", od->lay.L,
                 t->order_s[level] > t->order_s[level - 1] ? t->order_s[level] : t->order_s[level - 1]);
+  tree_counts(td);
   if (td->prec32) {
     int N = (int)t->order_s[level];
     if (t->order_s[level - 1] != t->order_s[level] || !mfma_order(N))
@@ -1364,6 +1408,39 @@ static uint32_t *all_boxes(unsigned level, unsigned *n)
   return list;
 }
 
+/* the boxes of all_boxes grouped by child digit, one list per level, built
+   by the first call that needs it (finished before it is published) and
+   kept */
+static uint32_t *g_all_cls[M2L_MFMA_MAX_LEVEL + 1];
+
+/* the target boxes of a level grouped by child digit: list, start and
+   count of each digit */
+static const uint32_t *target_classes(tree_dev *td, unsigned level, unsigned *cstart,
+                                      unsigned *ccount)
+{
+  unsigned c;
+  tree_counts(td);
+  if (td->have_targets) {
+    memcpy(cstart, td->cls_start[level], sizeof(unsigned) * 8);
+    memcpy(ccount, td->cls_count[level], sizeof(unsigned) * 8);
+    return td->d_cls[level];
+  }
+  mu_lock(&g_all_mu);
+  if (!g_all_cls[level]) {
+    uint32_t *d = NULL;
+    HIPOK(wbfmm_hip_malloc((void **)&d, sizeof(uint32_t) << (3 * level)));
+    HIPOK(wbfmm_hip_all_classes(level, d));
+    HIPOK(wbfmm_hip_sync());
+    g_all_cls[level] = d;
+  }
+  mu_unlock(&g_all_mu);
+  for (c = 0; c < 8; c++) {
+    ccount[c] = 1u << (3 * level - 3);
+    cstart[c] = c * ccount[c];
+  }
+  return g_all_cls[level];
+}
+
 /* FP64 L2L of one component from the parents tl at `level' (in) into
    their children at level+1 (out, added) */
 static void lap_l2l_plane(wbfmm_tree_t *t, ops_dev *od, guint level, const uint32_t *tl,
@@ -1400,6 +1477,7 @@ static gint lap_downward(wbfmm_tree_t *t, wbfmm_shift_operators_t *op,
     WBFMM_FATAL("coefficients not initialised at level %u", level);
   if ((int)t->order_s[level] > od->lay.L || (int)t->order_r[level] > od->lay.L)
     WBFMM_FATAL("operators built to order %d", od->lay.L);
+  tree_counts(td);
   if (td->have_targets) {
     tl = td->d_act[level];
     nt = td->nact[level];
@@ -1409,21 +1487,19 @@ static gint lap_downward(wbfmm_tree_t *t, wbfmm_shift_operators_t *op,
   if (td->prec32) {
     int N = (int)t->order_s[level];
     unsigned cstart[8], ccount[8];
-    uint32_t *cls;
+    const uint32_t *cls;
     if (t->order_r[level] != t->order_s[level] || !mfma_order(N) ||
         (level < t->depth && t->order_r[level + 1] != t->order_r[level]))
       WBFMM_FATAL("FP32 passes need equal orders in %d..%d", M2L_MFMA_MIN, SHIFT_MFMA_MAX);
     if (level > M2L_MFMA_MAX_LEVEL)
       WBFMM_FATAL("FP32 passes serve levels up to %d", M2L_MFMA_MAX_LEVEL);
     ensure_f32_tables(od, N);
-    HIPOK(wbfmm_hip_malloc((void **)&cls, sizeof(uint32_t) * (nt ? nt : 1)));
-    HIPOK(wbfmm_hip_split_classes(tl, nt, cls, cstart, ccount));
+    cls = target_classes(td, level, cstart, ccount);
     HIPOK(wbfmm_hip_lap_m2l_mfma_f32(cls, cstart, ccount, td->d_start[level],
                                      td->d_end[level], level, N,
                                      (const float *)t->mps[level], (float *)t->mpr[level],
                                      od->m2l_plan_dev[N], od->f_A1[N], od->f_A3[N],
                                      od->f_A2[N], od->f_CS[N], od->m2l_plan[N]));
-    wbfmm_hip_free(cls);
     if (level == t->depth) return 0;
     if (!t->mpr[level + 1]) WBFMM_FATAL("coefficients not initialised at level %u", level + 1);
     HIPOK(wbfmm_hip_lap_shift_mfma_f32(1, tl, nt, NULL, NULL,
@@ -1439,10 +1515,9 @@ static gint lap_downward(wbfmm_tree_t *t, wbfmm_shift_operators_t *op,
        every component) */
     int N = (int)t->order_s[level];
     unsigned cstart[8], ccount[8], c;
-    uint32_t *cls;
+    const uint32_t *cls;
     ensure_m2l_plan(od, N);
-    HIPOK(wbfmm_hip_malloc((void **)&cls, sizeof(uint32_t) * (nt ? nt : 1)));
-    HIPOK(wbfmm_hip_split_classes(tl, nt, cls, cstart, ccount));
+    cls = target_classes(td, level, cstart, ccount);
     for (c = 0; c < t->nq; c++)
       HIPOK(wbfmm_hip_lap_m2l_mfma(cls, cstart, ccount, td->d_start[level],
                                    td->d_end[level], level, t->D, N,
@@ -1450,7 +1525,6 @@ static gint lap_downward(wbfmm_tree_t *t, wbfmm_shift_operators_t *op,
                                    od->m2l_plan_dev[N], od->m2l_A1[N], od->m2l_A3[N],
                                    m2l_coax(od, N, t->D / (double)(1u << level)),
                                    od->m2l_CS[N], od->m2l_plan[N]));
-    wbfmm_hip_free(cls);
   } else {
     unsigned c;
     ensure_lap_coax(od);
@@ -1504,12 +1578,12 @@ static void stage_targets(const void *xt, size_t tstr, unsigned n,
   HIPOK(wbfmm_hip_malloc((void **)dx, sizeof(double) * 4 * (n ? n : 1)));
   HIPOK(wbfmm_hip_malloc((void **)did, sizeof(uint32_t) * (n ? n : 1)));
   HIPOK(wbfmm_hip_malloc((void **)dcodes, sizeof(uint64_t) * (n ? n : 1)));
-  HIPOK(wbfmm_hip_morton(xt, tstr, n, x0, D, raw, *dcodes, *did, &nbad));
+  if (sort_them)
+    HIPOK(wbfmm_hip_points_sorted(xt, tstr, n, x0, D, raw, *dx, *dcodes, *did, &nbad));
+  else
+    HIPOK(wbfmm_hip_morton(xt, tstr, n, x0, D, *dx, *dcodes, *did, &nbad));
   if (nbad)
     WBFMM_FATAL("%u target points do not lie in the tree's domain", nbad);
-  if (sort_them) HIPOK(wbfmm_hip_sort(*dcodes, *did, n));
-  HIPOK(wbfmm_hip_gather4(raw, *did, n, *dx));
-  HIPOK(wbfmm_hip_sync());
   wbfmm_hip_free(raw);
 }
 
@@ -1552,6 +1626,7 @@ static void lap_field_run(tree_dev *td, const double *dxt,
   int staged;
   size_t nelem;
   if (!t->mpr[lv]) WBFMM_FATAL("coefficients not initialised at level %u", lv);
+  build_levels(td);
   if (t->normals == NULL && d != NULL)
     WBFMM_FATAL("no normals in tree but dipole strengths specified (d != NULL)");
   if (t->nq > 1 || (field & 4)) {
@@ -1818,18 +1893,19 @@ wbfmm_target_list_t *wbfmm_target_list_new(wbfmm_tree_t *t, guint npts)
 static void register_targets(tree_dev *td, const uint64_t *dcodes, unsigned n)
 {
   unsigned l;
-  for (l = 0; l <= td->t.depth; l++) {
-    size_t nb = (size_t)1 << (3 * l);
+  build_levels(td);
+  for (l = 0; l <= td->t.depth; l++)
     if (!td->d_flag[l]) {
-      HIPOK(wbfmm_hip_malloc((void **)&td->d_flag[l], sizeof(uint32_t) * nb));
-      HIPOK(wbfmm_hip_malloc((void **)&td->d_act[l], sizeof(uint32_t) * nb));
+      /* flags, list and class list in one block */
+      const size_t nb = (size_t)1 << (3 * l);
+      HIPOK(wbfmm_hip_malloc((void **)&td->d_flag[l], sizeof(uint32_t) * 3 * nb));
+      td->d_act[l] = td->d_flag[l] + nb;
+      td->d_cls[l] = td->d_act[l] + nb;
     }
-    HIPOK(wbfmm_hip_memset(td->d_flag[l], 0, sizeof(uint32_t) * nb));
-    HIPOK(wbfmm_hip_mark_boxes(td->d_codes, td->t.npoints, l, td->d_flag[l]));
-    HIPOK(wbfmm_hip_mark_boxes(dcodes, n, l, td->d_flag[l]));
-    HIPOK(wbfmm_hip_compact_boxes(td->d_start[l], td->d_end[l], td->d_flag[l],
-                                  l, td->d_act[l], &td->nact[l]));
-  }
+  HIPOK(wbfmm_hip_tree_targets(dcodes, n, td->t.depth, td->d_start, td->d_end, td->d_flag,
+                               td->d_act, td->d_cls, td->d_tot));
+  td->tgt_levels = td->t.depth + 1;
+  td->counts_due = 1;
   td->have_targets = 1;
 }
 
@@ -1933,10 +2009,7 @@ gint wbfmm_tree_free(wbfmm_tree_t *t)
   wbfmm_hip_sync();
   for (l = 0; l <= WBFMM_TREE_MAX_DEPTH; l++) {
     wbfmm_hip_free(td->d_start[l]);
-    wbfmm_hip_free(td->d_end[l]);
-    wbfmm_hip_free(td->d_occ[l]);
     wbfmm_hip_free(td->d_flag[l]);
-    wbfmm_hip_free(td->d_act[l]);
     wbfmm_hip_free(t->mps[l]);
     wbfmm_hip_free(t->mpr[l]);
     free(t->boxes[l]);
@@ -1945,6 +2018,7 @@ gint wbfmm_tree_free(wbfmm_tree_t *t)
   }
   wbfmm_hip_free(td->d_xyz);
   wbfmm_hip_free(td->d_xyz_raw);
+  wbfmm_hip_free(td->d_tot);
   wbfmm_hip_free(td->d_nrm);
   wbfmm_hip_free(td->d_codes);
   wbfmm_hip_free(td->d_idx);
@@ -2083,6 +2157,7 @@ gint wbfmm_tree_leaf_expansions(wbfmm_tree_t *t, gdouble k, gdouble *src,
     WBFMM_FATAL("tree has invalid number of components in source terms (%d)", t->nq);
   if (t->problem != WBFMM_PROBLEM_HELMHOLTZ) WBFMM_FATAL("tree is not a Helmholtz tree");
   if (!t->mps[d]) WBFMM_FATAL("coefficients not initialised at level %u", d);
+  tree_counts(td);
   hel_prepare(t, k); /* mixed precision: the levels' precision follows k */
   if (zero_expansions) HIPOK(wbfmm_hip_memset(t->mps[d], 0, td->mps_bytes[d]));
   if (src == NULL && dipoles == NULL) return 0;
@@ -2324,6 +2399,7 @@ gint wbfmm_upward_pass(wbfmm_tree_t *t, wbfmm_shift_operators_t *op, guint level
   if (!op->SS[level]) WBFMM_FATAL("S|S operators not initialised at level %u", level);
   if ((Nc > Np ? Nc : Np) > od->ss_L[level] || (Nc > Np ? Nc : Np) > op->Lmax)
     WBFMM_FATAL("operators at level %u built to order %u", level, od->ss_L[level]);
+  tree_counts(td);
   if (td->prec32) {
     hel_upward_mixed(t, od, level);
     return 0;
@@ -2580,30 +2656,26 @@ static void hel_m2l64(wbfmm_tree_t *t, ops_dev *od, guint level, const uint32_t 
     /* matrix-core form: targets grouped by Morton child digit */
     int N = (int)Ns;
     unsigned cstart[8], ccount[8];
-    uint32_t *cls;
+    const uint32_t *cls;
     ensure_plan(od, N);
     ensure_hel_rot_tiles(od, N);
     ensure_hel_coax_tiles(od, level, N);
-    HIPOK(wbfmm_hip_malloc((void **)&cls, sizeof(uint32_t) * (nt ? nt : 1)));
-    HIPOK(wbfmm_hip_split_classes(tl, nt, cls, cstart, ccount));
+    cls = target_classes(td, level, cstart, ccount);
     HIPOK(wbfmm_hip_hel_m2l_mfma(cls, cstart, ccount, td->d_start[level], td->d_end[level],
                                  level, N, (double *)t->mps[level], (double *)t->mpr[level],
                                  od->m2l_plan_dev[N], od->hel_A[N], od->hel_A2[level],
                                  od->m2l_CS[N], od->m2l_plan[N]));
-    wbfmm_hip_free(cls);
   } else if (hel_wide_serves(Ns, Nr) && level <= M2L_MFMA_MAX_LEVEL) {
     int N = (int)(Ns > Nr ? Ns : Nr);
     unsigned cstart[8], ccount[8];
-    uint32_t *cls;
+    const uint32_t *cls;
     ensure_wide_plan(od, N);
     ensure_wide_rot(od, N);
-    HIPOK(wbfmm_hip_malloc((void **)&cls, sizeof(uint32_t) * (nt ? nt : 1)));
-    HIPOK(wbfmm_hip_split_classes(tl, nt, cls, cstart, ccount));
+    cls = target_classes(td, level, cstart, ccount);
     HIPOK(wbfmm_hip_hel_wide_m2l(cls, cstart, ccount, td->d_start[level], td->d_end[level],
                                  level, (int)Ns, (int)Nr, (double *)t->mps[level],
                                  (double *)t->mpr[level], od->wide_plan_dev[N], od->wide_A[N],
                                  wide_coax(od, level, N, 0), od->wide_CS[N], od->wide_plan[N]));
-    wbfmm_hip_free(cls);
   } else {
     ensure_hel_rotations(od); /* the vector kernels' H tables, on first use */
     HIPOK(wbfmm_hip_hel_m2l(tl, nt, td->d_start[level], td->d_end[level], level, (int)Ns,
@@ -2665,6 +2737,7 @@ static gint hel_downward(wbfmm_tree_t *t, wbfmm_shift_operators_t *op, guint lev
   if ((Ns > Nr ? Ns : Nr) > op->L[level])
     WBFMM_FATAL("S|R operators at level %u built to order %u", level, op->L[level]);
   if ((Ns > Nr ? Ns : Nr) > op->Lmax) WBFMM_FATAL("rotations built to order %u", op->Lmax);
+  tree_counts(td);
   if (td->have_targets) {
     tl = td->d_act[level];
     nt = td->nact[level];
@@ -2856,17 +2929,15 @@ static void hel_downward_mixed(wbfmm_tree_t *t, ops_dev *od, guint level, const 
   if (!td->h64[level]) {
     int N = (int)Ns;
     unsigned cstart[8], ccount[8];
-    uint32_t *cls;
+    const uint32_t *cls;
     if (Ns != Nr) WBFMM_FATAL("FP32 level %u with unequal orders", level);
     ensure_hel_f32_order(od, N);
     ensure_hel_f32_m2l_tiles(od, t->D, level, N, td->hk);
-    HIPOK(wbfmm_hip_malloc((void **)&cls, sizeof(uint32_t) * (nt ? nt : 1)));
-    HIPOK(wbfmm_hip_split_classes(tl, nt, cls, cstart, ccount));
+    cls = target_classes(td, level, cstart, ccount);
     HIPOK(wbfmm_hip_hel_m2l_mfma_f32(cls, cstart, ccount, td->d_start[level], td->d_end[level],
                                      level, N, (const float *)t->mps[level],
                                      (float *)t->mpr[level], od->m2l_plan_dev[N], od->f_hA[N],
                                      od->f_hA2[level], od->f_hCS[N], od->m2l_plan[N]));
-    wbfmm_hip_free(cls);
   } else {
     hel_m2l64(t, od, level, tl, nt);
   }
@@ -2956,6 +3027,7 @@ static void hel_field_run(tree_dev *td, double k, const double *dxt,
   int staged, f32;
   size_t nelem;
   if (!t->mpr[lv]) WBFMM_FATAL("coefficients not initialised at level %u", lv);
+  build_levels(td);
   if (t->normals == NULL && d != NULL)
     WBFMM_FATAL("no normals in tree but dipole strengths specified (d != NULL)");
   f32 = level_f32(td, lv);
