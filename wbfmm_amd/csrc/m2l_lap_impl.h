@@ -289,6 +289,17 @@ __global__ __launch_bounds__(64) void k_lap_m2l_mfma(
 // is deterministic: every LDS slot has one writer.
 // ---------------------------------------------------------------------
 
+// the chunked kernel's double buffer: M2LDouble, and with sixteen wavefronts
+// (one block per CU) wherever the two copies and the tables fit 160 KB
+// (orders 16..20)
+template <typename T, int N, int W>
+struct M2LChunkDouble {
+  using SH = M2LShape<N>;
+  static constexpr int bytes = 2 * (SH::S + 1) * 16 * (int)sizeof(T) + 3 * 4 * SH::NB * 16 +
+                               SH::NU * 16 + 2 * (N + 1) * 2 * (int)sizeof(T) + 1024;
+  static constexpr bool value = M2LDouble<T, N>::value || (W == 16 && bytes <= 160 * 1024);
+};
+
 template <typename T, int N, int W, int WI>
 __device__ __forceinline__ void m2l_w2_loop(
     T *R, const int4 *tmap1, const int4 *tmap2, const int4 *tmap3, const int4 *uinf,
@@ -303,7 +314,7 @@ __device__ __forceinline__ void m2l_w2_loop(
   typedef typename MF<T>::v4 V4;
   using SH = M2LShape<N>;
   constexpr int C = SH::C, NU = SH::NU;
-  constexpr bool DB = M2LDouble<T, N>::value;
+  constexpr bool DB = M2LChunkDouble<T, N, W>::value;
   T *R1 = R + (SH::S + 1) * 16;  // the second buffer (DB only)
   constexpr int NAW = (NU + 4 * W - 1) / (4 * W);  // units per lane
   constexpr WaveSeq WS = make_seq(SH::BN, W, WI);
@@ -574,7 +585,8 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(
   typedef typename MF<T>::t2 T2;
   using SH = M2LShape<N>;
   constexpr int NB = SH::NB, NU = SH::NU, S = SH::S;
-  __shared__ T R[(M2LDouble<T, N>::value ? 2 : 1) * (S + 1) * 16];
+  constexpr int NR = (M2LChunkDouble<T, N, W>::value ? 2 : 1) * (S + 1) * 16;
+  __shared__ T R[NR];
   __shared__ int4 tmap1[4 * NB], tmap2[4 * NB], tmap3[4 * NB];
   __shared__ int4 uinf[NU];
   __shared__ T2 cs[2][N + 1];
@@ -606,7 +618,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(
     uinf[u] = make_int4(n * n + (m ? 2 * m - 1 : 0), m, P->s1[u] & 0xffff,
                         (P->s1[u] >> 16) & 0xffff);
   }
-  for (int i = tid; i < (M2LDouble<T, N>::value ? 2 : 1) * (S + 1) * 16; i += 64 * W) R[i] = T(0);
+  for (int i = tid; i < NR; i += 64 * W) R[i] = T(0);
   for (int i = tid; i < 16 * 7; i += 64 * W) vm[i / 7][i % 7] = 0u;
 
   const int split = (int)(blockIdx.x % (unsigned)nsplit);
@@ -648,11 +660,23 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(
       m2l_w2_loop<T, N, 2, 1>(R, tmap1, tmap2, tmap3, uinf, cs, vm, anym, lane, col, grp, tvalid, tb,
                             ti, tj, tk, px, py, pz, c, k16, split, nsplit, ca, P, A1, A3, A2,
                             CS, zero, mps, mpr, part, ntot);
-  } else if constexpr (W == 8) {
+  } else if constexpr (W >= 8) {
 #define CHUNK8(WI)                                                                            \
-  m2l_w2_loop<T, N, 8, WI>(R, tmap1, tmap2, tmap3, uinf, cs, vm, anym, lane, col, grp, tvalid, \
+  m2l_w2_loop<T, N, W, WI>(R, tmap1, tmap2, tmap3, uinf, cs, vm, anym, lane, col, grp, tvalid, \
                            tb, ti, tj, tk, px, py, pz, c, k16, split, nsplit, ca, P, A1, A3,  \
                            A2, CS, zero, mps, mpr, part, ntot)
+    if constexpr (W == 16) {
+      switch (wv) {
+        case 8: CHUNK8(8); return;
+        case 9: CHUNK8(9); return;
+        case 10: CHUNK8(10); return;
+        case 11: CHUNK8(11); return;
+        case 12: CHUNK8(12); return;
+        case 13: CHUNK8(13); return;
+        case 14: CHUNK8(14); return;
+        case 15: CHUNK8(15); return;
+      }
+    }
     switch (wv) {
       case 0: CHUNK8(0); break;
       case 1: CHUNK8(1); break;
@@ -2211,8 +2235,11 @@ static int launch_m2l(const uint32_t *cls, const ClassArgs &ca, unsigned nchunks
   // several wavefronts per chunk: eight for FP64 orders 9..15 (at order 12
   // the 11 bins of a stage take 2 per wavefront instead of 3); four fit
   // three per SIMD without spilling at every order; two fit two per SIMD
-  // for FP32 and for FP64 up to 12; orders above 15 (blocks spanning
-  // several bins) have the four-wavefront kernel only
+  // for FP32 and for FP64 up to 12.  FP64 orders 16..20: sixteen (one block
+  // per CU with the doubled buffer, every operand of a stage held across
+  // the stage before; four wavefronts left one or two per SIMD: order 20 at
+  // 32768 full boxes, M2L 22.0 -> 14.4 ms); 21..24, whose two copies do
+  // not fit, eight (sixteen spill 36 to 290 registers)
   if constexpr (sizeof(T) == 8 && N >= 9 && N <= 15) {
     if (m2l_waves() == 8) {
       WBFMM_LAUNCH("lap_m2l", (k_lap_m2l_mfma2<T, N, 8>), dim3(grid), dim3(512), 0,
@@ -2221,12 +2248,17 @@ static int launch_m2l(const uint32_t *cls, const ClassArgs &ca, unsigned nchunks
       goto reduce;
     }
   }
-  if (N > 15 || m2l_waves() == 4 || m2l_waves() == 8) {
+  if constexpr (sizeof(T) == 8 && N >= 16) {
+    constexpr int WN = N <= 20 ? 16 : 8;
+    WBFMM_LAUNCH("lap_m2l", (k_lap_m2l_mfma2<T, N, WN>), dim3(grid), dim3(64 * WN), 0, cls, cx,
+                 occ, level, mps, mpr, (const wbfmm_m2l_plan_t *)plan, A1, A3, A2, CS, zero,
+                 nsplit, part, ntot);
+  } else if (m2l_waves() == 4 || m2l_waves() == 8) {
     WBFMM_LAUNCH(sizeof(T) == 4 ? "lap_m2l_f32" : "lap_m2l", (k_lap_m2l_mfma2<T, N, 4>),
                  dim3(grid), dim3(256), 0, cls,
                  cx, occ, level, mps, mpr, (const wbfmm_m2l_plan_t *)plan,
                  A1, A3, A2, CS, zero, nsplit, part, ntot);
-  } else if constexpr (N <= 15) {
+  } else {
     if (m2l_waves() >= 2 && (sizeof(T) == 4 || N <= 12))
       WBFMM_LAUNCH(sizeof(T) == 4 ? "lap_m2l_f32" : "lap_m2l", (k_lap_m2l_mfma2<T, N, 2>),
                    dim3(grid), dim3(128), 0, cls,
