@@ -104,6 +104,148 @@ __device__ __forceinline__ void stage_cx_wo(const T *__restrict__ ar,
   }
 }
 
+// The stages of the single-buffered form with the first operands of a
+// stage's tables requested before the barriers that precede it, so that the
+// loads run while the stage before is exchanged: op holds the first 16
+// k-steps of a rotation, or the first 8 of a complex coaxial stage (real
+// parts, then imaginary parts); the later ones follow through the same ring
+// as in stage_w and stage_cx.  1e5-point sphere, FP64, orders 25/23: M2L 7.7
+// -> 7.1 ms (sixteen wavefronts instead of eight: 596 to 1624 registers
+// spilled); 1e6-point sphere, FP32, order 23: 30.6 -> 29.5 ms.
+template <int N, int W, int WI>
+struct HelOps {
+  static constexpr WaveSeq WS = make_seq(M2LShape<N>::BN, W, WI);
+  static constexpr int n = WS.n < 16 ? (WS.n > 0 ? WS.n : 1) : 16;
+  static constexpr int nc = WS.n < 8 ? (WS.n > 0 ? WS.n : 1) : 8;
+};
+
+template <typename T, int N, int W, int WI>
+__device__ __forceinline__ void hel_ops(T *op, const T *__restrict__ a, int lane) {
+  constexpr WaveSeq WS = make_seq(M2LShape<N>::BN, W, WI);
+  constexpr int AD = HelOps<N, W, WI>::n;
+#pragma unroll
+  for (int s = 0; s < AD && s < WS.n; s++) op[s] = a[WS.t[s] * 64 + lane];
+}
+
+template <typename T, int N, int W, int WI>
+__device__ __forceinline__ void hel_ops_cx(T *op, const T *__restrict__ ar,
+                                           const T *__restrict__ ai, int lane) {
+  constexpr WaveSeq WS = make_seq(M2LShape<N>::BN, W, WI);
+  constexpr int AD = HelOps<N, W, WI>::nc;
+#pragma unroll
+  for (int s = 0; s < AD && s < WS.n; s++) {
+    op[s] = ar[WS.t[s] * 64 + lane];
+    op[8 + s] = ai[WS.t[s] * 64 + lane];
+  }
+}
+
+template <typename T, int N, int W, int WI>
+__device__ __forceinline__ void hel_stage_w(T *op, const T *__restrict__ a, const T *R, int lane,
+                                            int grp, int col, V4t<T> *y) {
+  constexpr Bins BN = M2LShape<N>::BN;
+  constexpr WaveSeq WS = make_seq(BN, W, WI);
+  constexpr int AD = HelOps<N, W, WI>::n;
+#pragma unroll
+  for (int lb = 0; lb < WS.nb; lb++) {
+    const int b = WI + W * lb;
+    V4t<T> r4 = {T(0), T(0), T(0), T(0)};
+#pragma unroll
+    for (int j = 0; j < BN.nk[b]; j++) {
+      const int s = WS.start[lb] + j;
+      r4 = MF<T>::mma(op[s % AD], R[(BN.kbase[b] + 4 * j + grp) * 16 + col], r4);
+      if (s + AD < WS.n) op[s % AD] = a[WS.t[s + AD] * 64 + lane];
+    }
+    y[lb] = r4;
+  }
+}
+
+template <typename T, int N, int W, int WI>
+__device__ __forceinline__ void hel_stage_cx(T *op, const T *__restrict__ ar,
+                                             const T *__restrict__ ai, const T *R, int lane,
+                                             int grp, int col, V4t<T> *y) {
+  constexpr Bins BN = M2LShape<N>::BN;
+  constexpr WaveSeq WS = make_seq(BN, W, WI);
+  constexpr int AD = HelOps<N, W, WI>::nc;
+  const T sg = (col & 1) ? T(1) : T(-1);
+  const int pc = col ^ 1;
+#pragma unroll
+  for (int lb = 0; lb < WS.nb; lb++) {
+    const int b = WI + W * lb;
+    V4t<T> r4 = {T(0), T(0), T(0), T(0)}, i4 = {T(0), T(0), T(0), T(0)};
+#pragma unroll
+    for (int j = 0; j < BN.nk[b]; j++) {
+      const int s = WS.start[lb] + j;
+      const int row = (BN.kbase[b] + 4 * j + grp) * 16;
+      r4 = MF<T>::mma(op[s % AD], R[row + col], r4);
+      i4 = MF<T>::mma(op[8 + s % AD], R[row + pc], i4);
+      if (s + AD < WS.n) {
+        op[s % AD] = ar[WS.t[s + AD] * 64 + lane];
+        op[8 + s % AD] = ai[WS.t[s + AD] * 64 + lane];
+      }
+    }
+    y[lb] = r4 + sg * i4;
+  }
+}
+
+// the same stages with the results of a bin stored at once into the other
+// copy of a doubled buffer
+template <typename T, int N, int W, int WI>
+__device__ __forceinline__ void hel_stage_wo(T *op, const T *__restrict__ a, const T *Rin, T *Rout,
+                                             const int4 *tm, int lane, int grp, int col) {
+  constexpr Bins BN = M2LShape<N>::BN;
+  constexpr WaveSeq WS = make_seq(BN, W, WI);
+  constexpr int AD = HelOps<N, W, WI>::n;
+#pragma unroll
+  for (int lb = 0; lb < WS.nb; lb++) {
+    const int b = WI + W * lb;
+    V4t<T> r4 = {T(0), T(0), T(0), T(0)};
+#pragma unroll
+    for (int j = 0; j < BN.nk[b]; j++) {
+      const int s = WS.start[lb] + j;
+      r4 = MF<T>::mma(op[s % AD], Rin[(BN.kbase[b] + 4 * j + grp) * 16 + col], r4);
+      if (s + AD < WS.n) op[s % AD] = a[WS.t[s + AD] * 64 + lane];
+    }
+    const int4 d = tm[4 * b + grp];
+    Rout[d.x * 16 + col] = r4[0];
+    Rout[d.y * 16 + col] = r4[1];
+    Rout[d.z * 16 + col] = r4[2];
+    Rout[d.w * 16 + col] = r4[3];
+  }
+}
+
+template <typename T, int N, int W, int WI>
+__device__ __forceinline__ void hel_stage_cx_wo(T *op, const T *__restrict__ ar,
+                                                const T *__restrict__ ai, const T *Rin, T *Rout,
+                                                const int4 *tm, int lane, int grp, int col) {
+  constexpr Bins BN = M2LShape<N>::BN;
+  constexpr WaveSeq WS = make_seq(BN, W, WI);
+  constexpr int AD = HelOps<N, W, WI>::nc;
+  const T sg = (col & 1) ? T(1) : T(-1);
+  const int pc = col ^ 1;
+#pragma unroll
+  for (int lb = 0; lb < WS.nb; lb++) {
+    const int b = WI + W * lb;
+    V4t<T> r4 = {T(0), T(0), T(0), T(0)}, i4 = {T(0), T(0), T(0), T(0)};
+#pragma unroll
+    for (int j = 0; j < BN.nk[b]; j++) {
+      const int s = WS.start[lb] + j;
+      const int row = (BN.kbase[b] + 4 * j + grp) * 16;
+      r4 = MF<T>::mma(op[s % AD], Rin[row + col], r4);
+      i4 = MF<T>::mma(op[8 + s % AD], Rin[row + pc], i4);
+      if (s + AD < WS.n) {
+        op[s % AD] = ar[WS.t[s + AD] * 64 + lane];
+        op[8 + s % AD] = ai[WS.t[s + AD] * 64 + lane];
+      }
+    }
+    const V4t<T> y = r4 + sg * i4;
+    const int4 d = tm[4 * b + grp];
+    Rout[d.x * 16 + col] = y[0];
+    Rout[d.y * 16 + col] = y[1];
+    Rout[d.z * 16 + col] = y[2];
+    Rout[d.w * 16 + col] = y[3];
+  }
+}
+
 template <typename T, int N, int W, int WI>
 __device__ __forceinline__ void hel_m2l_loop(
     T *R, const int4 *tmap1, const int4 *tmap2, const int4 *tmap3, const int4 *uinf,
@@ -219,6 +361,8 @@ __device__ __forceinline__ void hel_m2l_loop(
     load_sources(source_of(k, 0), uinf, ubase, col & 1);
     deposit(uinf, ubase, col, 0);
   }
+  T op[16];
+  if constexpr (!DB) hel_ops<T, N, W, WI>(op, A + (size_t)th * KT * 64, lane);
   __syncthreads();
   while (k < 216) {
     int z0;
@@ -247,19 +391,20 @@ __device__ __forceinline__ void hel_m2l_loop(
       RZ = R1;
     } else {
       V4t<T> y[NBW > 0 ? NBW : 1];
-      stage_w<T, N, W, WI>(A + (size_t)th * KT * 64, R, ln, gp, cl, y);
+      const T *ar = A2 + (size_t)(2 * ri) * KT * 64, *ai = ar + (size_t)KT * 64;
+      hel_stage_w<T, N, W, WI>(op, A + (size_t)th * KT * 64, R, ln, gp, cl, y);
+      hel_ops_cx<T, N, W, WI>(op, ar, ai, ln);
       __syncthreads();
       write_out(t1, y, gp, cl);
       __syncthreads();
       if (kn < 216) load_sources(source_of(kn, p ^ 1), tu, ub, sp);
-
-      stage_cx<T, N, W, WI>(A2 + (size_t)(2 * ri) * KT * 64, A2 + (size_t)(2 * ri + 1) * KT * 64,
-                         R, ln, gp, cl, y);
+      hel_stage_cx<T, N, W, WI>(op, ar, ai, R, ln, gp, cl, y);
+      hel_ops<T, N, W, WI>(op, A + (size_t)th * KT * 64, ln);
       __syncthreads();
       write_out(t2, y, gp, cl);
       __syncthreads();
-
-      stage_w<T, N, W, WI>(A + (size_t)th * KT * 64, R, ln, gp, cl, y);
+      hel_stage_w<T, N, W, WI>(op, A + (size_t)th * KT * 64, R, ln, gp, cl, y);
+      hel_ops<T, N, W, WI>(op, A + (size_t)th_n * KT * 64, ln);
       __syncthreads();
       write_out(t3, y, gp, cl);
       __syncthreads();
@@ -404,7 +549,19 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(
   hel_m2l_loop<T, N, W, WI>(R, tmap1, tmap2, tmap3, uinf, cs, vm, anym, lane, col, grp, tvalid,  \
                          tb, ti, tj, tk, px, py, pz, c, k8, split, nsplit, ca, P, A, A2, CS, \
                          zero, mps, mpr, part, ntot)
-  static_assert(W == 4 || W == 8, "four or eight wavefronts per block");
+  static_assert(W == 4 || W == 8 || W == 16, "four, eight or sixteen wavefronts per block");
+  if constexpr (W == 16) {
+    switch (wv) {
+      case 8: HEL_LOOP(8); return;
+      case 9: HEL_LOOP(9); return;
+      case 10: HEL_LOOP(10); return;
+      case 11: HEL_LOOP(11); return;
+      case 12: HEL_LOOP(12); return;
+      case 13: HEL_LOOP(13); return;
+      case 14: HEL_LOOP(14); return;
+      case 15: HEL_LOOP(15); return;
+    }
+  }
   if constexpr (W == 4) {
     switch (wv) {
       case 0: HEL_LOOP(0); break;
@@ -453,6 +610,19 @@ struct HelPackedFits {
   static constexpr bool value = sizeof(T) == 4 && N >= 8 && N <= 27;
 };
 
+// the packed kernel's double buffer: M2LDouble, and with sixteen wavefronts
+// (one block per CU) wherever the two copies and the lists fit 160 KB
+// (orders 16..26): five barriers per tile instead of eight, 29.5 -> 28.1 ms
+// on the 1e6-point sphere (with the owners' sums read as pairs and halved
+// once at the end)
+template <typename T, int N, int W>
+struct HelPackedDouble {
+  using SH = M2LShape<N>;
+  static constexpr int bytes = 2 * (SH::S + 1) * 16 * (int)sizeof(T) + 3 * 4 * SH::NB * 16 +
+                               SH::NU * 16 + 16 * (N + 1) * 2 * (int)sizeof(T) + 14 * 1024;
+  static constexpr bool value = M2LDouble<T, N>::value || (W == 16 && bytes <= 160 * 1024);
+};
+
 template <typename T, int N, int W, int WI>
 __device__ __forceinline__ void hel_packed_loop(
     T *R, const int4 *tmap1, const int4 *tmap2, const int4 *tmap3, const int4 *uinf,
@@ -468,7 +638,7 @@ __device__ __forceinline__ void hel_packed_loop(
   constexpr int NAW = (NU + 4 * W - 1) / (4 * W);  // units per lane (deposit)
   constexpr WaveSeq WS = make_seq(SH::BN, W, WI);
   constexpr int NBW = WS.nb;
-  constexpr bool DB = M2LDouble<T, N>::value;
+  constexpr bool DB = HelPackedDouble<T, N, W>::value;
   constexpr int G = 2 * W;                       // unit groups of the owners
   constexpr int NAQ = (NU + G - 1) / G;          // owner units per lane
   T *R1 = R + (SH::S + 1) * 16;  // the second buffer (DB only)
@@ -546,6 +716,7 @@ __device__ __forceinline__ void hel_packed_loop(
     }
   };
 
+  const T sgn = osg ? T(-1) : T(1);
   T acc_re[NAQ], acc_im[NAQ];
 #pragma unroll
   for (int i = 0; i < NAQ; i++) acc_re[i] = acc_im[i] = T(0);
@@ -561,6 +732,8 @@ __device__ __forceinline__ void hel_packed_loop(
     load_sources(source_of(g, t, 0, true, icol), uinf, ubase, col & 1);
     deposit(uinf, ubase, col, 0, icol);
   }
+  T op[16];
+  hel_ops<T, N, W, WI>(op, A + (size_t)th * KT * 64, lane);
   __syncthreads();
   while (g < ncls) {
     int z0;
@@ -586,34 +759,40 @@ __device__ __forceinline__ void hel_packed_loop(
     // the chunked kernel (their registers are not held across all three)
     T *RZ = R;
     if constexpr (DB) {
-      stage_wo<T, N, W, WI>(A + (size_t)th * KT * 64, R, R1, t1, ln, gp, cl);
+      const T *ar = A2 + (size_t)(2 * ri) * KT * 64, *ai = ar + (size_t)KT * 64;
+      hel_stage_wo<T, N, W, WI>(op, A + (size_t)th * KT * 64, R, R1, t1, ln, gp, cl);
+      hel_ops_cx<T, N, W, WI>(op, ar, ai, ln);
       __syncthreads();
       if (gn < ncls) load_sources(source_of(gn, tn, pn, newc, icol_n), tu, ub, sp);
-      stage_cx_wo<T, N, W, WI>(A2 + (size_t)(2 * ri) * KT * 64, A2 + (size_t)(2 * ri + 1) * KT * 64,
-                               R1, R, t2, ln, gp, cl);
+      hel_stage_cx_wo<T, N, W, WI>(op, ar, ai, R1, R, t2, ln, gp, cl);
+      hel_ops<T, N, W, WI>(op, A + (size_t)th * KT * 64, ln);
       __syncthreads();
-      stage_wo<T, N, W, WI>(A + (size_t)th * KT * 64, R, R1, t3, ln, gp, cl);
+      hel_stage_wo<T, N, W, WI>(op, A + (size_t)th * KT * 64, R, R1, t3, ln, gp, cl);
+      hel_ops<T, N, W, WI>(op, A + (size_t)th_n * KT * 64, ln);
       __syncthreads();
       RZ = R1;
     } else {
       V4t<T> y[NBW > 0 ? NBW : 1];
-      stage_w<T, N, W, WI>(A + (size_t)th * KT * 64, R, ln, gp, cl, y);
+      const T *ar = A2 + (size_t)(2 * ri) * KT * 64, *ai = ar + (size_t)KT * 64;
+      hel_stage_w<T, N, W, WI>(op, A + (size_t)th * KT * 64, R, ln, gp, cl, y);
+      hel_ops_cx<T, N, W, WI>(op, ar, ai, ln);
       __syncthreads();
       write_out(t1, y, gp, cl);
       __syncthreads();
       if (gn < ncls) load_sources(source_of(gn, tn, pn, newc, icol_n), tu, ub, sp);
-      stage_cx<T, N, W, WI>(A2 + (size_t)(2 * ri) * KT * 64, A2 + (size_t)(2 * ri + 1) * KT * 64,
-                            R, ln, gp, cl, y);
+      hel_stage_cx<T, N, W, WI>(op, ar, ai, R, ln, gp, cl, y);
+      hel_ops<T, N, W, WI>(op, A + (size_t)th * KT * 64, ln);
       __syncthreads();
       write_out(t2, y, gp, cl);
       __syncthreads();
-      stage_w<T, N, W, WI>(A + (size_t)th * KT * 64, R, ln, gp, cl, y);
+      hel_stage_w<T, N, W, WI>(op, A + (size_t)th * KT * 64, R, ln, gp, cl, y);
+      hel_ops<T, N, W, WI>(op, A + (size_t)th_n * KT * 64, ln);
       __syncthreads();
       write_out(t3, y, gp, cl);
       __syncthreads();
     }
-    // owners: y_{+-nu} = (P +- Q)/2 of the target's column pair, then
-    // L^{+-nu} += e^{-+i nu chi} y
+    // owners: y_{+-nu} = P +- Q of the target's column pair, then
+    // L^{+-nu} += e^{-+i nu chi} y (halved when the sums are stored)
     {
       const int Tt = gT[g], z = zinfo[g][ot];
       const int r = z & 15, q = (z >> 4) & 15, cnt = z >> 8;
@@ -629,12 +808,11 @@ __device__ __forceinline__ void hel_packed_loop(
           if (u >= NU) continue;
           const int nu = tu[u].y;
           const T2t<T> e = cs[p][ic][nu];
-          const T es = osg ? -e.y : e.y;
-          const T pr = RZ[u * 16 + c0], pi = RZ[u * 16 + c0 + 1];
-          const T qr = nu ? RZ[(NU + u) * 16 + c0] : T(0);
-          const T qi = nu ? RZ[(NU + u) * 16 + c0 + 1] : T(0);
-          const T yr = T(0.5) * (osg ? pr - qr : pr + qr);
-          const T yi = T(0.5) * (osg ? pi - qi : pi + qi);
+          const T es = sgn * e.y;
+          const T2t<T> P = *(const T2t<T> *)&RZ[u * 16 + c0];
+          const T2t<T> Q = *(const T2t<T> *)&RZ[(NU + u) * 16 + c0];
+          // (the row of Q at order 0 holds another stage's values)
+          const T yr = nu ? P.x + sgn * Q.x : P.x, yi = nu ? P.y + sgn * Q.y : P.y;
           acc_re[i] += e.x * yr + es * yi;
           acc_im[i] += e.x * yi - es * yr;
         }
@@ -661,7 +839,7 @@ __device__ __forceinline__ void hel_packed_loop(
     if (osg && inf.y == 0) continue;  // L^0 is the sign-0 owner's
     const int r = inf.x + (osg ? -inf.y : inf.y);
     const T2t<T> o = dst[r];
-    dst[r] = mk2<T>(o.x + acc_re[i], o.y + acc_im[i]);
+    dst[r] = mk2<T>(o.x + T(0.5) * acc_re[i], o.y + T(0.5) * acc_im[i]);
   }
 }
 
@@ -677,7 +855,8 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(
   using SH = M2LShape<N>;
   constexpr int NB = SH::NB, NU = SH::NU, S = SH::S;
   static_assert(W == 4 || W == 8 || W == 16, "four, eight or sixteen wavefronts per block");
-  __shared__ T R[(M2LDouble<T, N>::value ? 2 : 1) * (S + 1) * 16];
+  constexpr int NR = (HelPackedDouble<T, N, W>::value ? 2 : 1) * (S + 1) * 16;
+  __shared__ T R[NR];
   __shared__ int4 tmap1[4 * NB], tmap2[4 * NB], tmap3[4 * NB];
   __shared__ int4 uinf[NU];
   __shared__ T2t<T> cs[2][8][N + 1];
@@ -714,8 +893,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(
     const int m = u - n * (n + 1) / 2;
     uinf[u] = make_int4(n * (n + 1), m, P->s1[u] & 0xffff, (P->s1[u] >> 16) & 0xffff);
   }
-  for (int i = tid; i < (M2LDouble<T, N>::value ? 2 : 1) * (S + 1) * 16; i += 64 * W)
-    R[i] = T(0);
+  for (int i = tid; i < NR; i += 64 * W) R[i] = T(0);
   for (int i = tid; i < kHelPackT * 7; i += 64 * W) vm[i / 7][i % 7] = 0u;
 
   int c;
