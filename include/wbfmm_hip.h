@@ -111,10 +111,11 @@ int wbfmm_hip_box_ranges(const uint64_t *codes, unsigned n, unsigned level,
                          uint32_t *start, uint32_t *end);
 /* points (host or device, byte stride) in Morton order: positions (4
    doubles each), codes and caller indices; raw: scratch of 4 n doubles;
-   *nbad: points outside the domain.  Returns when the points are read and
-   *nbad is known. */
+   *nbad: points outside the domain; low (0..57): the lowest bits of the
+   codes left out of the order.  Returns when the points are read and *nbad
+   is known. */
 int wbfmm_hip_points_sorted(const void *pts, size_t pstr, unsigned n, const double *x0, double D,
-                            double *raw, double *xyz, uint64_t *codes, uint32_t *idx,
+                            int low, double *raw, double *xyz, uint64_t *codes, uint32_t *idx,
                             unsigned *nbad);
 /* dense [start, end) ranges (0, 0 where empty) and ascending lists of the
    occupied boxes of the levels lo..hi (at most 10) over the sorted codes,

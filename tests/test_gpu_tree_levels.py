@@ -76,11 +76,11 @@ def test_all_classes(wb):
 
 
 def test_points_sorted(wb):
-    # device and strided host points, ties kept in the caller's order, the
-    # count of points outside
+    # device and strided host points, ties (of the codes without their low
+    # bits) kept in the caller's order, the count of points outside
     lib = wb.lib()
     rng = np.random.default_rng(3)
-    for n, stride in ((1, 24), (1000, 40), (5000, 24)):
+    for n, stride, low in ((1, 24, 0), (1000, 40, 0), (5000, 24, 0), (5000, 24, 45), (9, 24, 57)):
         x = rng.uniform(0.01, 0.99, (n, stride // 8))
         x[n // 2:, :3] = x[:n - n // 2, :3]
         if n == 1000:
@@ -93,7 +93,7 @@ def test_points_sorted(wb):
             nbad = ctypes.c_uint(99)
             assert lib.wbfmm_hip_points_sorted(
                 _vp(src.ptr if dev else x.ctypes.data), ctypes.c_size_t(stride), n,
-                _vp(x0.ctypes.data), ctypes.c_double(1.0), _vp(raw.ptr), _vp(xyz.ptr),
+                _vp(x0.ctypes.data), ctypes.c_double(1.0), low, _vp(raw.ptr), _vp(xyz.ptr),
                 _vp(codes.ptr), _vp(idx.ptr), ctypes.byref(nbad)) == 0
             assert nbad.value == (1 if n == 1000 else 0)
             i = idx.download(np.zeros(n, np.uint32))
@@ -104,7 +104,7 @@ def test_points_sorted(wb):
                 for a in range(3):
                     want |= ((g[:, a] >> np.uint64(b)) & np.uint64(1)) << np.uint64(3 * b + a)
             if n != 1000:
-                order = np.argsort(want, kind="stable")
+                order = np.argsort(want >> np.uint64(low), kind="stable")
                 assert np.array_equal(i, order) and np.array_equal(c, want[order])
                 assert np.array_equal(xyz.download(np.zeros((n, 4)))[:, :3], x[order, :3])
             if src:

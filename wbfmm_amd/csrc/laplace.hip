@@ -45,6 +45,61 @@ __device__ __forceinline__ const double *coax_row(const double *cf, int L,
   return cf + ((size_t)m * (L + 1) + n) * (L + 1);
 }
 
+// The factors of the regular functions' recurrences and of the gradient per
+// (j, k), 0 <= k <= j, and the ladder factors of the second derivatives:
+// one table per process, built once on the device, read instead of several
+// square roots and divisions per step.
+struct LapCol {
+  double al, be;      // P_j^k = Cth al P_{j-1}^k - be P_{j-2}^k (j > k)
+  double f0, f1, f2;  // d/dz, and D+ from L_{j+1}^{k-1} and L_{j+1}^{k+1}
+  double dg;          // P_k^k = dg Sth P_{k-1}^{k-1} (at j = k > 0)
+  double rj;          // 1 / (2 j + 1)
+  double pad;
+};
+constexpr int kLapTabN = WBFMM_HIP_MAX_ORDER + 3;
+struct LapTab {
+  LapCol c[(WBFMM_HIP_MAX_ORDER + 1) * (WBFMM_HIP_MAX_ORDER + 2) / 2];
+  double la[kLapTabN][kLapTabN];          // lad_a(n, m)
+  double lb[kLapTabN][2 * kLapTabN + 1];  // lad_s(mu) lad_b(n, mu), mu - kLapTabN
+};
+
+__device__ __forceinline__ double lad_kn(int n) { return (2.0 * n + 1) / (2.0 * n - 1); }
+__device__ __forceinline__ double lad_a(int n, int m) {
+  return n >= 1 && m <= n ? sqrt(lad_kn(n) * (double)(n - m) * (double)(n + m)) : 0.0;
+}
+__device__ __forceinline__ double lad_b(int n, int mu) {
+  const double v = (double)(n - mu) * (double)(n - mu - 1);
+  return (n >= 1 && v > 0.0) ? sqrt(lad_kn(n) * v) : 0.0;
+}
+__device__ __forceinline__ double lad_s(int mu) { return mu >= 0 ? -1.0 : 1.0; }
+
+__global__ void k_lap_tab(LapTab *T) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < (WBFMM_HIP_MAX_ORDER + 1) * (WBFMM_HIP_MAX_ORDER + 2) / 2) {
+    int j = 0;
+    while ((j + 1) * (j + 2) / 2 <= t) j++;
+    const int k = t - j * (j + 1) / 2, n1 = j + 1;
+    LapCol c = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 1.0 / (2 * j + 1), 0.0};
+    if (j > k) {
+      const double h = sqrt((2.0 * j + 1) / (double)(j * j - k * k));
+      c.al = sqrt(2.0 * j - 1) * h;
+      c.be = j - 1 > k ? sqrt((double)((j - 1) * (j - 1) - k * k) / (2 * j - 3)) * h : 0.0;
+    } else if (k > 0) {
+      c.dg = sqrt((2.0 * k + 1) / (2.0 * k));
+    }
+    const double fc = sqrt((2.0 * n1 + 1) / (2.0 * n1 - 1));
+    c.f0 = fc * sqrt((double)(n1 - k) * (n1 + k));
+    c.f1 = k >= 1 ? fc * sqrt((double)(n1 - k + 1) * (n1 - k)) : 0.0;
+    c.f2 = fc * sqrt((double)(n1 + k + 1) * (n1 + k));
+    T->c[t] = c;
+  }
+  if (t < kLapTabN * kLapTabN) T->la[t / kLapTabN][t % kLapTabN] = lad_a(t / kLapTabN, t % kLapTabN);
+  if (t < kLapTabN * (2 * kLapTabN + 1)) {
+    const int n = t / (2 * kLapTabN + 1), mu = t % (2 * kLapTabN + 1) - kLapTabN;
+    T->lb[n][mu + kLapTabN] = (mu < 0 ? -mu : mu) <= n ? lad_s(mu) * lad_b(n, mu) : 0.0;
+  }
+}
+
 // ---------------------------------------------------------------------
 // P2M (src/laplace.c:35-129, :315-423, :854-989)
 // ---------------------------------------------------------------------
@@ -294,12 +349,18 @@ __global__ __launch_bounds__(256) void k_lap_p2m_cols(
 // complete in program order.  The groups' copies are added in group order
 // and the sum added to the box's expansion: no atomics, the same bits on
 // every run.
+//
+// The factors of the recurrences and of the dipole terms come from the table
+// (with square roots and divisions per step: 200003 points at order 20 0.82
+// -> 0.41 ms, 3e5 at order 9, FP32, 0.32 -> 0.17, 6e4 with dipoles at order
+// 10 0.21 -> 0.10).
 // ---------------------------------------------------------------------
 template <typename T, int GS>
 __global__ __launch_bounds__(64) void k_lap_p2m_wave(
     const uint32_t *boxes, unsigned nbox, const uint32_t *start, const uint32_t *end,
     const double *xyz, const double *q, const double *nrm, const double *dip, int level,
-    double x0, double y0, double z0, double D, int N, double rs, T *mps) {
+    double x0, double y0, double z0, double D, int N, double rs, T *mps,
+    const LapTab *__restrict__ tab) {
   extern __shared__ double pacc[];  // (64 / GS) copies of C coefficients
   constexpr int G = 64 / GS;
   const int lane = threadIdx.x, g = lane / GS, m = lane % GS;
@@ -340,7 +401,7 @@ __global__ __launch_bounds__(64) void k_lap_p2m_wave(
     // P_m^m, r^m and e^{i m phi} of this lane's column
     double pmm = s4pi, rm = 1.0, cm = 1.0, sm = 0.0;
     for (int i = 1; i <= m; i++) {
-      pmm *= sqrt((2.0 * i + 1) / (2.0 * i)) * Sth;
+      pmm *= tab->c[i * (i + 1) / 2 + i].dg * Sth;
       rm *= rr;
       const double tcm = cm * cp - sm * sp;
       sm = sm * cp + cm * sp;
@@ -348,29 +409,28 @@ __global__ __launch_bounds__(64) void k_lap_p2m_wave(
     }
     double p1 = 0.0, p0 = pmm, rn = rm;
     for (int n = m; n <= N; n++) {
+      const LapCol tc = tab->c[n * (n + 1) / 2 + m];
       if (n > m) {
-        const double pn = (Cth * sqrt(2.0 * (n - 1) + 1) * p0 -
-                           sqrt((double)((n - 1) * (n - 1) - m * m) / (2 * (n - 1) - 1)) * p1) *
-                          sqrt((2.0 * (n - 1) + 3) / (double)(n * n - m * m));
+        const double pn = Cth * tc.al * p0 - tc.be * p1;
         p1 = p0;
         p0 = pn;
         rn *= rr;
       }
       const double Rr = rn * p0 * cm, Ri = rn * p0 * sm;
       if (qs != 0.0) {
-        const double f = qs / (2 * n + 1);
+        const double f = qs * tc.rj;
         put(n, m, f * Rr, f * Ri);
       }
       if (ds != 0.0 && n < N) {
         // streaming form of M_{n+1} += d conj(nrm . grad R_{n+1})/(2n+3),
         // as in k_lap_p2m: (a) column m, (b) column m - 1, (c) column m + 1
         const int np = n + 1;
-        const double fc = sqrt((2.0 * np + 1) / (2.0 * np - 1)) * ds / (2 * np + 1);
-        const double a = fc * sqrt((double)(np - m) * (np + m));
+        const double fc = ds / (2 * np + 1);
+        const double a = fc * tc.f0;
         put(np, m, nz * a * Rr, nz * a * Ri);
         if (m >= 1) {
           const int mm = m - 1;
-          const double b1 = fc * sqrt((double)(np - mm) * (np - mm - 1));
+          const double b1 = fc * tc.f1;
           const double ur = 0.5 * nx, ui = -0.5 * ny;  // nu+
           const double vr = ur * Rr - ui * Ri, vi = ur * Ri + ui * Rr;
           if (mm == 0)
@@ -380,7 +440,7 @@ __global__ __launch_bounds__(64) void k_lap_p2m_wave(
         }
         {
           const int mp = m + 1;
-          const double b2 = fc * sqrt((double)(np + mp) * (np + mp - 1));
+          const double b2 = fc * tc.f2;
           const double ur = 0.5 * nx, ui = 0.5 * ny;  // nu-
           const double vr = ur * Rr - ui * Ri, vi = ur * Ri + ui * Rr;
           put(np, mp, b2 * vr, b2 * vi);
@@ -570,59 +630,6 @@ __device__ __forceinline__ void lcoef_nb(const T *mpr, uint64_t b, int C, int n,
   re = mpr[coef_at(b, ir, C)];
   const double v = mpr[coef_at(b, ii, C)];
   im = m ? v : 0.0;
-}
-
-// The factors of the regular functions' recurrences and of the gradient per
-// (j, k), 0 <= k <= j, and the ladder factors of the second derivatives:
-// one table per process, built once on the device, read instead of several
-// square roots and divisions per step.
-struct LapCol {
-  double al, be;      // P_j^k = Cth al P_{j-1}^k - be P_{j-2}^k (j > k)
-  double f0, f1, f2;  // d/dz, and D+ from L_{j+1}^{k-1} and L_{j+1}^{k+1}
-  double dg;          // P_k^k = dg Sth P_{k-1}^{k-1} (at j = k > 0)
-};
-constexpr int kLapTabN = WBFMM_HIP_MAX_ORDER + 3;
-struct LapTab {
-  LapCol c[(WBFMM_HIP_MAX_ORDER + 1) * (WBFMM_HIP_MAX_ORDER + 2) / 2];
-  double la[kLapTabN][kLapTabN];          // lad_a(n, m)
-  double lb[kLapTabN][2 * kLapTabN + 1];  // lad_s(mu) lad_b(n, mu), mu - kLapTabN
-};
-
-__device__ __forceinline__ double lad_kn(int n) { return (2.0 * n + 1) / (2.0 * n - 1); }
-__device__ __forceinline__ double lad_a(int n, int m) {
-  return n >= 1 && m <= n ? sqrt(lad_kn(n) * (double)(n - m) * (double)(n + m)) : 0.0;
-}
-__device__ __forceinline__ double lad_b(int n, int mu) {
-  const double v = (double)(n - mu) * (double)(n - mu - 1);
-  return (n >= 1 && v > 0.0) ? sqrt(lad_kn(n) * v) : 0.0;
-}
-__device__ __forceinline__ double lad_s(int mu) { return mu >= 0 ? -1.0 : 1.0; }
-
-__global__ void k_lap_tab(LapTab *T) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < (WBFMM_HIP_MAX_ORDER + 1) * (WBFMM_HIP_MAX_ORDER + 2) / 2) {
-    int j = 0;
-    while ((j + 1) * (j + 2) / 2 <= t) j++;
-    const int k = t - j * (j + 1) / 2, n1 = j + 1;
-    LapCol c = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    if (j > k) {
-      const double h = sqrt((2.0 * j + 1) / (double)(j * j - k * k));
-      c.al = sqrt(2.0 * j - 1) * h;
-      c.be = j - 1 > k ? sqrt((double)((j - 1) * (j - 1) - k * k) / (2 * j - 3)) * h : 0.0;
-    } else if (k > 0) {
-      c.dg = sqrt((2.0 * k + 1) / (2.0 * k));
-    }
-    const double fc = sqrt((2.0 * n1 + 1) / (2.0 * n1 - 1));
-    c.f0 = fc * sqrt((double)(n1 - k) * (n1 + k));
-    c.f1 = k >= 1 ? fc * sqrt((double)(n1 - k + 1) * (n1 - k)) : 0.0;
-    c.f2 = fc * sqrt((double)(n1 + k + 1) * (n1 + k));
-    T->c[t] = c;
-  }
-  if (t < kLapTabN * kLapTabN) T->la[t / kLapTabN][t % kLapTabN] = lad_a(t / kLapTabN, t % kLapTabN);
-  if (t < kLapTabN * (2 * kLapTabN + 1)) {
-    const int n = t / (2 * kLapTabN + 1), mu = t % (2 * kLapTabN + 1) - kLapTabN;
-    T->lb[n][mu + kLapTabN] = (mu < 0 ? -mu : mu) <= n ? lad_s(mu) * lad_b(n, mu) : 0.0;
-  }
 }
 
 // G lanes per target (G a power of two): the columns k of the local
@@ -994,9 +1001,10 @@ __global__ __launch_bounds__(128) void k_lap_field_vec(
   const int nout = vec_width(mode, nq);
 #pragma unroll
   for (int i = 0; i < NO; i++) {
-    if (i >= nout) break;
-    const double v = group_sum<G>(out[i]);
-    if (lane == 0) o[i] += v;
+    if (i < nout) {
+      const double v = group_sum<G>(out[i]);
+      if (lane == 0) o[i] += v;
+    }
   }
 }
 
@@ -1185,18 +1193,21 @@ static int lap_p2m_wave(const uint32_t *boxes, unsigned nbox, const uint32_t *st
   if (N < 0 || N > kMaxN) return WBFMM_HIP_ERR_ORDER;
   if (nbox == 0) return 0;
   const size_t C = (size_t)(N + 1) * (N + 1);
+  const LapTab *tab = nullptr;
+  const int rc = lap_tab(&tab);
+  if (rc) return rc;
   if (N <= 15) {
     WBFMM_LAUNCH(name, (k_lap_p2m_wave<T, 16>), dim3(nbox), dim3(64), 4 * C * sizeof(double),
                  boxes, nbox, start, end, xyz, q, nrm, dip, (int)level, x0[0], x0[1], x0[2], D,
-                 N, rs, mps);
+                 N, rs, mps, tab);
   } else if (N <= 31) {
     WBFMM_LAUNCH(name, (k_lap_p2m_wave<T, 32>), dim3(nbox), dim3(64), 2 * C * sizeof(double),
                  boxes, nbox, start, end, xyz, q, nrm, dip, (int)level, x0[0], x0[1], x0[2], D,
-                 N, rs, mps);
+                 N, rs, mps, tab);
   } else {
     WBFMM_LAUNCH(name, (k_lap_p2m_wave<T, 64>), dim3(nbox), dim3(64), C * sizeof(double),
                  boxes, nbox, start, end, xyz, q, nrm, dip, (int)level, x0[0], x0[1], x0[2], D,
-                 N, rs, mps);
+                 N, rs, mps, tab);
   }
   return 0;
 }

@@ -771,14 +771,17 @@ int wbfmm_hip_compact_boxes(const uint32_t *start, const uint32_t *end,
 }
 
 // points in Morton order: positions (4 doubles), codes and caller indices;
-// raw: scratch of 4 n doubles; *nbad: points outside the domain
+// raw: scratch of 4 n doubles; *nbad: points outside the domain; low: the
+// lowest bits of the codes left out of the order (a multiple of 3: points
+// of one box of level 20 - low / 3 keep the caller's order)
 int wbfmm_hip_points_sorted(const void *pts, size_t pstr, unsigned n, const double *x0, double D,
-                            double *raw, double *xyz, uint64_t *codes, uint32_t *idx,
+                            int low, double *raw, double *xyz, uint64_t *codes, uint32_t *idx,
                             unsigned *nbad) {
   *nbad = 0;
+  if (low < 0 || low > 57) return WBFMM_HIP_ERR_ARG;
   if (n == 0) return 0;
   size_t sort_bytes = 0;
-  WBFMM_CHECK(rocprim::radix_sort_pairs(nullptr, sort_bytes, codes, codes, idx, idx, n, 0, 60,
+  WBFMM_CHECK(rocprim::radix_sort_pairs(nullptr, sort_bytes, codes, codes, idx, idx, n, low, 60,
                                         stream()));
   // one block: counter, unsorted codes and indices, the caller's strided
   // host block as it lies, the sort's scratch
@@ -801,8 +804,8 @@ int wbfmm_hip_points_sorted(const void *pts, size_t pstr, unsigned n, const doub
   WBFMM_LAUNCH("tree_morton", k_morton, dim3(nblk(n, 256)), dim3(256), 0, dpts, pstr, n, x0[0],
                x0[1], x0[2], D, raw, tcodes, tidx, (unsigned *)tmp);
   timing_begin("tree_sort");
-  WBFMM_CHECK(rocprim::radix_sort_pairs(tmp + o_sort, sort_bytes, tcodes, codes, tidx, idx, n, 0,
-                                        60, stream()));
+  WBFMM_CHECK(rocprim::radix_sort_pairs(tmp + o_sort, sort_bytes, tcodes, codes, tidx, idx, n,
+                                        low, 60, stream()));
   timing_end("tree_sort");
   WBFMM_LAUNCH("gather4", k_gather4, dim3(nblk(n, 256)), dim3(256), 0, raw, idx, n, xyz);
   WBFMM_CHECK(hipMemcpyAsync(nbad, tmp, sizeof(unsigned), hipMemcpyDeviceToHost, stream()));

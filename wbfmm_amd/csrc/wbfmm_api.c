@@ -653,7 +653,7 @@ static gint add_points_dbl(wbfmm_tree_t *t, gpointer pts, gsize pstr, gpointer n
   t->normals = (char *)normals;
   t->nstr = nstr;
   t->sorted = sorted;
-  HIPOK(wbfmm_hip_points_sorted(pts, pstr, npts, x0, t->D, td->d_xyz_raw, td->d_xyz,
+  HIPOK(wbfmm_hip_points_sorted(pts, pstr, npts, x0, t->D, 0, td->d_xyz_raw, td->d_xyz,
                                 td->d_codes, td->d_idx, &nbad));
   if (nbad)
     WBFMM_FATAL("%u points do not lie in box of width %g at (%g,%g,%g)", nbad,
@@ -1566,11 +1566,13 @@ gint wbfmm_laplace_downward_pass_avx(wbfmm_tree_t *t,
   return lap_downward(t, op, level);
 }
 
-/* stage n points (host or device, byte stride) as 4-double device rows
-   with identity ids; returns device buffers that the caller frees */
+/* stage n points (host or device, byte stride) as 4-double device rows, in
+   the order of the boxes of level `depth' when sort_them (a fraction of the
+   passes that a sort by the whole code takes; the order within a box is
+   the caller's); returns device buffers that the caller frees */
 static void stage_targets(const void *xt, size_t tstr, unsigned n,
                           double **dx, uint32_t **did, uint64_t **dcodes,
-                          const double *x0, double D, int sort_them)
+                          const double *x0, double D, int depth, int sort_them)
 {
   unsigned nbad = 0;
   double *raw;
@@ -1579,7 +1581,8 @@ static void stage_targets(const void *xt, size_t tstr, unsigned n,
   HIPOK(wbfmm_hip_malloc((void **)did, sizeof(uint32_t) * (n ? n : 1)));
   HIPOK(wbfmm_hip_malloc((void **)dcodes, sizeof(uint64_t) * (n ? n : 1)));
   if (sort_them)
-    HIPOK(wbfmm_hip_points_sorted(xt, tstr, n, x0, D, raw, *dx, *dcodes, *did, &nbad));
+    HIPOK(wbfmm_hip_points_sorted(xt, tstr, n, x0, D, depth > 0 && depth < 20 ? 60 - 3 * depth : 0,
+                                  raw, *dx, *dcodes, *did, &nbad));
   else
     HIPOK(wbfmm_hip_morton(xt, tstr, n, x0, D, *dx, *dcodes, *did, &nbad));
   if (nbad)
@@ -1680,7 +1683,7 @@ gint wbfmm_laplace_field_targets(wbfmm_tree_t *t, gdouble *xt, gsize tstr,
   if (fstr < lap_vec_width(fl, (int)t->nq)) return -2;
   if (ntgt == 0) return 0;
   stage_targets(xt, tstr, ntgt, &dx, &did, &dc, ORIGIN(t),
-                t->D, 1);
+                t->D, (int)t->depth, 1);
   lap_field_run(td, dx, did, ntgt, src, sstr, d, dstr, fl, f, fstr, ntgt);
   HIPOK(wbfmm_hip_sync());
   wbfmm_hip_free(dx);
@@ -1720,7 +1723,7 @@ gint wbfmm_laplace_box_field(wbfmm_tree_t *t, guint level, guint b,
   if ((fl & 4) && t->nq < 3)
     WBFMM_FATAL("not enough source components (%u) for curl calculation", t->nq);
   stage_targets(x, 3 * sizeof(double), 1, &dx, &did, &dc,
-                ORIGIN(t), t->D, 0);
+                ORIGIN(t), t->D, 0, 0);
   if (!eval_neighbours) { src = NULL; d = NULL; }
   {
     /* potential: component k at f[k fstr]; gradient: d_j of component k
@@ -1924,8 +1927,10 @@ gint wbfmm_target_list_add_points(wbfmm_target_list_t *l, gpointer pts,
   l->points = (char *)pts;
   l->pstr = pstr;
   l->npoints = npts;
-  stage_targets(pts, pstr, npts, &ld->d_xt, &ld->d_tid, &ld->d_codes,
-                ORIGIN(l->t), l->t->D, 1);
+  /* (a Helmholtz list's codes are also segmented at the depth the tree has
+     when the field is asked for: wbfmm_hip_hel_field_box) */
+  stage_targets(pts, pstr, npts, &ld->d_xt, &ld->d_tid, &ld->d_codes, ORIGIN(l->t), l->t->D,
+                l->t->problem == WBFMM_PROBLEM_LAPLACE ? (int)l->t->depth : 0, 1);
   register_targets(td, ld->d_codes, npts);
   return 0;
 }
@@ -3100,7 +3105,7 @@ gint wbfmm_tree_box_local_field(wbfmm_tree_t *t, guint level, guint b, gdouble k
       WBFMM_FATAL("unrecognized field identifier (%u)", field);
   }
   stage_targets(x, 3 * sizeof(double), 1, &dx, &did, &dc, ORIGIN(t),
-                t->D, 0);
+                t->D, 0, 0);
   if (!eval_neighbours) { src = NULL; d = NULL; }
   hel_field_run(td, k, dx, did, dc, 1, src, sstr, d, dstr, fl, tmp, 8, 1);
   for (i = 0; i < (fl == 1 ? 2 : 6); i++) f[i] += tmp[i];
@@ -3127,7 +3132,7 @@ gint wbfmm_helmholtz_field_targets(wbfmm_tree_t *t, gdouble k, gdouble *xt,
   if (fl == 0 || (field & ~3u)) return -2;
   if (fstr < ((fl & 1) ? 2 : 0) + ((fl & 2) ? 6 : 0)) return -2;
   if (ntgt == 0) return 0;
-  stage_targets(xt, tstr, ntgt, &dx, &did, &dc, ORIGIN(t), t->D, 1);
+  stage_targets(xt, tstr, ntgt, &dx, &did, &dc, ORIGIN(t), t->D, (int)t->depth, 1);
   hel_field_run(td, k, dx, did, dc, ntgt, src, sstr, d, dstr, fl, f, fstr, ntgt);
   HIPOK(wbfmm_hip_sync());
   wbfmm_hip_free(dx);
