@@ -68,6 +68,10 @@ int wbfmm_hip_mem_info(size_t *free_bytes, size_t *total_bytes);
    returns after the copy when a host buffer is involved */
 int wbfmm_hip_memcpy(void *dst, const void *src, size_t bytes);
 int wbfmm_hip_memset(void *p, int v, size_t bytes);
+/* zeroes rows list[0..n) (device) of each of `planes' arrays of `rows' rows
+   of row_bytes bytes (a multiple of 4), one after the other from p */
+int wbfmm_hip_clear_rows(void *p, const uint32_t *list, unsigned n, size_t rows,
+                         size_t row_bytes, unsigned planes);
 /* 1 when p is device (or managed) memory, 0 for host memory */
 int wbfmm_hip_is_device(const void *p);
 int wbfmm_hip_sync(void);

@@ -1,0 +1,79 @@
+"""A tree used again clears its level arrays by the boxes that were written
+(wbfmm_hip_clear_rows): every level of the second and third solve must hold
+what a fresh tree of the same points holds, and zeros in every other box."""
+
+import ctypes
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def sphere(rng, n, cap):
+    """n points on the unit sphere, z above or below as cap says"""
+    x = rng.normal(size=(n, 3))
+    x /= np.linalg.norm(x, axis=1)[:, None]
+    if cap:
+        x[:, 2] = cap * np.abs(x[:, 2])
+    return np.ascontiguousarray(x)
+
+
+@pytest.mark.parametrize("kind", ["laplace", "fp32", "vector", "helmholtz", "mixed"])
+def test_reused_tree(wb, kind):
+    rng = np.random.default_rng(3)
+    n, depth, p = 700, 4, 6
+    helm, nq = kind in ("helmholtz", "mixed"), 3 if kind == "vector" else 1
+    bits = 32 if kind in ("fp32", "mixed") else 64
+    orders = [0, p] + [p] * (depth - 1)
+    x0, D = np.array([-1.1, -1.1, -1.1]), 2.2
+    q = rng.normal(size=(n, 2 if helm else nq))
+
+    def solver(xs, xt):
+        if helm:
+            return wb.HelmholtzSolver(xs, x0, D, depth, orders, orders, 2.0, targets=xt,
+                                      precision=bits)
+        return wb.LaplaceSolver(xs, x0, D, depth, orders, orders, targets=xt, precision=bits,
+                                host_mirror=False, nq=nq)
+
+    def levels(s):
+        return [s.coefficients(l, w) for l in range(2, depth + 1) for w in (0, 1)]
+
+    # above, below, everywhere; registered targets, then none
+    sets = [(sphere(rng, n, c), t) for c, t in ((1, 1), (-1, 1), (0, 1), (1, 0), (-1, 1))]
+    used = solver(sets[0][0], sets[0][0])
+    for xs, with_targets in sets:
+        xt = sphere(rng, n, 0)[:300] if with_targets else None
+        used.xs, used.targets, used.ntgt = xs, xt, 300
+        fresh = solver(xs, xt)
+        for s in (used, fresh):
+            s.build_tree()
+            s.passes(q, sstr=q.shape[1])
+            s.passes(q, sstr=q.shape[1])   # (clears whole levels first)
+        for a, b in zip(levels(used), levels(fresh)):
+            assert np.abs(b).max() > 0
+            assert np.array_equal(a, b)
+        # the same points again: levels cleared by the lists of the first time
+        used.build_tree()
+        used.passes(q, sstr=q.shape[1])
+        for a, b in zip(levels(used), levels(fresh)):
+            assert np.array_equal(a, b)
+        fresh.close()
+    used.close()
+
+
+@pytest.mark.parametrize("row", [4, 36, 1352, 4608])
+@pytest.mark.parametrize("n", [0, 1, 5, 63])
+def test_clear_rows(wb, row, n):
+    rng = np.random.default_rng(row + n)
+    rows, planes = 64, 3
+    a = rng.integers(1, 255, (planes, rows, row), dtype=np.uint8)
+    lst = np.sort(rng.permutation(rows)[:n]).astype(np.uint32)
+    d, dl = wb.DeviceBuffer.from_array(a), wb.DeviceBuffer.from_array(
+        lst if n else np.zeros(1, np.uint32))
+    f = wb.lib().wbfmm_hip_clear_rows
+    vp, sz, u = ctypes.c_void_p, ctypes.c_size_t, ctypes.c_uint
+    assert f(vp(d.ptr), vp(dl.ptr), u(n), sz(rows), sz(row), u(planes)) == 0
+    wb.sync()
+    a[:, lst] = 0
+    assert np.array_equal(d.download(np.zeros_like(a)), a)

@@ -573,7 +573,6 @@ int solve_body(void *arg) {
   rc = wbfmm_hip_memset(S.df, 0, sizeof(double) * S.fw * std::max(S.ntgt, 1u));
   if (rc) return rc;
 
-  for (int l = 1; l <= p.depth; l++) wbfmm_tree_coefficients_zero(t, (guint)l);
   if (helm) {
     wbfmm_tree_leaf_expansions(t, r.k, const_cast<double *>(r.q), cplx,
                                const_cast<double *>(r.dip), cplx, TRUE, nullptr);

@@ -138,6 +138,10 @@ typedef struct {
   int have_targets; /* d_flag/d_act describe the current points */
   unsigned tgt_levels; /* the levels 0..tgt_levels-1 of them */
   size_t mps_bytes[WBFMM_TREE_MAX_DEPTH + 1], mpr_bytes[WBFMM_TREE_MAX_DEPTH + 1];
+  /* bytes per box of mps[l] (0) and mpr[l] (1), and what the array holds
+     (LEVEL_*) */
+  size_t box_bytes[2][WBFMM_TREE_MAX_DEPTH + 1];
+  unsigned char held[2][WBFMM_TREE_MAX_DEPTH + 1];
   double *d_q, *d_dip; /* strengths in sorted order */
   unsigned cap_q, cap_dip;
   int prec32; /* FP32 coefficients scaled by the box width (Laplace) */
@@ -558,6 +562,51 @@ gint wbfmm_tree_host_mirror(wbfmm_tree_t *t, gboolean on)
   return 0;
 }
 
+/* What a level array holds: zeros; zeros but in the boxes of d_occ (mps) or
+   d_act (mpr), whose lists and counts are those that the passes wrote it
+   by; or values anywhere.  An array is cleared by the boxes that were
+   written, and not at all when none was.  Trees with a host mirror hand out
+   pointers into the arrays (box mps, mpr): theirs are always cleared
+   whole. */
+enum { LEVEL_ZERO, LEVEL_LISTED, LEVEL_ANY };
+
+/* the passes are about to write boxes of the current lists (listed) or any
+   boxes of a level array */
+static void level_written(tree_dev *td, unsigned l, int which, int listed)
+{
+  unsigned char *h = &td->held[which][l];
+  if (!listed) *h = LEVEL_ANY;
+  else if (*h == LEVEL_ZERO) *h = LEVEL_LISTED;
+}
+
+/* the lists of levels lo..hi are about to change */
+static void level_lists_change(tree_dev *td, unsigned lo, unsigned hi, int which)
+{
+  unsigned l;
+  for (l = lo; l <= hi; l++)
+    if (td->held[which][l] == LEVEL_LISTED) td->held[which][l] = LEVEL_ANY;
+}
+
+/* zero a level array: by the list up to half of the boxes, where the list
+   writes less and reaches nearly the rate of the fill (1e6 points in a cube
+   at depth 7, 38 % of the leaf boxes: solve 76.0 -> 75.1 ms; on a sphere,
+   5 %: 51.7 -> 46.3) */
+static void level_clear(tree_dev *td, unsigned l, int which)
+{
+  void *p = which ? td->t.mpr[l] : td->t.mps[l];
+  const size_t bytes = which ? td->mpr_bytes[l] : td->mps_bytes[l], nb = (size_t)1 << (3 * l);
+  const size_t row = td->box_bytes[which][l];
+  const uint32_t *list = which ? td->d_act[l] : td->d_occ[l];
+  const unsigned n = which ? td->nact[l] : td->nocc[l];
+  const int held = td->host_mirror ? LEVEL_ANY : td->held[which][l];
+  if (held == LEVEL_ZERO) return;
+  if (held == LEVEL_LISTED && n <= nb / 2)
+    HIPOK(wbfmm_hip_clear_rows(p, list, n, nb, row, (unsigned)(bytes / (nb * row))));
+  else
+    HIPOK(wbfmm_hip_memset(p, 0, bytes));
+  td->held[which][l] = LEVEL_ZERO;
+}
+
 /* box ranges and occupied lists of the levels up to the tree's depth, as far
    as they are not built, without waiting for the device */
 static void build_levels(tree_dev *td)
@@ -565,6 +614,7 @@ static void build_levels(tree_dev *td)
   const unsigned lo = td->built, hi = td->t.depth;
   unsigned l;
   if (lo > hi) return;
+  level_lists_change(td, lo, hi, 0);
   for (l = lo; l <= hi; l++)
     if (!td->d_start[l]) {
       /* start, end and list in one block */
@@ -746,6 +796,7 @@ gint wbfmm_tree_coefficients_zero(wbfmm_tree_t *t, guint level)
   tree_dev *td = TD(t);
   if (t->mps[level]) HIPOK(wbfmm_hip_memset(t->mps[level], 0, td->mps_bytes[level]));
   if (t->mpr[level]) HIPOK(wbfmm_hip_memset(t->mpr[level], 0, td->mpr_bytes[level]));
+  td->held[0][level] = td->held[1][level] = LEVEL_ZERO;
   return 0;
 }
 
@@ -859,25 +910,28 @@ static void set_box_pointers(tree_dev *td, unsigned l, int which, int C)
   }
 }
 
-static void alloc_level(tree_dev *td, unsigned l, int which, size_t bytes)
+/* level array of box_bytes per box and `planes' components, zeroed */
+static void alloc_level(tree_dev *td, unsigned l, int which, size_t box_bytes, unsigned planes)
 {
   wbfmm_tree_t *t = &td->t;
   void **slot = which ? &t->mpr[l] : &t->mps[l];
   size_t *have = which ? &td->mpr_bytes[l] : &td->mps_bytes[l];
+  const size_t bytes = (box_bytes << (3 * l)) * planes;
   if (*slot && *have != bytes) {
     wbfmm_hip_free(*slot);
     *slot = NULL;
   }
+  if (!*slot || td->box_bytes[which][l] != box_bytes) td->held[which][l] = LEVEL_ANY;
   if (!*slot) HIPOK(wbfmm_hip_malloc(slot, bytes));
   *have = bytes;
-  HIPOK(wbfmm_hip_memset(*slot, 0, bytes));
+  td->box_bytes[which][l] = box_bytes;
+  level_clear(td, l, which);
 }
 
 gint wbfmm_tree_laplace_coefficient_init(wbfmm_tree_t *t, guint l, guint nr,
                                          guint ns)
 {
   tree_dev *td = TD(t);
-  size_t nb = (size_t)1 << (3 * l);
   if ((int)t->nq < 1)
     WBFMM_FATAL("tree has invalid number of components in source terms (%d)", t->nq);
   if ((int)t->nq > LAP_MAX_NQ)
@@ -897,11 +951,11 @@ gint wbfmm_tree_laplace_coefficient_init(wbfmm_tree_t *t, guint l, guint nr,
        q 8^l (n+1)^2 (box pointers, when mirrored, point into plane 0) */
     const size_t es = td->prec32 ? sizeof(float) : sizeof(double);
     if (ns) {
-      alloc_level(td, l, 0, t->nq * nb * (ns + 1) * (ns + 1) * es);
+      alloc_level(td, l, 0, (ns + 1) * (ns + 1) * es, t->nq);
       if (td->host_mirror) set_box_pointers(td, l, 0, (ns + 1) * (ns + 1));
     }
     if (nr) {
-      alloc_level(td, l, 1, t->nq * nb * (nr + 1) * (nr + 1) * es);
+      alloc_level(td, l, 1, (nr + 1) * (nr + 1) * es, t->nq);
       if (td->host_mirror) set_box_pointers(td, l, 1, (nr + 1) * (nr + 1));
     }
   }
@@ -955,10 +1009,11 @@ gint wbfmm_tree_laplace_leaf_expansions(wbfmm_tree_t *t, gdouble *src,
   if (t->problem != WBFMM_PROBLEM_LAPLACE) WBFMM_FATAL("tree is not a Laplace tree");
   if (!t->mps[d]) WBFMM_FATAL("coefficients not initialised at level %u", d);
   tree_counts(td);
-  if (zero_expansions) HIPOK(wbfmm_hip_memset(t->mps[d], 0, td->mps_bytes[d]));
+  if (zero_expansions) level_clear(td, d, 0);
   if (src == NULL && dipoles == NULL) return 0;
   if (t->normals == NULL && dipoles != NULL)
     WBFMM_FATAL("no normals in tree but dipole strengths specified (dipoles != NULL)");
+  level_written(td, d, 0, 1);
   /* one wavefront per box where the occupied leaves hold 4 or more points
      on average, one thread per box otherwise */
   wave = t->npoints >= 4u * td->nocc[d];
@@ -1355,6 +1410,7 @@ gint wbfmm_laplace_upward_pass(wbfmm_tree_t *t, wbfmm_shift_operators_t *op,
     WBFMM_FATAL("operators built to order %d, tree needs %u", od->lay.L,
                 t->order_s[level] > t->order_s[level - 1] ? t->order_s[level] : t->order_s[level - 1]);
   tree_counts(td);
+  level_written(td, level - 1, 0, 1);
   if (td->prec32) {
     int N = (int)t->order_s[level];
     if (t->order_s[level - 1] != t->order_s[level] || !mfma_order(N))
@@ -1484,6 +1540,9 @@ static gint lap_downward(wbfmm_tree_t *t, wbfmm_shift_operators_t *op,
   } else {
     tl = all_boxes(level, &nt);
   }
+  level_written(td, level, 1, td->have_targets && level < td->tgt_levels);
+  if (level < t->depth)
+    level_written(td, level + 1, 1, td->have_targets && level + 1 < td->tgt_levels);
   if (td->prec32) {
     int N = (int)t->order_s[level];
     unsigned cstart[8], ccount[8];
@@ -1897,6 +1956,7 @@ static void register_targets(tree_dev *td, const uint64_t *dcodes, unsigned n)
 {
   unsigned l;
   build_levels(td);
+  level_lists_change(td, 0, WBFMM_TREE_MAX_DEPTH, 1);
   for (l = 0; l <= td->t.depth; l++)
     if (!td->d_flag[l]) {
       /* flags, list and class list in one block */
@@ -2045,7 +2105,7 @@ gint wbfmm_hip_synchronize(void) { return wbfmm_hip_sync(); }
 gint wbfmm_tree_coefficient_init(wbfmm_tree_t *t, guint l, guint nr, guint ns)
 {
   tree_dev *td = TD(t);
-  size_t nb = (size_t)1 << (3 * l), es = td->prec32 ? sizeof(float) : sizeof(double);
+  const size_t es = td->prec32 ? sizeof(float) : sizeof(double);
   if ((int)t->nq < 1)
     WBFMM_FATAL("tree has invalid number of components in source terms (%d)", t->nq);
   if (t->nq != 1) WBFMM_FATAL("only nq == 1 is supported (nq = %u)", t->nq);
@@ -2062,11 +2122,11 @@ gint wbfmm_tree_coefficient_init(wbfmm_tree_t *t, guint l, guint nr, guint ns)
   td->h64[l] = 0;
   td->hk_set = 0;
   if (ns) {
-    alloc_level(td, l, 0, nb * 2 * (ns + 1) * (ns + 1) * es);
+    alloc_level(td, l, 0, 2 * (ns + 1) * (ns + 1) * es, 1);
     if (td->host_mirror) set_box_pointers(td, l, 0, 2 * (ns + 1) * (ns + 1));
   }
   if (nr) {
-    alloc_level(td, l, 1, nb * 2 * (nr + 1) * (nr + 1) * es);
+    alloc_level(td, l, 1, 2 * (nr + 1) * (nr + 1) * es, 1);
     if (td->host_mirror) set_box_pointers(td, l, 1, 2 * (nr + 1) * (nr + 1));
   }
   return 0;
@@ -2118,14 +2178,13 @@ static void hel_prepare(wbfmm_tree_t *t, double k)
   if (!td->prec32 || (td->hk_set && td->hk == k)) return;
   for (l = 1; l <= t->depth; l++) {
     const unsigned ns = t->order_s[l], nr = t->order_r[l], N = ns > nr ? ns : nr;
-    const size_t nb = (size_t)1 << (3 * l);
     const int want64 = hel_scale_arg(k, t->D, l) > hel_fp64_ka() || ns != nr ||
                        (int)N < M2L_MFMA_MIN || (int)N > HEL_MFMA_MAX ||
                        l > M2L_MFMA_MAX_LEVEL;
     if (want64 != td->h64[l]) {
       const size_t es = want64 ? sizeof(double) : sizeof(float);
-      if (ns && t->mps[l]) alloc_level(td, l, 0, nb * 2 * (ns + 1) * (ns + 1) * es);
-      if (nr && t->mpr[l]) alloc_level(td, l, 1, nb * 2 * (nr + 1) * (nr + 1) * es);
+      if (ns && t->mps[l]) alloc_level(td, l, 0, 2 * (ns + 1) * (ns + 1) * es, 1);
+      if (nr && t->mpr[l]) alloc_level(td, l, 1, 2 * (nr + 1) * (nr + 1) * es, 1);
       td->h64[l] = want64;
     }
     free(td->hsc[l]);
@@ -2164,10 +2223,11 @@ gint wbfmm_tree_leaf_expansions(wbfmm_tree_t *t, gdouble k, gdouble *src,
   if (!t->mps[d]) WBFMM_FATAL("coefficients not initialised at level %u", d);
   tree_counts(td);
   hel_prepare(t, k); /* mixed precision: the levels' precision follows k */
-  if (zero_expansions) HIPOK(wbfmm_hip_memset(t->mps[d], 0, td->mps_bytes[d]));
+  if (zero_expansions) level_clear(td, d, 0);
   if (src == NULL && dipoles == NULL) return 0;
   if (t->normals == NULL && dipoles != NULL)
     WBFMM_FATAL("no normals in tree but dipole strengths specified (dipoles != NULL)");
+  level_written(td, d, 0, 1);
   q = gather_strengths_n(td, src, sstr, 0, 2);
   dp = gather_strengths_n(td, dipoles, dstr, 1, 2);
   if (level_f32(td, d)) {
@@ -2405,6 +2465,7 @@ gint wbfmm_upward_pass(wbfmm_tree_t *t, wbfmm_shift_operators_t *op, guint level
   if ((Nc > Np ? Nc : Np) > od->ss_L[level] || (Nc > Np ? Nc : Np) > op->Lmax)
     WBFMM_FATAL("operators at level %u built to order %u", level, od->ss_L[level]);
   tree_counts(td);
+  level_written(td, level - 1, 0, 1);
   if (td->prec32) {
     hel_upward_mixed(t, od, level);
     return 0;
@@ -2749,6 +2810,9 @@ static gint hel_downward(wbfmm_tree_t *t, wbfmm_shift_operators_t *op, guint lev
   } else {
     tl = all_boxes(level, &nt);
   }
+  level_written(td, level, 1, td->have_targets && level < td->tgt_levels);
+  if (level < t->depth)
+    level_written(td, level + 1, 1, td->have_targets && level + 1 < td->tgt_levels);
   if (level < t->depth) {
     guint Nc = t->order_r[level + 1];
     if (!t->mpr[level + 1]) WBFMM_FATAL("coefficients not initialised at level %u", level + 1);
