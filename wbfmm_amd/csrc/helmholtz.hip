@@ -24,6 +24,7 @@
 //   L2P+P2P  one thread per target, regular functions streamed by order
 //            with the gradient in the re-indexed form of G&D (2004) eq 3.7
 
+#include <algorithm>
 #include <cstdio>
 #include <cstring>
 
@@ -94,25 +95,6 @@ __device__ inline void bessel_j(int N, double x, double *j) {
     j[n + 1] = (x > n + 1) ? j[n] * (2 * n + 1) / x - j[n - 1] : bessel_j_series(n + 1, x);
 }
 
-// j_n(x) of one order by the rule of bessel_j (upward recursion from j_0,
-// j_1 for x > n, the power series otherwise), so that the lanes of a
-// wavefront compute the orders side by side
-__device__ inline double bessel_j_one(int n, double x) {
-  if (!(x > 0.0)) return n == 0 ? 1.0 : 0.0;
-  const double j0 = sin(x) / x;
-  if (n == 0) return j0;
-  const double j1 = j0 / x - cos(x) / x;
-  if (n == 1) return j1;
-  if (!(x > n)) return bessel_j_series(n, x);
-  double a = j0, b = j1;
-  for (int q = 1; q < n; q++) {
-    const double c = b * (2 * q + 1) / x - a;
-    a = b;
-    b = c;
-  }
-  return b;
-}
-
 // spherical coordinates of x - x0: r, cos/sin theta, cos/sin phi
 __device__ __forceinline__ void sph(double dx, double dy, double dz, double &r,
                                     double &C, double &S, double &cp, double &sp) {
@@ -145,8 +127,8 @@ __device__ __forceinline__ double pbar_up(int n, int m, double C, double pn, dou
 
 // The factors of these recurrences per (n, m), as one table per process
 // built once on the device by the functions above (the same values), for
-// the field kernels: their loops over (n, m) are the same in every lane,
-// so the table is read with scalar loads instead of a square root and a
+// the field kernels and P2M: the loops of the former over (n, m) are the
+// same in every lane, so the table is read with scalar loads instead of a square root and a
 // division per factor and target.
 constexpr int kRT = WBFMM_HIP_MAX_ORDER + 3;
 struct RecTab {
@@ -156,6 +138,7 @@ struct RecTab {
   double pb[kRT][kRT];          // sqrt((i^2 - m^2) / (2 i - 1))
   double pd[kRT][kRT];          // 1 / sqrt(((i + 1)^2 - m^2) / (2 i + 3))
   double pc[kRT];               // sqrt((2 i + 1) / (2 i))
+  double df[kRT];               // (2 i + 1)!!
 };
 
 __global__ void k_rec_tab(RecTab *T) {
@@ -173,7 +156,37 @@ __global__ void k_rec_tab(RecTab *T) {
   if (t < kRT) {
     T->pa[t] = sqrt(2.0 * t + 1);
     T->pc[t] = t ? sqrt((2.0 * t + 1) / (2.0 * t)) : 1.0;
+    T->df[t] = 1.0;
+    for (int q = 1; q <= t; q++) T->df[t] *= 2 * q + 1;
   }
+}
+
+// j_n(x) of one order, 0 <= n <= WBFMM_HIP_MAX_ORDER + 1, by the rule of
+// bessel_j (upward recursion from j_0, j_1 for x > n, the power series
+// otherwise), so that the lanes of a wavefront compute the orders side by
+// side; x^n / (2n+1)!! with the double factorial from the table
+__device__ inline double bessel_j_tab(const RecTab *__restrict__ T, int n, double x) {
+  if (!(x > 0.0)) return n == 0 ? 1.0 : 0.0;
+  if (n >= 2 && !(x > n)) {
+    double pw = x, term = 1.0, s = 1.0;
+    const double x2 = x * x;
+    for (int q = 1; q < n; q++) pw *= x;
+    for (int q = 0; q < 80 && fabs(term) > 1e-17; q++) {
+      term *= -x2 / ((2 * q + 2) * (double)(2 * n + 2 * (q + 1) + 1));
+      s += term;
+    }
+    return s * (pw / T->df[n]);
+  }
+  const double j0 = sin(x) / x;
+  if (n == 0) return j0;
+  const double j1 = j0 / x - cos(x) / x;
+  double a = j0, b = j1;
+  for (int q = 1; q < n; q++) {
+    const double c = b * (2 * q + 1) / x - a;
+    a = b;
+    b = c;
+  }
+  return b;
 }
 
 // rec_a(n, m) for n >= -1, |m| <= n + 1 <= WBFMM_HIP_MAX_ORDER + 1
@@ -263,21 +276,34 @@ __device__ void coax_wave(const double2 *in, int Ni, double2 *out, int No,
 //       each;
 //   (2) column m of R_n^m(p) (n = m..N+1, m >= 0) for every (p, m), one
 //       thread each, into LDS;
-//   (3) every thread adds the batch's contributions, point by point in
-//       source order, to the coefficients n(n+1)+m it owns (tid + 256 i),
-//       held in registers until the box is done.
-// The sums run in source order per coefficient: results do not depend on
-// the launch.
+//   (3) every thread adds the batch's points, in source order, to the
+//       moments of the table slots (n, m >= 0) it owns (tid + 256 i): with
+//       w = q, -d nz, -d (nx + i ny)/2 and -d (nx - i ny)/2 of a point, the
+//       four products of the parts of w and of R, which give both
+//       sum w conj(R_n^m) and sum w conj(R_n^-m) = sum w R_n^m.
+// The derivative of R is a combination of its neighbours in (n, m) with
+// factors that no point enters, so it is taken once per box, of the
+// moments, instead of once per point: 16 multiply-adds per point and slot
+// where every coefficient took its six neighbours for each point; with the
+// constants of (1) and (2) from the table and e^{i m phi} by repeated
+// squaring (sincos of m atan2 before): 1e6 points with dipoles on a sphere,
+// order 23, 6.09 -> 3.26 ms; 100003 points, orders 25/23, 0.68 -> 0.32;
+// 30000 monopoles at order 30 0.28 -> 0.14.  Tasks of (1) and (2) lie order
+// by order, so that a wavefront's loops have about one length.
+// Sums in source order: results do not depend on the launch.
 constexpr int kP2MThreads = 256, kP2MBatch = 8;
-constexpr int kP2MCoef =
-    ((WBFMM_HIP_MAX_ORDER + 1) * (WBFMM_HIP_MAX_ORDER + 1) + kP2MThreads - 1) / kP2MThreads;
+constexpr int p2m_slots(int N) { return (N + 2) * (N + 3) / 2; }
+constexpr int kP2MSlots = (p2m_slots(WBFMM_HIP_MAX_ORDER) + kP2MThreads - 1) / kP2MThreads;
 
 // O: double2 (FP64 coefficients) or float2 (FP32 coefficients, each degree
 // n divided by sc[n] in FP64 before rounding; sc NULL: no scaling)
-// NC: coefficients per thread, ceil((N+1)^2 / 256); three blocks per CU
-// (the LDS of a batch is at most 60 KiB)
-template <typename O, int NC>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_hel_p2m(
+// NS: slots per thread, ceil((N+2)(N+3)/2 / 256); DIP: with dipoles; three
+// blocks per CU (the LDS of a batch and of two weights' moments is at most
+// 60 KiB), two with the dipoles' moments of three or four slots (above
+// order 29)
+template <typename O, int NS, bool DIP>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
+    DIP && NS > 2 ? 2 : 3))) void k_hel_p2m(
     const uint32_t *__restrict__ boxes, unsigned nbox,
     const uint32_t *__restrict__ start, const uint32_t *__restrict__ end,
     const double *__restrict__ xyz, const double2 *__restrict__ q,
@@ -296,105 +322,131 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
   const double xc = x0 + (compact3(b) + 0.5) * w, yc = y0 + (compact3(b >> 1) + 0.5) * w,
                zc = z0 + (compact3(b >> 2) + 0.5) * w;
   const uint32_t s0 = start[b], s1 = end[b];
-  double2 acc[NC];
+  // sums of wx x, wy y, wy x and wx y over the points, R = x + i y
+  constexpr int NW = DIP ? 4 : 1;
+  double mo[NS][NW][4];
 #pragma unroll
-  for (int i = 0; i < NC; i++) acc[i] = make_double2(0.0, 0.0);
+  for (int i = 0; i < NS; i++)
+#pragma unroll
+    for (int w4 = 0; w4 < 4 * NW; w4++) mo[i][w4 / 4][w4 % 4] = 0.0;
 
   for (uint32_t sb = s0; sb < s1; sb += (uint32_t)pb) {
     const int np = (int)min((uint32_t)pb, s1 - sb);
     for (int it = tid; it < np * (N1 + 1); it += kP2MThreads) {
-      const int p = it / (N1 + 1), n = it - p * (N1 + 1);
+      const int n = it / np, p = it - n * np;
       const uint32_t s = sb + p;
-      double r, C, S, cp, sp;
-      sph(xyz[4 * s] - xc, xyz[4 * s + 1] - yc, xyz[4 * s + 2] - zc, r, C, S, cp, sp);
-      jn[p * (N1 + 1) + n] = bessel_j_one(n, k * r);
+      const double dx = xyz[4 * s] - xc, dy = xyz[4 * s + 1] - yc, dz = xyz[4 * s + 2] - zc;
+      jn[p * (N1 + 1) + n] = bessel_j_tab(RT, n, k * sqrt(dx * dx + dy * dy + dz * dz));
     }
     __syncthreads();
     for (int it = tid; it < np * (N1 + 1); it += kP2MThreads) {
-      const int p = it / (N1 + 1), m = it - p * (N1 + 1);
+      const int m = it / np, p = it - m * np;
       const uint32_t s = sb + p;
       double r, C, S, cp, sp;
       sph(xyz[4 * s] - xc, xyz[4 * s + 1] - yc, xyz[4 * s + 2] - zc, r, C, S, cp, sp);
-      double sn, cs;
-      sincos((double)m * atan2(sp, cp), &sn, &cs);
+      double2 e = make_double2(1.0, 0.0), z = make_double2(cp, sp);  // (cp + i sp)^m
+      for (int h = m; h; h >>= 1) {
+        if (h & 1) e = cmul(e, z);
+        z = cmul(z, z);
+      }
       const double *j = jn + p * (N1 + 1);
       double2 *Rp = R + (size_t)p * NT;
-      double pv = pbar_mm(m, S), pprev = 0.0;
+      double pv = 1.0 / sqrt(4.0 * kPi), pprev = 0.0;  // Pbar_m^m
+      for (int h = 1; h <= m; h++) pv *= RT->pc[h] * S;
       for (int n = m; n <= N1; n++) {
-        Rp[n * (n + 1) / 2 + m] = make_double2(j[n] * pv * cs, j[n] * pv * sn);
+        Rp[n * (n + 1) / 2 + m] = make_double2(j[n] * pv * e.x, j[n] * pv * e.y);
         const double pn = (n + 1 <= N1) ? tab_pbar_up(RT, n, m, C, pv, pprev) : 0.0;
         pprev = pv;
         pv = pn;
       }
     }
     __syncthreads();
+    for (int p = 0; p < np; p++) {
+      const uint32_t s = sb + p;
+      double2 wt[NW];
+      wt[0] = q ? q[s] : make_double2(0.0, 0.0);
+      if constexpr (DIP) {
+        const double2 d = dip[s];
+        const double nx = 0.5 * nrm[4 * s], ny = 0.5 * nrm[4 * s + 1], nz = nrm[4 * s + 2];
+        wt[1] = make_double2(-d.x * nz, -d.y * nz);
+        wt[2] = make_double2(d.y * ny - d.x * nx, -(d.x * ny + d.y * nx));
+        wt[3] = make_double2(-(d.x * nx + d.y * ny), d.x * ny - d.y * nx);
+      }
+      const double2 *Rp = R + (size_t)p * NT;
 #pragma unroll
-    for (int i = 0; i < NC; i++) {
-      const int c = tid + kP2MThreads * i;
-      if (c >= N1 * N1) break;
-      const int n = isqrt_deg(c), mm = c - n * (n + 1);
-      // G&D 2004 eq 3.7 coefficients of this (n, mm)
-      const double a0 = tab_a(RT, n - 1, mm), a1 = -tab_a(RT, n, mm);
-      const double bp0 = tab_b(RT, n + 1, -mm - 1), bp1 = -tab_b(RT, n, mm);
-      const double bm0 = tab_b(RT, n + 1, mm - 1), bm1 = -tab_b(RT, n, -mm);
-      // the LDS slots of the R_{n'}^{m'} this coefficient reads, with
-      // R^{-m'} = conj R^{m'} as a sign on the imaginary part and a weight 0
-      // (slot 0) for (n', m') outside the table: (n, mm), (n - 1, mm),
-      // (n + 1, mm), (n + 1, mm + 1), (n - 1, mm + 1), (n + 1, mm - 1),
-      // (n - 1, mm - 1)
-      int ix[7];
-      double sx[7], sy[7];
-      {
-        const int nqs[7] = {n, n - 1, n + 1, n + 1, n - 1, n + 1, n - 1};
-        const int mqs[7] = {mm, mm, mm, mm + 1, mm + 1, mm - 1, mm - 1};
+      for (int i = 0; i < NS; i++) {
+        const int u = tid + kP2MThreads * i;
+        if (u >= NT) continue;
+        const double2 r = Rp[u];
 #pragma unroll
-        for (int e = 0; e < 7; e++) {
-          const int nq = nqs[e], mq = mqs[e];
-          const bool ok = !(nq < 0 || nq > N1 || mq > nq || -mq > nq);
-          ix[e] = ok ? nq * (nq + 1) / 2 + (mq < 0 ? -mq : mq) : 0;
-          sx[e] = ok ? 1.0 : 0.0;
-          sy[e] = ok ? (mq >= 0 ? 1.0 : -1.0) : 0.0;
+        for (int v = 0; v < NW; v++) {
+          mo[i][v][0] += wt[v].x * r.x;
+          mo[i][v][1] += wt[v].y * r.y;
+          mo[i][v][2] += wt[v].y * r.x;
+          mo[i][v][3] += wt[v].x * r.y;
         }
       }
-      double2 ac = acc[i];
-      for (int p = 0; p < np; p++) {
-        const uint32_t s = sb + p;
-        const double2 *Rp = R + (size_t)p * NT;
-        auto Rg = [&](int e) -> double2 {
-          const double2 v = Rp[ix[e]];
-          return make_double2(v.x * sx[e], v.y * sy[e]);
-        };
-        double2 v = make_double2(0.0, 0.0);
-        if (q) v = cmulc(q[s], Rg(0));
-        if (dip) {
-          const double2 dd = dip[s];
-          const double nx = nrm[4 * s], ny = nrm[4 * s + 1], nz = nrm[4 * s + 2];
-          const double2 dz = cscale(cadd(cscale(Rg(1), a0), cscale(Rg(2), a1)), k);
-          const double2 dp = cscale(cadd(cscale(Rg(3), bp0), cscale(Rg(4), bp1)), k);
-          const double2 dm = cscale(cadd(cscale(Rg(5), bm0), cscale(Rg(6), bm1)), k);
-          // gx = (dp + dm)/2, gy = -i (dp - dm)/2
-          const double2 gx = cscale(cadd(dp, dm), 0.5);
-          const double2 dd2 = cscale(cadd(dp, cscale(dm, -1.0)), 0.5);
-          const double2 gy = make_double2(dd2.y, -dd2.x);
-          const double2 g = cadd(cadd(cscale(gx, nx), cscale(gy, ny)), cscale(dz, nz));
-          const double2 t = cmulc(dd, g);
-          v = cadd(v, make_double2(-t.x, -t.y));
-        }
-        ac = cadd(ac, v);
-      }
-      acc[i] = ac;
     }
     __syncthreads();  // R and jn are rewritten by the next batch
   }
+  // the moments of two weights at a time through LDS, each slot as the sums
+  // for m and for -m; the weights of a phase that a box has not are left out
+  constexpr int NO = 2 * NS;  // coefficients per thread: (N + 1)^2 < 2 slots
+  double2 *M = smem;                     // [slot][weight of the phase][m, -m]
   O *out = mps + (size_t)b * N1 * N1;
+  double2 res[NO];
 #pragma unroll
-  for (int i = 0; i < NC; i++) {
+  for (int ph = 0; ph < (DIP ? 2 : 1); ph++) {
+#pragma unroll
+    for (int i = 0; i < NS; i++) {
+      const int u = tid + kP2MThreads * i;
+      if (u >= NT) continue;
+#pragma unroll
+      for (int v = 0; v < (DIP ? 2 : 1); v++) {
+        const double *a = mo[i][DIP ? 2 * ph + v : 0];
+        M[4 * u + 2 * v] = make_double2(a[0] + a[1], a[2] - a[3]);
+        M[4 * u + 2 * v + 1] = make_double2(a[0] - a[1], a[2] + a[3]);
+      }
+    }
+    __syncthreads();
+    // sum over the points of weight v's w conj(R_n^m), 0 outside the table
+    auto mom = [&](int v, int n, int m) -> double2 {
+      const int am = m < 0 ? -m : m;
+      if (n < 0 || am > n) return make_double2(0.0, 0.0);
+      return M[4 * (n * (n + 1) / 2 + am) + 2 * v + (m < 0 ? 1 : 0)];
+    };
+#pragma unroll
+    for (int i = 0; i < NO; i++) {
+      const int c = tid + kP2MThreads * i;
+      if (c >= N1 * N1) continue;
+      const int n = isqrt_deg(c), mm = c - n * (n + 1);
+      // G&D 2004 eq 3.7 coefficients of this (n, mm)
+      if (ph == 0) {
+        double2 v = mom(0, n, mm);
+        if constexpr (DIP)
+          v = cadd(v, cscale(cadd(cscale(mom(1, n - 1, mm), tab_a(RT, n - 1, mm)),
+                                  cscale(mom(1, n + 1, mm), -tab_a(RT, n, mm))), k));
+        res[i] = v;
+      } else {
+        const double2 dp =
+            cadd(cscale(mom(0, n + 1, mm + 1), tab_b(RT, n + 1, -mm - 1)),
+                 cscale(mom(0, n - 1, mm + 1), -tab_b(RT, n, mm)));
+        const double2 dm =
+            cadd(cscale(mom(1, n + 1, mm - 1), tab_b(RT, n + 1, mm - 1)),
+                 cscale(mom(1, n - 1, mm - 1), -tab_b(RT, n, -mm)));
+        res[i] = cadd(res[i], cscale(cadd(dp, dm), k));
+      }
+    }
+    if (DIP && ph == 0) __syncthreads();  // the next phase's moments take the place
+  }
+#pragma unroll
+  for (int i = 0; i < NO; i++) {
     const int c = tid + kP2MThreads * i;
     if (c < N1 * N1) {
       const double s = sc ? 1.0 / sc[isqrt_deg(c)] : 1.0;
       O o = out[c];
-      o.x += acc[i].x * s;
-      o.y += acc[i].y * s;
+      o.x += res[i].x * s;
+      o.y += res[i].y * s;
       out[c] = o;
     }
   }
@@ -533,11 +585,12 @@ struct HelFieldJ {
   static constexpr int n = G > 1 ? (128 / G) * (NMAX + 2) : 1;
 };
 template <int NMAX, int G>
-__device__ __forceinline__ const double *hel_field_bessel(int N, double x, int g, double *lds,
+__device__ __forceinline__ const double *hel_field_bessel(const RecTab *__restrict__ RT, int N,
+                                                          double x, int g, double *lds,
                                                           double *own) {
   if constexpr (G > 1) {
     double *J = lds + (threadIdx.x / G) * (NMAX + 2);
-    for (int nn = g; nn <= N + 1; nn += G) J[nn] = bessel_j_one(nn, x);
+    for (int nn = g; nn <= N + 1; nn += G) J[nn] = bessel_j_tab(RT, nn, x);
     __syncthreads();
     return J;
   } else {
@@ -548,7 +601,7 @@ __device__ __forceinline__ const double *hel_field_bessel(int N, double x, int g
 #define HEL_FIELD_BESSEL                                                        \
   __shared__ double jlds[HelFieldJ<NMAX, G>::n];                                \
   double jown[G > 1 ? 1 : NMAX + 2];                                            \
-  const double *jn = hel_field_bessel<NMAX, G>(N, k * r, g, jlds, jown);
+  const double *jn = hel_field_bessel<NMAX, G>(RT, N, k * r, g, jlds, jown);
 #define HEL_FIELD_STORE                                                         \
   const double2 v[4] = {pot, gx, gy, gz};                                       \
   double sum[8];                                                                \
@@ -1199,19 +1252,22 @@ int wbfmm_hip_hel_p2m(const uint32_t *boxes, unsigned nbox, const uint32_t *star
     if (rc) return rc;
   }
   {
-    const int nc = ((N + 1) * (N + 1) + kP2MThreads - 1) / kP2MThreads;
-#define HP2M(NCV) \
-    WBFMM_LAUNCH("hel_p2m", (k_hel_p2m<double2, NCV>), dim3(nbox), dim3(kP2MThreads), per * pb, boxes, \
-                 nbox, start, end, xyz, (const double2 *)q, nrm, (const double2 *)dip, level, \
-                 x0[0], x0[1], x0[2], D, N, k, pb, (const double *)nullptr, (double2 *)mps, RT)
-    switch (nc) {
+    const int ns = (p2m_slots(N) + kP2MThreads - 1) / kP2MThreads;
+    const size_t lds = std::max(per * pb, 4 * sizeof(double2) * (size_t)p2m_slots(N));
+#define HP2M(NSV) \
+    if (dip) \
+      WBFMM_LAUNCH("hel_p2m", (k_hel_p2m<double2, NSV, true>), dim3(nbox), dim3(kP2MThreads), lds, boxes, \
+                   nbox, start, end, xyz, (const double2 *)q, nrm, (const double2 *)dip, level, \
+                   x0[0], x0[1], x0[2], D, N, k, pb, (const double *)nullptr, (double2 *)mps, RT); \
+    else \
+      WBFMM_LAUNCH("hel_p2m", (k_hel_p2m<double2, NSV, false>), dim3(nbox), dim3(kP2MThreads), lds, boxes, \
+                   nbox, start, end, xyz, (const double2 *)q, nrm, (const double2 *)dip, level, \
+                   x0[0], x0[1], x0[2], D, N, k, pb, (const double *)nullptr, (double2 *)mps, RT)
+    switch (ns) {
       case 1: HP2M(1); break;
       case 2: HP2M(2); break;
       case 3: HP2M(3); break;
-      case 4: HP2M(4); break;
-      case 5: HP2M(5); break;
-      case 6: HP2M(6); break;
-      default: HP2M(kP2MCoef); break;
+      default: HP2M(kP2MSlots); break;
     }
 #undef HP2M
   }
@@ -1234,19 +1290,22 @@ int wbfmm_hip_hel_p2m_f32(const uint32_t *boxes, unsigned nbox, const uint32_t *
     if (rc) return rc;
   }
   {
-    const int nc = ((N + 1) * (N + 1) + kP2MThreads - 1) / kP2MThreads;
-#define HP2M(NCV) \
-    WBFMM_LAUNCH("hel_p2m_f32", (k_hel_p2m<float2, NCV>), dim3(nbox), dim3(kP2MThreads), per * pb, boxes, \
-                 nbox, start, end, xyz, (const double2 *)q, nrm, (const double2 *)dip, level, \
-                 x0[0], x0[1], x0[2], D, N, k, pb, scale, (float2 *)mps, RT)
-    switch (nc) {
+    const int ns = (p2m_slots(N) + kP2MThreads - 1) / kP2MThreads;
+    const size_t lds = std::max(per * pb, 4 * sizeof(double2) * (size_t)p2m_slots(N));
+#define HP2M(NSV) \
+    if (dip) \
+      WBFMM_LAUNCH("hel_p2m_f32", (k_hel_p2m<float2, NSV, true>), dim3(nbox), dim3(kP2MThreads), lds, boxes, \
+                   nbox, start, end, xyz, (const double2 *)q, nrm, (const double2 *)dip, level, \
+                   x0[0], x0[1], x0[2], D, N, k, pb, scale, (float2 *)mps, RT); \
+    else \
+      WBFMM_LAUNCH("hel_p2m_f32", (k_hel_p2m<float2, NSV, false>), dim3(nbox), dim3(kP2MThreads), lds, boxes, \
+                   nbox, start, end, xyz, (const double2 *)q, nrm, (const double2 *)dip, level, \
+                   x0[0], x0[1], x0[2], D, N, k, pb, scale, (float2 *)mps, RT)
+    switch (ns) {
       case 1: HP2M(1); break;
       case 2: HP2M(2); break;
       case 3: HP2M(3); break;
-      case 4: HP2M(4); break;
-      case 5: HP2M(5); break;
-      case 6: HP2M(6); break;
-      default: HP2M(kP2MCoef); break;
+      default: HP2M(kP2MSlots); break;
     }
 #undef HP2M
   }
