@@ -733,12 +733,16 @@ __global__ __launch_bounds__(128) void k_hel_field(
                                        make_double2(ir * ir, 0.0)));
       const double nx = nrm[4 * (size_t)s], ny = nrm[4 * (size_t)s + 1],
                    nz = nrm[4 * (size_t)s + 2];
-      const double nr = nx * ux + ny * uy + nz * uz;
+      // rounded once (rx / r): close points of a surface have n nearly
+      // orthogonal to x - y, where the sum loses what a second rounding of
+      // rx * (1 / r) would add (1e5 points on a sphere: 1e-13 of the largest)
+      const double vx = rx / r, vy = ry / r, vz = rz / r;
+      const double nr = nx * vx + ny * vy + nz * vz;
       pot = cadd(pot, cscale(cmul(dq, dG), nr));
       const double2 t1 = cscale(cmul(dq, G2), nr), t2 = cscale(cmul(dq, dG), ir);
-      gx = cadd(gx, cadd(cscale(t1, ux), cscale(t2, nx - nr * ux)));
-      gy = cadd(gy, cadd(cscale(t1, uy), cscale(t2, ny - nr * uy)));
-      gz = cadd(gz, cadd(cscale(t1, uz), cscale(t2, nz - nr * uz)));
+      gx = cadd(gx, cadd(cscale(t1, vx), cscale(t2, nx - nr * vx)));
+      gy = cadd(gy, cadd(cscale(t1, vy), cscale(t2, ny - nr * vy)));
+      gz = cadd(gz, cadd(cscale(t1, vz), cscale(t2, nz - nr * vz)));
     }
   });
   HEL_FIELD_STORE
