@@ -64,6 +64,10 @@ int wbfmm_hip_set_variant(int which, int value);
 int wbfmm_hip_get_variant(int which);
 /* free and total device memory */
 int wbfmm_hip_mem_info(size_t *free_bytes, size_t *total_bytes);
+/* bytes of freed blocks that the library keeps for its next allocations (at
+   most 1 GiB), and their return to the runtime's pool */
+size_t wbfmm_hip_pool_bytes(void);
+int wbfmm_hip_pool_release(void);
 /* copy of any kind (host/device either side), ordered on the stream;
    returns after the copy when a host buffer is involved */
 int wbfmm_hip_memcpy(void *dst, const void *src, size_t bytes);
@@ -275,6 +279,14 @@ int wbfmm_hip_lap_shift_tables(const wbfmm_m2l_plan_t *plan, double *A1,
    c t^(nu-n) (L2L), t = sqrt(3)/2 times the child box width */
 int wbfmm_hip_lap_shift_coax(const wbfmm_m2l_plan_t *plan, int kind, double t,
                              double *A2);
+/* The coaxial tables above at any width from those of width 1: the power of
+   the width in each of the KT x 64 entries (0 for an empty one) of kind 0,
+   1 (wbfmm_hip_lap_shift_coax) or 2 (wbfmm_hip_lap_m2l_coax, the same for
+   each length), and out[i] = unit[i] w^e[i mod period], i < n, on the
+   device (device arrays; powers within -100..100) */
+int wbfmm_hip_lap_coax_powers(const wbfmm_m2l_plan_t *plan, int kind, signed char *e);
+int wbfmm_hip_lap_coax_scale(const double *unit, const signed char *e, size_t n, size_t period,
+                             double w, double *out);
 /* MFMA M2M (mode 0: each listed parent from its children, child ranges
    cstart/cend; the parent is overwritten) or L2L (mode 1: each listed
    parent's local expansion added to its children with cflag != 0, all

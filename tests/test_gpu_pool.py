@@ -1,0 +1,98 @@
+"""Freed blocks kept by the library: handed out again on the stream that
+freed them and on no other, bounded, given back on request and with their
+stream, and not for streams that the library did not create."""
+
+import ctypes
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+MIB = 1 << 20
+_vp = ctypes.c_void_p
+
+
+@pytest.fixture
+def lib(wb):
+    L = wb.lib()
+    wb.sync()
+    L.wbfmm_hip_pool_release()
+    assert L.wbfmm_hip_pool_bytes() == 0
+    yield L
+    L.wbfmm_hip_set_stream(None, None)
+    wb.sync()
+    L.wbfmm_hip_pool_release()
+
+
+def take(L, n):
+    p = _vp()
+    assert L.wbfmm_hip_malloc(ctypes.byref(p), n) == 0
+    return p.value
+
+
+def test_reused_on_its_stream_only(wb, lib):
+    a = take(lib, 3 * MIB)
+    lib.wbfmm_hip_free(a)
+    assert lib.wbfmm_hip_pool_bytes() == 3 * MIB
+    s = _vp()
+    assert lib.wbfmm_hip_stream_create(ctypes.byref(s)) == 0
+    lib.wbfmm_hip_set_stream(s, None)
+    b = take(lib, 3 * MIB)
+    assert b != a and lib.wbfmm_hip_pool_bytes() == 3 * MIB
+    lib.wbfmm_hip_free(b)
+    assert lib.wbfmm_hip_pool_bytes() == 6 * MIB
+    lib.wbfmm_hip_set_stream(None, None)
+    assert lib.wbfmm_hip_stream_destroy(s) == 0        # b's block goes with its stream
+    assert lib.wbfmm_hip_pool_bytes() == 3 * MIB
+    assert take(lib, 3 * MIB - 100) == a               # a little smaller: the same block
+    assert lib.wbfmm_hip_pool_bytes() == 0
+    lib.wbfmm_hip_free(a)
+    c = take(lib, MIB)                                 # much smaller: not that block
+    assert c != a and lib.wbfmm_hip_pool_bytes() == 3 * MIB
+    lib.wbfmm_hip_free(c)
+
+
+def test_bounded(wb, lib):
+    ps = [take(lib, 200 * MIB) for _ in range(8)] + [take(lib, 300 * MIB)]
+    for p in ps:
+        lib.wbfmm_hip_free(p)
+    assert 0 < lib.wbfmm_hip_pool_bytes() <= 1024 * MIB
+    assert lib.wbfmm_hip_pool_bytes() % (200 * MIB) == 0   # (300 MiB: never kept)
+    assert lib.wbfmm_hip_pool_release() == 0 and lib.wbfmm_hip_pool_bytes() == 0
+
+
+def test_foreign_stream(wb, lib):
+    """a stream of the caller's: nothing kept, and a block of the library's
+    stream freed there goes back to the runtime"""
+    # the HIP runtime that the library has loaded
+    path = next(l.split()[-1] for l in open("/proc/self/maps") if "libamdhip64" in l)
+    hip = ctypes.CDLL(path)
+    s = _vp()
+    assert hip.hipStreamCreate(ctypes.byref(s)) == 0
+    a = take(lib, MIB)
+    wb.sync()
+    lib.wbfmm_hip_set_stream(s, None)
+    b = take(lib, MIB)
+    lib.wbfmm_hip_free(b)
+    lib.wbfmm_hip_free(a)
+    assert lib.wbfmm_hip_pool_bytes() == 0
+    lib.wbfmm_hip_set_stream(None, None)
+    assert hip.hipStreamSynchronize(s) == 0 and hip.hipStreamDestroy(s) == 0
+
+
+def test_contents_in_stream_order(wb, lib):
+    """a block handed out again while its last use is still queued"""
+    n = 8 * MIB // 8
+    want = np.arange(n, dtype=np.float64)
+    for rep in range(8):
+        a = wb.DeviceBuffer.from_array(want + rep)
+        c = wb.DeviceBuffer(8 * n)
+        assert lib.wbfmm_hip_memcpy(c.ptr, a.ptr, 8 * n) == 0   # device copy, queued
+        a.free()
+        b = wb.DeviceBuffer(8 * n)                              # the same block
+        b.zero()
+        assert np.array_equal(c.download(np.zeros(n)), want + rep)
+        assert not b.download(np.ones(n)).any()
+        b.free()
+        c.free()
