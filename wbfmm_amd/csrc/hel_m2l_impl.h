@@ -268,12 +268,15 @@ __device__ __forceinline__ void hel_m2l_loop(
   // the used offsets of this block's split as scalar bit words; the next
   // one after k by a scan of the words (216 when there is none)
   unsigned am[7];
+  int ks = split;  // the split's offsets: k = split (mod nsplit)
 #pragma unroll
   for (int w = 0; w < 7; w++) {
     unsigned v = __builtin_amdgcn_readfirstlane(anym[w]);
-    if (nsplit > 1)
-      for (int b = 0; b < 32; b++)
-        if ((32 * w + b) % nsplit != split) v &= ~(1u << b);
+    if (nsplit > 1) {
+      unsigned mine = 0;
+      for (; ks < 32 * (w + 1); ks += nsplit) mine |= 1u << (ks - 32 * w);
+      v &= mine;
+    }
     am[w] = v;
   }
   auto next_k = [&](int k) {
@@ -549,19 +552,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(
   hel_m2l_loop<T, N, W, WI>(R, tmap1, tmap2, tmap3, uinf, cs, vm, anym, lane, col, grp, tvalid,  \
                          tb, ti, tj, tk, px, py, pz, c, k8, split, nsplit, ca, P, A, A2, CS, \
                          zero, mps, mpr, part, ntot)
-  static_assert(W == 4 || W == 8 || W == 16, "four, eight or sixteen wavefronts per block");
-  if constexpr (W == 16) {
-    switch (wv) {
-      case 8: HEL_LOOP(8); return;
-      case 9: HEL_LOOP(9); return;
-      case 10: HEL_LOOP(10); return;
-      case 11: HEL_LOOP(11); return;
-      case 12: HEL_LOOP(12); return;
-      case 13: HEL_LOOP(13); return;
-      case 14: HEL_LOOP(14); return;
-      case 15: HEL_LOOP(15); return;
-    }
-  }
+  static_assert(W == 4 || W == 8, "four or eight wavefronts per block");
   if constexpr (W == 4) {
     switch (wv) {
       case 0: HEL_LOOP(0); break;
@@ -1050,9 +1041,6 @@ static int launch_hel_m2l(const uint32_t *cls, const ClassArgs &ca, unsigned nch
     fprintf(stderr, "wbfmm (HIP): M2L plan for order %d does not match the kernel's bins\n", N);
     return WBFMM_HIP_ERR_ARG;
   }
-  // the offsets of a chunk split over up to 8 blocks when there are few
-  // chunks (the split depends on the chunk count only: fixed summation
-  // order for a given problem)
   constexpr int C = (N + 1) * (N + 1);
   unsigned ntot = 0;
   for (int c = 0; c < 8; c++) ntot += ca.count[c];
@@ -1078,7 +1066,7 @@ static int launch_hel_m2l(const uint32_t *cls, const ClassArgs &ca, unsigned nch
       return 0;
     }
   }
-  const int nsplit = nchunks >= 1024 ? 1 : (int)(2048 / nchunks < 8 ? 2048 / nchunks : 8);
+  const int nsplit = m2l_nsplit(level, nchunks, sizeof(T2t<T>) * C);
   T2t<T> *part = nullptr;
   if (nsplit > 1 && dmalloc((void **)&part, sizeof(T2t<T>) * (size_t)nsplit * ntot * C))
     return WBFMM_HIP_ERR_NOMEM;

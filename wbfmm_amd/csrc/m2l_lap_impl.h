@@ -327,12 +327,15 @@ __device__ __forceinline__ void m2l_w2_loop(
   // the used offsets of this block's split as scalar bit words; the next
   // one after k by a scan of the words (216 when there is none)
   unsigned am[7];
+  int ks = split;  // the split's offsets: k = split (mod nsplit)
 #pragma unroll
   for (int w = 0; w < 7; w++) {
     unsigned v = __builtin_amdgcn_readfirstlane(anym[w]);
-    if (nsplit > 1)
-      for (int b = 0; b < 32; b++)
-        if ((32 * w + b) % nsplit != split) v &= ~(1u << b);
+    if (nsplit > 1) {
+      unsigned mine = 0;
+      for (; ks < 32 * (w + 1); ks += nsplit) mine |= 1u << (ks - 32 * w);
+      v &= mine;
+    }
     am[w] = v;
   }
   auto next_k = [&](int k) {
@@ -2119,10 +2122,6 @@ static int launch_m2l(const uint32_t *cls, const ClassArgs &ca, unsigned nchunks
     fprintf(stderr, "wbfmm (HIP): M2L plan for order %d does not match the kernel's bins\n", N);
     return WBFMM_HIP_ERR_ARG;
   }
-  // Few chunks leave most of the chip idle while each wavefront works
-  // through ~189 offsets in series: split the offsets over up to 8 blocks
-  // per chunk.  The split depends on the chunk count only, so a given
-  // problem always sums in the same order.
   constexpr int C = (N + 1) * (N + 1);
   unsigned ntot = 0;
   for (int c = 0; c < 8; c++) ntot += ca.count[c];
@@ -2210,7 +2209,7 @@ static int launch_m2l(const uint32_t *cls, const ClassArgs &ca, unsigned nchunks
       // orders 13..15 with the class-packed kernel switched off: chunked
     }
   }
-  const int nsplit = m2l_nsplit(nchunks);
+  const int nsplit = m2l_nsplit(level, nchunks, sizeof(T) * C);
   // class order; WBFMM_M2L_XCD=1 interleaves the 8 classes on each XCD at
   // unsplit levels
   ClassArgs cx = ca;

@@ -14,12 +14,6 @@
 
 namespace wbfmm {
 
-// blocks per chunk of the split M2L form: levels with fewer than 1024
-// chunks spread each chunk's offsets over up to 8 blocks (2048 in all)
-static inline int m2l_nsplit(unsigned nchunks) {
-  return nchunks >= 1024 ? 1 : (int)(2048 / nchunks < 8 ? 2048 / nchunks : 8);
-}
-
 #define WBFMM_LAP_RANGES(X) X(2, 7) X(8, 10) X(11, 12) X(13, 15) X(16, 18) X(19, 21) X(22, 24)
 
 #define WBFMM_LAP_RANGE_DECLARE(LO, HI)                                                      \

@@ -157,6 +157,7 @@ static int shift_entry(int mode, const uint32_t *parents, unsigned npar,
 constexpr size_t kScratchBytes = (size_t)64 << 20;
 constexpr size_t kScratchOcc = (size_t)16 << 10;
 constexpr size_t kScratchPart = kScratchOcc + ((size_t)2 << 20);
+static_assert(kScratchBytes - kScratchPart == kSplitBytes, "m2l_nsplit's bound");
 constexpr unsigned kScratchMaxLevel = 8;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 constexpr int kScratchDevices = 64;
@@ -224,9 +225,9 @@ static int m2l_entry(const uint32_t *cls, const unsigned *cstart, const unsigned
     }
     unsigned ntot = 0;
     for (int c = 0; c < 8; c++) ntot += ccount[c];
-    const int nsplit = m2l_nsplit(nch);
-    const size_t need =
-        nsplit > 1 ? sizeof(T) * (size_t)nsplit * ntot * (size_t)((N + 1) * (N + 1)) : 0;
+    const size_t one = sizeof(T) * (size_t)((N + 1) * (N + 1));
+    const int nsplit = m2l_nsplit((int)level, nch, one);
+    const size_t need = nsplit > 1 ? (size_t)nsplit * ntot * one : 0;
     if (need > kScratchBytes - kScratchPart) {
       snprintf(msg, sizeof(msg),
                "M2L without allocation: %u targets at order %d need %zu bytes of split "
