@@ -32,6 +32,7 @@
 // lane l supplies A[l%16][l/16] and B[l/16][l%16]; the result holds
 // D[l/16 + 4q][l%16], q = 0..3.
 
+#include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -107,6 +108,17 @@ __global__ void k_class_count(const uint32_t *list, unsigned n,
   if (threadIdx.x < 8 && h[threadIdx.x]) atomicAdd(&counts[threadIdx.x], h[threadIdx.x]);
 }
 
+
+// out[i] = unit[i] w^e[i mod period]: the coaxial tables of a box width from
+// those of width 1, with the powers -100..100 of w as an argument
+struct WidthPowers {
+  double v[201];
+};
+__global__ void k_coax_scale(const double *unit, const signed char *e, size_t n, size_t period,
+                             WidthPowers pw, double *out) {
+  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) out[i] = unit[i] * pw.v[e[i % period] + 100];
+}
 
 // the zero expansion (its bytes are zero for either precision, real or
 // complex coefficients)
@@ -311,6 +323,17 @@ int wbfmm_hip_lap_shift_mfma_f32(int mode, const uint32_t *parents, unsigned npa
                                  const wbfmm_m2l_plan_t *plan_host) {
   return shift_entry<float>(mode, parents, npar, cstart, cend, cflag, N, in, out, plan_dev,
                             A1, A3, A2, CS, plan_host);
+}
+
+int wbfmm_hip_lap_coax_scale(const double *unit, const signed char *e, size_t n, size_t period,
+                             double w, double *out) {
+  if (n == 0) return 0;
+  if (period == 0 || !(w > 0.0)) return WBFMM_HIP_ERR_ARG;
+  WidthPowers pw;
+  for (int k = -100; k <= 100; k++) pw.v[k + 100] = pow(w, (double)k);
+  WBFMM_LAUNCH("lap_coax_scale", k_coax_scale, dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
+               unit, e, n, period, pw, out);
+  return 0;
 }
 
 int wbfmm_hip_mfma_layout_probe(double *host_out) {

@@ -187,6 +187,10 @@ typedef struct {
   int m2l_A2_N[M2L_A2_CACHE], m2l_A2_kind[M2L_A2_CACHE];
   double m2l_A2_w[M2L_A2_CACHE];
   double *m2l_A2[M2L_A2_CACHE];
+  /* the same at width 1 (shared by the process) and the power of the width
+     in each entry, per kind and order */
+  double *lap_unit[3][WBFMM_HIP_MAX_ORDER + 1];
+  signed char *lap_pow[3][WBFMM_HIP_MAX_ORDER + 1];
   /* MFMA M2M / L2L rotation tiles and child-direction phases per order */
   double *sh_A1[WBFMM_HIP_MAX_ORDER + 1], *sh_A3[WBFMM_HIP_MAX_ORDER + 1];
   double *sh_CSup[WBFMM_HIP_MAX_ORDER + 1], *sh_CSdn[WBFMM_HIP_MAX_ORDER + 1];
@@ -1237,14 +1241,45 @@ static void copy_order_tables(ops_dev *od, int N)
 
 static void ensure_m2l_plan(ops_dev *od, int N) { ensure_order_tables(od, N); }
 
+/* the coaxial tables of order N and a kind at width 1, and their powers of
+   the width, in the shared set */
+static void ensure_lap_unit(const wbfmm_m2l_plan_t *P, int kind)
+{
+  const int N = P->N;
+  const size_t n2 = (size_t)P->KT * 64, n = (kind == 2 ? P->NR : 1) * n2;
+  double *h, *d = NULL;
+  signed char *e, *de = NULL;
+  mu_lock(&g_ord_mu[N]);
+  if (!g_tab.lap_unit[kind][N]) {
+    h = malloc(sizeof(double) * n);
+    e = malloc(n2);
+    if (!h || !e) WBFMM_FATAL("out of host memory");
+    if (kind == 2) HIPOK(wbfmm_hip_lap_m2l_coax(P, 1.0, h));
+    else HIPOK(wbfmm_hip_lap_shift_coax(P, kind, 1.0, h));
+    HIPOK(wbfmm_hip_lap_coax_powers(P, kind, e));
+    HIPOK(wbfmm_hip_malloc((void **)&d, sizeof(double) * n));
+    HIPOK(wbfmm_hip_malloc((void **)&de, n2));
+    HIPOK(wbfmm_hip_memcpy(d, h, sizeof(double) * n));
+    HIPOK(wbfmm_hip_memcpy(de, e, n2));
+    free(h);
+    free(e);
+    g_tab.lap_pow[kind][N] = de;
+    g_tab.lap_unit[kind][N] = d;
+  }
+  mu_unlock(&g_ord_mu[N]);
+}
+
 /* device coaxial tiles of the MFMA passes for order N: kind 2 S|R at the
    15 list-4 lengths for box width w (M2L), kind 0 S|S and kind 1 R|R at
-   distance w (M2M, L2L); a few entries are kept */
+   distance w (M2M, L2L), scaled on the device from those of width 1 (with
+   the powers taken on the host, every level of a new domain's first solve,
+   20 of the 46 ms of 200003 points at order 20; 0.03 now); a few entries
+   are kept */
 static const double *mfma_coax(ops_dev *od, int N, int kind, double w)
 {
   const wbfmm_m2l_plan_t *P = od->m2l_plan[N];
   size_t n = (size_t)(kind == 2 ? P->NR : 1) * P->KT * 64;
-  double *h;
+  double *t = NULL;
   int i;
   for (i = 0; i < od->m2l_nA2; i++)
     if (od->m2l_A2_N[i] == N && od->m2l_A2_kind[i] == kind && od->m2l_A2_w[i] == w)
@@ -1258,18 +1293,17 @@ static const double *mfma_coax(ops_dev *od, int N, int kind, double w)
     memmove(od->m2l_A2, od->m2l_A2 + 1, sizeof(double *) * (M2L_A2_CACHE - 1));
     od->m2l_nA2--;
   }
-  h = malloc(sizeof(double) * n);
-  if (!h) WBFMM_FATAL("out of host memory");
-  if (kind == 2) HIPOK(wbfmm_hip_lap_m2l_coax(P, w, h));
-  else HIPOK(wbfmm_hip_lap_shift_coax(P, kind, w, h));
+  ensure_lap_unit(P, kind);
+  HIPOK(wbfmm_hip_malloc((void **)&t, sizeof(double) * n));
+  HIPOK(wbfmm_hip_lap_coax_scale(g_tab.lap_unit[kind][N], g_tab.lap_pow[kind][N], n,
+                                 (size_t)P->KT * 64, w, t));
+  HIPOK(wbfmm_hip_sync()); /* the set may be used on another stream next */
   i = od->m2l_nA2++;
   od->m2l_A2_N[i] = N;
   od->m2l_A2_kind[i] = kind;
   od->m2l_A2_w[i] = w;
-  HIPOK(wbfmm_hip_malloc((void **)&od->m2l_A2[i], sizeof(double) * n));
-  HIPOK(wbfmm_hip_memcpy(od->m2l_A2[i], h, sizeof(double) * n));
-  free(h);
-  return od->m2l_A2[i];
+  od->m2l_A2[i] = t;
+  return t;
 }
 
 static const double *m2l_coax(ops_dev *od, int N, double w) { return mfma_coax(od, N, 2, w); }

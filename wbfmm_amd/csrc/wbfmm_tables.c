@@ -917,6 +917,37 @@ int wbfmm_hip_lap_shift_coax_unit(const wbfmm_m2l_plan_t *P, int kind, double *A
   return WBFMM_HIP_ERR_ARG;
 }
 
+int wbfmm_hip_lap_coax_powers(const wbfmm_m2l_plan_t *P, int kind, signed char *e)
+{
+  packing p2;
+  int N = P->N, S = 16 * P->NB, m, n, nu, part;
+  const size_t n2 = (size_t)P->KT * 64;
+  size_t i;
+  double *T, *h;
+  if (kind < 0 || kind > 2) return WBFMM_HIP_ERR_ARG;
+  do_pack(N, 1, &p2);
+  T = calloc((size_t)S * S, sizeof(double));
+  h = malloc(sizeof(double) * n2);
+  if (!T || !h) {
+    free(T);
+    free(h);
+    return WBFMM_HIP_ERR_NOMEM;
+  }
+  for (m = 0; m <= N; m++)
+    for (part = 0; part < (m ? 2 : 1); part++)
+      for (n = m; n <= N; n++)
+        for (nu = m; nu <= N; nu++) {
+          if ((kind == 0 && nu > n) || (kind == 1 && nu < n)) continue;
+          T[(size_t)slot2(&p2, N, n, m, part) * S + slot2(&p2, N, nu, m, part)] =
+              kind == 2 ? -(n + nu + 1) : kind == 0 ? n - nu : nu - n;
+        }
+  put_tiles(h, T, P);
+  for (i = 0; i < n2; i++) e[i] = (signed char)h[i];
+  free(T);
+  free(h);
+  return 0;
+}
+
 static int shift_coax(const wbfmm_m2l_plan_t *P, int kind, double t, double a, double b,
                       double *A2)
 {
