@@ -65,7 +65,8 @@ int wbfmm_hip_get_variant(int which);
 /* free and total device memory */
 int wbfmm_hip_mem_info(size_t *free_bytes, size_t *total_bytes);
 /* bytes of freed blocks that the library keeps for its next allocations (at
-   most 1 GiB), and their return to the runtime's pool */
+   most 1 GiB; given back by itself when an allocation finds no memory), and
+   their return to the runtime's pool */
 size_t wbfmm_hip_pool_bytes(void);
 int wbfmm_hip_pool_release(void);
 /* copy of any kind (host/device either side), ordered on the stream;
@@ -83,6 +84,9 @@ const char *wbfmm_hip_last_error(void);
 /* failure-handling tests: the calling thread's next n device allocations
    (wbfmm_hip_malloc and the library's own) return WBFMM_HIP_ERR_NOMEM */
 int wbfmm_hip_debug_fail_allocs(int n);
+/* the same one step further down: the next n calls that these allocations
+   make to the runtime's allocator are answered as out of memory */
+int wbfmm_hip_debug_fail_mallocs(int n);
 
 /* per-kernel timing with HIP events on the library stream:
    enable(1) starts recording every launch; query returns, for kernel

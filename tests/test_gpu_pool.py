@@ -62,12 +62,47 @@ def test_bounded(wb, lib):
     assert lib.wbfmm_hip_pool_release() == 0 and lib.wbfmm_hip_pool_bytes() == 0
 
 
+def runtime():
+    """the HIP runtime that the library has loaded"""
+    path = next(l.split()[-1] for l in open("/proc/self/maps") if "libamdhip64" in l)
+    return ctypes.CDLL(path)
+
+
+@pytest.mark.parametrize("mib", [2, 300])               # below and above the largest kept block
+@pytest.mark.parametrize("foreign", [False, True])      # on the library's stream, on a caller's
+def test_given_back_when_the_runtime_is_out_of_memory(wb, lib, mib, foreign):
+    """an allocation that the runtime refuses is tried again after the kept
+    blocks of every stream are given back, whatever its size and stream; with
+    nothing to give back it fails"""
+    hip = runtime()
+    own, s = _vp(), _vp()
+    assert lib.wbfmm_hip_stream_create(ctypes.byref(own)) == 0
+    for st in (None, own):
+        lib.wbfmm_hip_set_stream(st, None)
+        lib.wbfmm_hip_free(take(lib, 40 * MIB))
+    lib.wbfmm_hip_set_stream(None, None)
+    assert lib.wbfmm_hip_pool_bytes() == 80 * MIB
+    assert hip.hipStreamCreate(ctypes.byref(s)) == 0
+    lib.wbfmm_hip_set_stream(s if foreign else None, None)
+    lib.wbfmm_hip_debug_fail_mallocs(1)
+    a = take(lib, mib * MIB)
+    assert lib.wbfmm_hip_pool_bytes() == 0
+    lib.wbfmm_hip_debug_fail_mallocs(1)
+    p = _vp()
+    assert lib.wbfmm_hip_malloc(ctypes.byref(p), mib * MIB) != 0 and not p.value
+    lib.wbfmm_hip_debug_fail_mallocs(0)
+    assert lib.wbfmm_hip_malloc(ctypes.byref(p), mib * MIB) == 0
+    lib.wbfmm_hip_free(p)
+    lib.wbfmm_hip_free(a)
+    lib.wbfmm_hip_set_stream(None, None)
+    assert hip.hipStreamSynchronize(s) == 0 and hip.hipStreamDestroy(s) == 0
+    assert lib.wbfmm_hip_stream_destroy(own) == 0
+
+
 def test_foreign_stream(wb, lib):
     """a stream of the caller's: nothing kept, and a block of the library's
     stream freed there goes back to the runtime"""
-    # the HIP runtime that the library has loaded
-    path = next(l.split()[-1] for l in open("/proc/self/maps") if "libamdhip64" in l)
-    hip = ctypes.CDLL(path)
+    hip = runtime()
     s = _vp()
     assert hip.hipStreamCreate(ctypes.byref(s)) == 0
     a = take(lib, MIB)

@@ -146,6 +146,7 @@ _SIGS = {
     "wbfmm_hip_free": (_i, [_vp]),
     "wbfmm_hip_pool_bytes": (_sz, []),
     "wbfmm_hip_pool_release": (_i, []),
+    "wbfmm_hip_debug_fail_mallocs": (_i, [_i]),
     "wbfmm_hip_memcpy": (_i, [_vp, _vp, _sz]),
     "wbfmm_hip_memset": (_i, [_vp, _i, _sz]),
     "wbfmm_hip_stage4": (_i, [_vp, _sz, _u, _vp]),

@@ -448,8 +448,9 @@ static inline unsigned nblk(size_t n, unsigned b) {
 }
 
 
-// allocations of this thread still to be refused (failure-handling tests)
-static thread_local int t_fail_allocs = 0;
+// allocations of this thread still to be refused, and calls of the runtime's
+// allocator still to be answered as out of memory (failure-handling tests)
+static thread_local int t_fail_allocs = 0, t_fail_mallocs = 0;
 
 // Freed blocks kept for the next allocation on the same stream.  hipMallocAsync
 // and hipFreeAsync take 10 to 70 us of host time each (the free of a block
@@ -462,7 +463,9 @@ static thread_local int t_fail_allocs = 0;
 // blocks belong to the graph, take the runtime's allocator.  At most 1 GiB is
 // kept, in blocks up to 256 MiB (a level array of a large tree is worth a
 // call), the longest unused given back first; a stream's blocks are given
-// back before it is destroyed, and every stream's when an allocation fails.
+// back before it is destroyed, and every stream's when the runtime has no
+// memory for an allocation, of any size and on any stream that is not under
+// capture (pool_give_back), which is then tried once more.
 constexpr size_t kPoolBytes = (size_t)1 << 30, kPoolBlock = (size_t)256 << 20;
 struct PoolBlock {
   void *p;
@@ -489,12 +492,15 @@ static bool pool_note(void *p, size_t b) {
   }
 }
 
+static bool capturing(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
+}
+
 // s is the library's own and not under capture (g_pool_mu held)
 static bool pool_serves(hipStream_t s) {
-  if (std::find(g_pool_streams.begin(), g_pool_streams.end(), s) == g_pool_streams.end())
-    return false;
-  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-  return hipStreamIsCapturing(s, &st) == hipSuccess && st == hipStreamCaptureStatusNone;
+  return std::find(g_pool_streams.begin(), g_pool_streams.end(), s) != g_pool_streams.end() &&
+         !capturing(s);
 }
 
 static void pool_add_stream(hipStream_t s) {
@@ -518,6 +524,37 @@ static void pool_flush(hipStream_t s) {
   std::lock_guard<std::mutex> lk(g_pool_mu);
   for (size_t i = g_pool_free.size(); i-- > 0;)
     if (!s || g_pool_free[i].s == s) pool_release(i);
+}
+
+// give every free block back, wait until its stream is done with it, and
+// let the runtime return what it holds unused to the device: the memory may
+// be wanted on another stream or in a larger piece.  False when none was
+// kept.  The lock is held throughout, so that no stream of a block ends here.
+static bool pool_give_back() {
+  std::lock_guard<std::mutex> lk(g_pool_mu);
+  std::vector<hipStream_t> used;
+  try {
+    for (const PoolBlock &b : g_pool_free)
+      if (std::find(used.begin(), used.end(), b.s) == used.end()) used.push_back(b.s);
+  } catch (...) {  // no host memory either
+    return false;
+  }
+  if (used.empty()) return false;
+  while (!g_pool_free.empty()) pool_release(g_pool_free.size() - 1);
+  for (hipStream_t s : used) (void)hipStreamSynchronize(s);
+  int dev = 0;
+  hipMemPool_t pool;
+  if (hipGetDevice(&dev) == hipSuccess && hipDeviceGetDefaultMemPool(&pool, dev) == hipSuccess)
+    (void)hipMemPoolTrimTo(pool, 0);
+  return true;
+}
+
+static hipError_t runtime_malloc(void **p, size_t bytes, hipStream_t s) {
+  if (t_fail_mallocs > 0) {
+    t_fail_mallocs--;
+    return hipErrorOutOfMemory;
+  }
+  return hipMallocAsync(p, bytes, s);
 }
 
 int dmalloc(void **p, size_t bytes) {
@@ -549,12 +586,10 @@ int dmalloc(void **p, size_t bytes) {
       return 0;
     }
   }
-  hipError_t e = hipMallocAsync(p, bytes, s);
-  if (e != hipSuccess && pooled) {
+  hipError_t e = runtime_malloc(p, bytes, s);
+  if (e != hipSuccess && !capturing(s)) {
     (void)hipGetLastError();
-    pool_flush(nullptr);
-    (void)hipStreamSynchronize(s);
-    e = hipMallocAsync(p, bytes, s);
+    if (pool_give_back()) e = runtime_malloc(p, bytes, s);
   }
   if (e != hipSuccess) {
     *p = nullptr;
@@ -689,6 +724,11 @@ const char *wbfmm_hip_last_error(void) { return g_err; }
 
 int wbfmm_hip_debug_fail_allocs(int n) {
   t_fail_allocs = n > 0 ? n : 0;
+  return 0;
+}
+
+int wbfmm_hip_debug_fail_mallocs(int n) {
+  t_fail_mallocs = n > 0 ? n : 0;
   return 0;
 }
 
