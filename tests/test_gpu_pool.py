@@ -99,6 +99,32 @@ def test_given_back_when_the_runtime_is_out_of_memory(wb, lib, mib, foreign):
     assert lib.wbfmm_hip_stream_destroy(own) == 0
 
 
+def test_blocks_of_a_capturing_stream_stay(wb, lib):
+    """while a stream is captured its kept blocks are neither released nor
+    evicted: the graph has no node for them, and they are released afterwards"""
+    hip = runtime()
+    s, g, nodes = _vp(), _vp(), ctypes.c_size_t(99)
+    assert lib.wbfmm_hip_stream_create(ctypes.byref(s)) == 0
+    lib.wbfmm_hip_set_stream(s, None)
+    lib.wbfmm_hip_free(take(lib, 100 * MIB))
+    lib.wbfmm_hip_set_stream(None, None)
+    ps = [take(lib, 200 * MIB) for _ in range(5)]
+    assert hip.hipStreamBeginCapture(s, 2) == 0            # relaxed mode
+    assert lib.wbfmm_hip_pool_release() == 0 and lib.wbfmm_hip_pool_bytes() == 100 * MIB
+    for p in ps:                                           # 1000 MiB more: 80 over the bound
+        lib.wbfmm_hip_free(p)
+    assert lib.wbfmm_hip_pool_bytes() == 900 * MIB         # the oldest that may go went
+    lib.wbfmm_hip_debug_fail_mallocs(1)
+    p = take(lib, MIB)                                     # tried again with what is released
+    assert lib.wbfmm_hip_pool_bytes() == 100 * MIB
+    assert hip.hipStreamEndCapture(s, ctypes.byref(g)) == 0
+    assert hip.hipGraphGetNodes(g, None, ctypes.byref(nodes)) == 0 and nodes.value == 0
+    assert hip.hipGraphDestroy(g) == 0
+    lib.wbfmm_hip_free(p)
+    assert lib.wbfmm_hip_stream_destroy(s) == 0
+    assert lib.wbfmm_hip_pool_bytes() == MIB
+
+
 def test_foreign_stream(wb, lib):
     """a stream of the caller's: nothing kept, and a block of the library's
     stream freed there goes back to the runtime"""

@@ -465,7 +465,8 @@ static thread_local int t_fail_allocs = 0, t_fail_mallocs = 0;
 // call), the longest unused given back first; a stream's blocks are given
 // back before it is destroyed, and every stream's when the runtime has no
 // memory for an allocation, of any size and on any stream that is not under
-// capture (pool_give_back), which is then tried once more.
+// capture (pool_give_back), which is then tried once more.  Blocks of a stream
+// that is being captured stay until the capture has ended.
 constexpr size_t kPoolBytes = (size_t)1 << 30, kPoolBlock = (size_t)256 << 20;
 struct PoolBlock {
   void *p;
@@ -511,36 +512,64 @@ static void pool_add_stream(hipStream_t s) {
   }
 }
 
-// give free block i back to the runtime (g_pool_mu held)
-static void pool_release(size_t i) {
-  (void)hipFreeAsync(g_pool_free[i].p, g_pool_free[i].s);
-  g_pool_bytes -= g_pool_free[i].bytes;
-  g_pool_free[i] = g_pool_free.back();
+// give free block i back to the runtime (g_pool_mu held); false, and the block
+// stays, while its stream is under capture (the free would be refused or
+// become part of that graph)
+static bool pool_release(size_t i) {
+  PoolBlock &b = g_pool_free[i];
+  if (capturing(b.s)) return false;
+  if (hipFreeAsync(b.p, b.s) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  g_pool_bytes -= b.bytes;
+  b = g_pool_free.back();
   g_pool_free.pop_back();
+  return true;
 }
 
-// give back every free block of stream s, or of all streams (null)
+// give back the free blocks of stream s, or of all streams (null)
 static void pool_flush(hipStream_t s) {
   std::lock_guard<std::mutex> lk(g_pool_mu);
   for (size_t i = g_pool_free.size(); i-- > 0;)
-    if (!s || g_pool_free[i].s == s) pool_release(i);
+    if (!s || g_pool_free[i].s == s) (void)pool_release(i);
+}
+
+// release free blocks, the longest unused first, until `bytes' more may be
+// kept (g_pool_mu held); false when those that are left cannot be released
+static bool pool_make_room(size_t bytes) {
+  uint64_t from = 0;  // stamps below are of blocks that stayed
+  while (g_pool_bytes + bytes > kPoolBytes) {
+    size_t old = g_pool_free.size();
+    for (size_t i = 0; i < g_pool_free.size(); i++)
+      if (g_pool_free[i].stamp >= from &&
+          (old == g_pool_free.size() || g_pool_free[i].stamp < g_pool_free[old].stamp))
+        old = i;
+    if (old == g_pool_free.size()) return false;
+    from = g_pool_free[old].stamp + 1;
+    (void)pool_release(old);
+  }
+  return true;
 }
 
 // give every free block back, wait until its stream is done with it, and
 // let the runtime return what it holds unused to the device: the memory may
 // be wanted on another stream or in a larger piece.  False when none was
-// kept.  The lock is held throughout, so that no stream of a block ends here.
+// released.  The lock is held throughout, so that no stream of a block ends
+// here.
 static bool pool_give_back() {
   std::lock_guard<std::mutex> lk(g_pool_mu);
   std::vector<hipStream_t> used;
   try {
-    for (const PoolBlock &b : g_pool_free)
-      if (std::find(used.begin(), used.end(), b.s) == used.end()) used.push_back(b.s);
+    used.reserve(g_pool_free.size());
   } catch (...) {  // no host memory either
     return false;
   }
+  for (size_t i = g_pool_free.size(); i-- > 0;) {
+    const hipStream_t s = g_pool_free[i].s;
+    if (pool_release(i) && std::find(used.begin(), used.end(), s) == used.end()) used.push_back(s);
+  }
   if (used.empty()) return false;
-  while (!g_pool_free.empty()) pool_release(g_pool_free.size() - 1);
   for (hipStream_t s : used) (void)hipStreamSynchronize(s);
   int dev = 0;
   hipMemPool_t pool;
@@ -611,13 +640,7 @@ static hipError_t free_block(void *p) {
     if (it != g_pool_live.end()) {
       const size_t bytes = it->second;
       g_pool_live.erase(it);
-      if (pool_serves(s)) {
-        while (g_pool_bytes + bytes > kPoolBytes && !g_pool_free.empty()) {
-          size_t old = 0;
-          for (size_t i = 1; i < g_pool_free.size(); i++)
-            if (g_pool_free[i].stamp < g_pool_free[old].stamp) old = i;
-          pool_release(old);
-        }
+      if (pool_serves(s) && pool_make_room(bytes)) {
         try {
           g_pool_free.push_back(PoolBlock{p, bytes, s, g_pool_stamp++});
           g_pool_bytes += bytes;
