@@ -142,6 +142,37 @@ def test_foreign_stream(wb, lib):
     assert hip.hipStreamSynchronize(s) == 0 and hip.hipStreamDestroy(s) == 0
 
 
+@pytest.mark.parametrize("foreign", [False, True])
+def test_address_that_comes_back_with_another_size(wb, lib, foreign):
+    """a block that its holder gave to hipFree: a later, smaller one at the
+    same address is kept with its own size, or, allocated on a caller's
+    stream, not at all"""
+    hip = runtime()
+    s, pool = _vp(), _vp()
+    assert hip.hipStreamCreate(ctypes.byref(s)) == 0
+    assert hip.hipDeviceGetDefaultMemPool(ctypes.byref(pool), 0) == 0
+    hip.hipMemPoolTrimTo(pool, ctypes.c_size_t(0))
+    a = take(lib, 2 * MIB)
+    wb.sync()
+    assert hip.hipFree(_vp(a)) == 0
+    hip.hipMemPoolTrimTo(pool, ctypes.c_size_t(0))
+    lib.wbfmm_hip_set_stream(s if foreign else None, None)
+    ps = [take(lib, MIB) for _ in range(8)]
+    lib.wbfmm_hip_set_stream(None, None)
+    assert hip.hipStreamSynchronize(s) == 0
+    back = a in ps
+    if back:
+        lib.wbfmm_hip_free(a)
+        assert lib.wbfmm_hip_pool_bytes() == (0 if foreign else MIB)
+    for p in ps:
+        if p != a:
+            lib.wbfmm_hip_free(p)
+    wb.sync()
+    assert hip.hipStreamDestroy(s) == 0
+    if not back:
+        pytest.skip("the runtime gave the address to no later block")
+
+
 def test_contents_in_stream_order(wb, lib):
     """a block handed out again while its last use is still queued"""
     n = 8 * MIB // 8
@@ -150,10 +181,14 @@ def test_contents_in_stream_order(wb, lib):
         a = wb.DeviceBuffer.from_array(want + rep)
         c = wb.DeviceBuffer(8 * n)
         assert lib.wbfmm_hip_memcpy(c.ptr, a.ptr, 8 * n) == 0   # device copy, queued
+        was = a.ptr
         a.free()
-        b = wb.DeviceBuffer(8 * n)                              # the same block
+        b = wb.DeviceBuffer(8 * n)
+        assert b.ptr == was                                     # the same block
         b.zero()
         assert np.array_equal(c.download(np.zeros(n)), want + rep)
         assert not b.download(np.ones(n)).any()
         b.free()
         c.free()
+        wb.sync()
+        lib.wbfmm_hip_pool_release()    # the next freed block is the only one kept

@@ -483,10 +483,11 @@ static size_t g_pool_bytes = 0;  // of g_pool_free
 static uint64_t g_pool_stamp = 0;
 
 // b becomes the size of block p, handed out; false when the host has no
-// memory for the entry
+// memory for the entry.  An entry may be there: of a block that its holder
+// gave to hipFree, whose address has come back with another size.
 static bool pool_note(void *p, size_t b) {
   try {
-    g_pool_live.emplace(p, b);
+    g_pool_live[p] = b;
     return true;
   } catch (...) {
     return false;
@@ -625,9 +626,9 @@ int dmalloc(void **p, size_t bytes) {
     fail("hipMallocAsync", e);
     return WBFMM_HIP_ERR_NOMEM;
   }
-  if (pooled) {
+  {
     std::lock_guard<std::mutex> lk(g_pool_mu);
-    (void)pool_note(*p, bytes);
+    if (!pooled || !pool_note(*p, bytes)) g_pool_live.erase(*p);
   }
   return 0;
 }
