@@ -1131,19 +1131,45 @@ __global__ void k_d2f(const double *in, float *out, size_t n) {
 using namespace wbfmm;
 
 // the factors' table, built by the first call that needs it (finished
-// before it is published: other streams read it then)
+// before it is published: other streams read it then).  While the calling
+// stream is captured the table is built on a stream of its own, in the
+// capture mode that allows it: the field entries allocate and wait for
+// nothing, and can be captured from a process's first call on.
 static LapTab *g_laptab = nullptr;
 static std::mutex g_laptab_mu;
+
+static int build_lap_tab(hipStream_t s) {
+  LapTab *t = nullptr;
+  WBFMM_CHECK(hipMalloc((void **)&t, sizeof(LapTab)));
+  hipLaunchKernelGGL(k_lap_tab, dim3(nblk(kLapTabN * (2 * kLapTabN + 1), 256)), dim3(256), 0, s, t);
+  hipError_t e = hipGetLastError();
+  if (e == hipSuccess) e = hipStreamSynchronize(s);
+  if (e != hipSuccess) {
+    (void)hipFree(t);
+    return fail("factor table", e);
+  }
+  g_laptab = t;
+  return 0;
+}
 
 static int lap_tab(const LapTab **out) {
   std::lock_guard<std::mutex> lk(g_laptab_mu);
   if (!g_laptab) {
-    LapTab *t = nullptr;
-    WBFMM_CHECK(hipMalloc((void **)&t, sizeof(LapTab)));
-    WBFMM_LAUNCH("lap_tab", k_lap_tab, dim3(nblk(kLapTabN * (2 * kLapTabN + 1), 256)),
-                 dim3(256), 0, t);
-    WBFMM_CHECK(hipStreamSynchronize(stream()));
-    g_laptab = t;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    WBFMM_CHECK(hipStreamIsCapturing(stream(), &st));
+    int rc;
+    if (st == hipStreamCaptureStatusNone) {
+      rc = build_lap_tab(stream());
+    } else {
+      hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+      WBFMM_CHECK(hipThreadExchangeStreamCaptureMode(&mode));
+      hipStream_t side = nullptr;
+      hipError_t e = hipStreamCreateWithFlags(&side, hipStreamNonBlocking);
+      rc = e == hipSuccess ? build_lap_tab(side) : fail("hipStreamCreateWithFlags", e);
+      if (side) (void)hipStreamDestroy(side);
+      (void)hipThreadExchangeStreamCaptureMode(&mode);
+    }
+    if (rc) return rc;
   }
   *out = g_laptab;
   return 0;
