@@ -200,6 +200,12 @@ gint wbfmm_points_origin_width(gdouble *x, gint str, gint n, gdouble *xmin,
                                gboolean init_limits);
 /* src/wbfmm.h:1134: zeroes mps and mpr at one level (device memset) */
 gint wbfmm_tree_coefficients_zero(wbfmm_tree_t *t, guint level);
+/* (addition) on: the caller promises to write the arrays t->mps and t->mpr
+   by passes only (no stores of its own through the members or the boxes'
+   pointers), and coefficient_init and leaf_expansions with zero_expansions
+   then clear the boxes that passes wrote and not the whole arrays.  Off, as
+   in a new tree, they clear the whole arrays, whatever wrote them. */
+gint wbfmm_tree_levels_private(wbfmm_tree_t *t, gboolean on);
 /* src/wbfmm.h:844-845 */
 gint wbfmm_truncation_number(wbfmm_tree_t *t, gdouble k, guint level,
                              gdouble tol);

@@ -62,6 +62,55 @@ def test_reused_tree(wb, kind):
     used.close()
 
 
+@pytest.mark.parametrize("kind", ["laplace", "fp32", "helmholtz", "mixed"])
+def test_levels_that_the_caller_wrote(wb, kind):
+    """t->mps and t->mpr are public: what a caller stored there is cleared by
+    coefficient_init, and by leaf_expansions with zero_expansions, whether the
+    library last left the array zeroed or written by its passes"""
+    rng = np.random.default_rng(4)
+    n, depth, p, k = 500, 3, 5, 2.0
+    helm = kind in ("helmholtz", "mixed")
+    orders = [0, p] + [p] * (depth - 1)
+    x0, D = np.array([-1.1, -1.1, -1.1]), 2.2
+    xs, q = sphere(rng, n, 0), rng.normal(size=(n, 2 if helm else 1))
+    make = wb.HelmholtzSolver if helm else wb.LaplaceSolver
+    args = (xs, x0, D, depth, orders, orders) + ((k,) if helm else ())
+    s = make(*args, targets=xs, precision=32 if kind in ("fp32", "mixed") else 64,
+             **({} if helm else {"host_mirror": False}))
+    L = wb.lib()
+
+    def levels():
+        return [s.coefficients(l, w) for l in range(2, depth + 1) for w in (0, 1)]
+
+    def scribble(which):
+        """every coefficient of the levels something else, as a caller does"""
+        es = 4 if kind in ("fp32", "mixed") else 8
+        for l in range(2, depth + 1):
+            a = (s.tree.contents.mps, s.tree.contents.mpr)[which][l]
+            nbytes = 8 ** l * (p + 1) ** 2 * es * (2 if helm else 1)
+            assert L.wbfmm_hip_memset(a, 0x3f, nbytes) == 0
+
+    s.build_tree()
+    s.passes(q)
+    want = levels()
+    for after_passes in (False, True):
+        for which in (0, 1):
+            s.build_tree()
+            if after_passes:
+                s.passes(q)
+            scribble(which)
+            s.build_tree()
+            assert all(not a.any() for a in levels())
+            s.passes(q)
+            assert all(np.array_equal(a, b) for a, b in zip(levels(), want))
+    # the leaf level alone, by zero_expansions
+    s.build_tree()
+    L.wbfmm_hip_memset(s.tree.contents.mps[depth], 0x3f, 8 ** depth * (p + 1) ** 2 * 4)
+    s.passes(q)
+    assert all(np.array_equal(a, b) for a, b in zip(levels(), want))
+    s.close()
+
+
 @pytest.mark.parametrize("row", [4, 36, 1352, 4608])
 @pytest.mark.parametrize("n", [0, 1, 5, 63])
 def test_clear_rows(wb, row, n):

@@ -128,6 +128,7 @@ _SIGS = {
     "wbfmm_tree_free": (_i, [_vp]),
     "wbfmm_tree_coefficients_download": (_i, [_vp, _u, _i, _vp]),
     "wbfmm_tree_coefficients_zero": (_i, [_vp, _u]),
+    "wbfmm_tree_levels_private": (_i, [_vp, _i]),
     "wbfmm_point_box": (ctypes.c_uint64, [_vp, _u, _vp]),
     "wbfmm_box_interaction_list_4": (_i, [_u, ctypes.c_uint64, _vp, _i]),
     "wbfmm_box_neighbours": (_i, [_u, ctypes.c_uint64, _vp]),
@@ -271,7 +272,29 @@ class Timing:
         return n.value, ms.value
 
 
-class LaplaceSolver:
+class _OwnTree:
+    """The tree of a solver.  Its level arrays are the solver's alone
+    (wbfmm_tree_levels_private) until the tree is asked for: who holds it may
+    write them, and from then on they are cleared whole."""
+
+    @property
+    def tree(self):
+        """the wbfmm_tree_t, as a ctypes pointer"""
+        self._shared()
+        return self._tree
+
+    @property
+    def t(self):
+        """the tree's address, for calls of the library (None once closed)"""
+        self._shared()
+        return self._t
+
+    def _shared(self):
+        if self._t:
+            lib().wbfmm_tree_levels_private(self._t, 0)
+
+
+class LaplaceSolver(_OwnTree):
     """Laplace FMM through the drop-in API, in the reference driver's call
     order (tools/wbfmm-laplace-tree-calc.c.in:380-460).
 
@@ -293,13 +316,14 @@ class LaplaceSolver:
         x0 = np.ascontiguousarray(x0, dtype=np.float64)
         self._x0 = x0
         self.xs = xs
-        self.tree = L.wbfmm_tree_new(ptr(x0), float(D), self.nsrc)
-        if not self.tree:
+        self._tree = L.wbfmm_tree_new(ptr(x0), float(D), self.nsrc)
+        if not self._tree:
             raise RuntimeError("wbfmm_tree_new failed")
-        self.t = ctypes.cast(self.tree, _vp).value
-        L.wbfmm_tree_host_mirror(self.t, 1 if host_mirror else 0)
+        self._t = ctypes.cast(self._tree, _vp).value
+        L.wbfmm_tree_levels_private(self._t, 1)
+        L.wbfmm_tree_host_mirror(self._t, 1 if host_mirror else 0)
         if precision != 64:
-            L.wbfmm_tree_set_precision(self.t, precision)
+            L.wbfmm_tree_set_precision(self._t, precision)
         lmax = max(max(order_s[2:depth + 1]), max(order_r[2:depth + 1]))
         L.wbfmm_shift_angle_table_init()
         self.op = L.wbfmm_shift_operators_new(lmax, 0, None)
@@ -317,17 +341,17 @@ class LaplaceSolver:
     def build_tree(self):
         """add_points + refine x depth + coefficient init (+ target list)."""
         L = lib()
-        L.wbfmm_tree_add_points(self.t, ptr(self.xs), self.pstr, ptr(self.normals),
+        L.wbfmm_tree_add_points(self._t, ptr(self.xs), self.pstr, ptr(self.normals),
                                 self.nstr if self.normals is not None else 0, self.nsrc, 0)
         for _ in range(self.depth):
-            L.wbfmm_tree_refine(self.t)
-        self.tree.contents.problem = WBFMM_PROBLEM_LAPLACE
-        self.tree.contents.nq = self.nq
+            L.wbfmm_tree_refine(self._t)
+        self._tree.contents.problem = WBFMM_PROBLEM_LAPLACE
+        self._tree.contents.nq = self.nq
         for l in range(1, self.depth + 1):
-            L.wbfmm_tree_laplace_coefficient_init(self.t, l, self.order_r[l], self.order_s[l])
+            L.wbfmm_tree_laplace_coefficient_init(self._t, l, self.order_r[l], self.order_s[l])
         if self.targets is not None:
             if self.tl is None:
-                self.tl = L.wbfmm_target_list_new(self.t, self.ntgt)
+                self.tl = L.wbfmm_target_list_new(self._t, self.ntgt)
             L.wbfmm_target_list_add_points(self.tl, ptr(self.targets), self.tstr, self.ntgt)
         self._fresh = True   # coefficient_init leaves every level zeroed
 
@@ -337,13 +361,13 @@ class LaplaceSolver:
         L = lib()
         if not getattr(self, "_fresh", False):
             for l in range(1, self.depth + 1):
-                L.wbfmm_tree_coefficients_zero(self.t, l)
+                L.wbfmm_tree_coefficients_zero(self._t, l)
         self._fresh = False
-        L.wbfmm_tree_laplace_leaf_expansions(self.t, ptr(q), sstr, ptr(d), dstr, 1, None)
+        L.wbfmm_tree_laplace_leaf_expansions(self._t, ptr(q), sstr, ptr(d), dstr, 1, None)
         for l in range(self.depth, 2, -1):
-            L.wbfmm_laplace_upward_pass(self.t, self.op, l, None)
+            L.wbfmm_laplace_upward_pass(self._t, self.op, l, None)
         for l in range(2, self.depth + 1):
-            L.wbfmm_laplace_downward_pass_ref(self.t, self.op, l, None, 0)
+            L.wbfmm_laplace_downward_pass_ref(self._t, self.op, l, None, 0)
 
     def field(self, q, f, field=3, fstr=4, sstr=1, d=None, dstr=1):
         """target-list field (L2P + near field) into f (accumulated)."""
@@ -358,7 +382,7 @@ class LaplaceSolver:
         components, field 1/2/3 gives the potentials and gradients of every
         component, 4 the curl, 6 the curl and its gradient"""
         n = len(xt) if ntgt is None else ntgt
-        rc = lib().wbfmm_laplace_field_targets(self.t, ptr(xt), tstr, n, ptr(q), sstr, ptr(d),
+        rc = lib().wbfmm_laplace_field_targets(self._t, ptr(xt), tstr, n, ptr(q), sstr, ptr(d),
                                                dstr, field, ptr(f), fstr)
         if rc != 0:
             raise RuntimeError(f"wbfmm_laplace_field_targets = {rc}")
@@ -375,7 +399,7 @@ class LaplaceSolver:
         nb = 8 ** level
         nq = self.nq
         buf = np.zeros(nb * C * nq)
-        rc = lib().wbfmm_tree_coefficients_download(self.t, level, which, ptr(buf))
+        rc = lib().wbfmm_tree_coefficients_download(self._t, level, which, ptr(buf))
         if rc != 0:
             raise RuntimeError("download failed")
         # [group of 8][coef][child][component] -> [box][coef] ([component][box][coef])
@@ -387,15 +411,15 @@ class LaplaceSolver:
         if self.tl:
             L.wbfmm_target_list_free(self.tl)
             self.tl = None
-        if self.t:
-            L.wbfmm_tree_free(self.t)
-            self.t = None
+        if self._t:
+            L.wbfmm_tree_free(self._t)
+            self._t = None
         if self.op:
             L.wbfmm_shift_operators_free(self.op)
             self.op = None
 
 
-class HelmholtzSolver:
+class HelmholtzSolver(_OwnTree):
     """Helmholtz FMM through the drop-in API, in the reference driver's
     call order (tools/wbfmm-tree-calc.c.in:306-417): shift operators,
     S|R tables for levels 2..depth and S|S tables for levels 3..depth,
@@ -420,13 +444,14 @@ class HelmholtzSolver:
         self.nstr = nstr
         self.order_s = list(order_s)
         self.order_r = list(order_r)
-        self.tree = L.wbfmm_tree_new(ptr(self._x0), float(D), self.nsrc)
-        if not self.tree:
+        self._tree = L.wbfmm_tree_new(ptr(self._x0), float(D), self.nsrc)
+        if not self._tree:
             raise RuntimeError("wbfmm_tree_new failed")
-        self.t = ctypes.cast(self.tree, _vp).value
-        L.wbfmm_tree_host_mirror(self.t, 0)
+        self._t = ctypes.cast(self._tree, _vp).value
+        L.wbfmm_tree_levels_private(self._t, 1)
+        L.wbfmm_tree_host_mirror(self._t, 0)
         if precision != 64:
-            L.wbfmm_tree_set_precision(self.t, precision)
+            L.wbfmm_tree_set_precision(self._t, precision)
         lmax = max(max(order_s[2:depth + 1]), max(order_r[2:depth + 1]))
         L.wbfmm_shift_angle_table_init()
         self.op = L.wbfmm_shift_operators_new(lmax, 0, None)
@@ -441,19 +466,19 @@ class HelmholtzSolver:
 
     def build_tree(self):
         L = lib()
-        L.wbfmm_tree_add_points(self.t, ptr(self.xs), self.pstr, ptr(self.normals),
+        L.wbfmm_tree_add_points(self._t, ptr(self.xs), self.pstr, ptr(self.normals),
                                 self.nstr if self.normals is not None else 0, self.nsrc, 0)
         for _ in range(self.depth):
-            L.wbfmm_tree_refine(self.t)
-        self.tree.contents.problem = WBFMM_PROBLEM_HELMHOLTZ
-        self.tree.contents.nq = 1
+            L.wbfmm_tree_refine(self._t)
+        self._tree.contents.problem = WBFMM_PROBLEM_HELMHOLTZ
+        self._tree.contents.nq = 1
         for l in range(1, self.depth + 1):
-            L.wbfmm_tree_coefficient_init(self.t, l, self.order_r[l], self.order_s[l])
+            L.wbfmm_tree_coefficient_init(self._t, l, self.order_r[l], self.order_s[l])
         if self.targets is not None:
             # registered targets restrict the downward pass to boxes holding
             # sources or targets
             if self.tl is None:
-                self.tl = L.wbfmm_target_list_new(self.t, self.ntgt)
+                self.tl = L.wbfmm_target_list_new(self._t, self.ntgt)
             L.wbfmm_target_list_add_points(self.tl, ptr(self.targets), self.tstr, self.ntgt)
         self._fresh = True   # coefficient_init leaves every level zeroed
 
@@ -461,17 +486,17 @@ class HelmholtzSolver:
         L = lib()
         if not getattr(self, "_fresh", False):
             for l in range(1, self.depth + 1):
-                L.wbfmm_tree_coefficients_zero(self.t, l)
+                L.wbfmm_tree_coefficients_zero(self._t, l)
         self._fresh = False
-        L.wbfmm_tree_leaf_expansions(self.t, self.k, ptr(q), sstr, ptr(d), dstr, 1, None)
+        L.wbfmm_tree_leaf_expansions(self._t, self.k, ptr(q), sstr, ptr(d), dstr, 1, None)
         for l in range(self.depth, 2, -1):
-            L.wbfmm_upward_pass(self.t, self.op, l, None)
+            L.wbfmm_upward_pass(self._t, self.op, l, None)
         for l in range(2, self.depth + 1):
-            L.wbfmm_downward_pass_ref(self.t, self.op, l, None, 0)
+            L.wbfmm_downward_pass_ref(self._t, self.op, l, None, 0)
 
     def field(self, xt, q, f, field=3, fstr=8, tstr=24, ntgt=None, sstr=2, d=None, dstr=2):
         n = len(xt) if ntgt is None else ntgt
-        rc = lib().wbfmm_helmholtz_field_targets(self.t, self.k, ptr(xt), tstr, n, ptr(q), sstr,
+        rc = lib().wbfmm_helmholtz_field_targets(self._t, self.k, ptr(xt), tstr, n, ptr(q), sstr,
                                                  ptr(d), dstr, field, ptr(f), fstr)
         if rc != 0:
             raise RuntimeError(f"wbfmm_helmholtz_field_targets = {rc}")
@@ -482,7 +507,7 @@ class HelmholtzSolver:
         C = (N + 1) ** 2
         nb = 8 ** level
         buf = np.zeros(nb * C * 2)
-        if lib().wbfmm_tree_coefficients_download(self.t, level, which, ptr(buf)) != 0:
+        if lib().wbfmm_tree_coefficients_download(self._t, level, which, ptr(buf)) != 0:
             raise RuntimeError("download failed")
         # [group of 8][coef][child][re, im] -> [box][coef]
         z = buf[0::2] + 1j * buf[1::2]
@@ -493,9 +518,9 @@ class HelmholtzSolver:
         if self.tl:
             L.wbfmm_target_list_free(self.tl)
             self.tl = None
-        if self.t:
-            L.wbfmm_tree_free(self.t)
-            self.t = None
+        if self._t:
+            L.wbfmm_tree_free(self._t)
+            self._t = None
         if self.op:
             L.wbfmm_shift_operators_free(self.op)
             self.op = None

@@ -548,8 +548,10 @@ int solve_body(void *arg) {
   double x0[3] = {p.x0[0], p.x0[1], p.x0[2]};
   S.t = wbfmm_tree_new(x0, p.D, r.nsrc);
   wbfmm_tree_t *t = S.t;
-  // the engine's trees are private: no host box arrays (8^l entries per
-  // level), which FP32 coefficients do not allow anyway
+  // the engine's trees are its own: their levels are written by passes only,
+  // and have no host box arrays (8^l entries per level), which FP32
+  // coefficients do not allow anyway
+  wbfmm_tree_levels_private(t, TRUE);
   wbfmm_tree_host_mirror(t, FALSE);
   if (p.precision == 32) wbfmm_tree_set_precision(t, 32);
   wbfmm_tree_add_points(t, (gpointer)r.xs, r.pstr, (gpointer)r.normals,

@@ -142,6 +142,7 @@ typedef struct {
      (LEVEL_*) */
   size_t box_bytes[2][WBFMM_TREE_MAX_DEPTH + 1];
   unsigned char held[2][WBFMM_TREE_MAX_DEPTH + 1];
+  int levels_private; /* wbfmm_tree_levels_private */
   double *d_q, *d_dip; /* strengths in sorted order */
   unsigned cap_q, cap_dip;
   int prec32; /* FP32 coefficients scaled by the box width (Laplace) */
@@ -560,19 +561,22 @@ wbfmm_tree_t *wbfmm_tree_new(gdouble *x, gdouble D, guint maxpoints)
   return t;
 }
 
-gint wbfmm_tree_host_mirror(wbfmm_tree_t *t, gboolean on)
-{
-  TD(t)->host_mirror = on ? 1 : 0;
-  return 0;
-}
-
 /* What a level array holds: zeros; zeros but in the boxes of d_occ (mps) or
    d_act (mpr), whose lists and counts are those that the passes wrote it
    by; or values anywhere.  An array is cleared by the boxes that were
-   written, and not at all when none was.  Trees with a host mirror hand out
-   pointers into the arrays (box mps, mpr): theirs are always cleared
-   whole. */
+   written, and not at all when none was, in trees whose levels are private
+   (wbfmm_tree_levels_private).  The arrays are public members, and a host
+   mirror hands out pointers into them (box mps, mpr): whatever else wrote
+   them is not seen here, so other trees' arrays are cleared whole. */
 enum { LEVEL_ZERO, LEVEL_LISTED, LEVEL_ANY };
+
+gint wbfmm_tree_host_mirror(wbfmm_tree_t *t, gboolean on)
+{
+  /* (pointers handed out by a mirror outlive it) */
+  if (TD(t)->host_mirror && !on) memset(TD(t)->held, LEVEL_ANY, sizeof(TD(t)->held));
+  TD(t)->host_mirror = on ? 1 : 0;
+  return 0;
+}
 
 /* the passes are about to write boxes of the current lists (listed) or any
    boxes of a level array */
@@ -602,7 +606,7 @@ static void level_clear(tree_dev *td, unsigned l, int which)
   const size_t row = td->box_bytes[which][l];
   const uint32_t *list = which ? td->d_act[l] : td->d_occ[l];
   const unsigned n = which ? td->nact[l] : td->nocc[l];
-  const int held = td->host_mirror ? LEVEL_ANY : td->held[which][l];
+  const int held = td->levels_private && !td->host_mirror ? td->held[which][l] : LEVEL_ANY;
   if (held == LEVEL_ZERO) return;
   if (held == LEVEL_LISTED && n <= nb / 2)
     HIPOK(wbfmm_hip_clear_rows(p, list, n, nb, row, (unsigned)(bytes / (nb * row))));
@@ -792,6 +796,15 @@ gint wbfmm_tree_refine(wbfmm_tree_t *t)
     t->boxes[l] = calloc((size_t)1 << (3 * l), sizeof(wbfmm_box_t));
   t->depth = l;
   mirror_level(td, l);
+  return 0;
+}
+
+gint wbfmm_tree_levels_private(wbfmm_tree_t *t, gboolean on)
+{
+  tree_dev *td = TD(t);
+  /* what was written before is not known */
+  if (on && !td->levels_private) memset(td->held, LEVEL_ANY, sizeof(td->held));
+  td->levels_private = on ? 1 : 0;
   return 0;
 }
 
