@@ -495,12 +495,7 @@ int wbfmm_hip_hel_wide_m2l(const uint32_t *cls, const unsigned *cstart, const un
     const int ro = occupancy_bits(sstart, send, level, &occ);
     if (ro) return ro;
   }
-  // one block runs on a CU at a time (its LDS): the offsets of a chunk are
-  // split over blocks until there are about three rounds of blocks.  The
-  // split depends on the chunk count only, so that a problem always sums
-  // in the same order
-  int nsplit = (int)(768 / nch);
-  nsplit = nsplit < 1 ? 1 : nsplit > 27 ? 27 : nsplit;
+  const int nsplit = wide_nsplit(nch);
   const size_t C = (size_t)(Nr + 1) * (Nr + 1);
   double *part = nullptr;
   if (nsplit > 1 && dmalloc((void **)&part, sizeof(double) * 2 * (size_t)nsplit * ntot * C)) {
@@ -536,7 +531,7 @@ int wbfmm_hip_hel_wide_shift(int mode, const uint32_t *parents, unsigned npar,
     // few parents: a block per child digit, so that the eight translations
     // of a chunk run side by side (64 parents at order 30: 0.37 ms in one
     // block each)
-    const int nsplit = nb < 128 ? 8 : 1;
+    const int nsplit = wide_m2m_nsplit(nb);
     const size_t C = (size_t)(Nout + 1) * (Nout + 1);
     double *part = nullptr;
     if (nsplit > 1 && dmalloc((void **)&part, sizeof(double) * 2 * nsplit * npar * C))

@@ -9,6 +9,7 @@
 #include <hip/hip_runtime.h>
 
 #include "hip_common.h"
+#include "m2l_split.h"
 
 namespace wbfmm {
 
@@ -318,29 +319,6 @@ template <typename T, int N>
 struct M2LDouble {
   static constexpr bool value = 2 * (M2LShape<N>::S + 1) * 16 * sizeof(T) <= 48 * 1024;
 };
-
-// Blocks per chunk of the split M2L form (a chunk's offsets dealt to several
-// blocks, whose partial sums k_m2l_reduce adds): levels with fewer than 1024
-// chunks take up to 2048 blocks in all, at most 8 a chunk, and levels 2 and 3,
-// where that leaves most of the chip idle while each block works through its
-// offsets in series, up to 25.  With 8 there, level 2 (64 boxes) took 0.077 ms
-// at order 8 and takes 0.035, levels 2 and 3 at order 13 0.217 and 0.152, 9
-// launches of 3 components at order 10 1.52 and 1.40; 35 a chunk or 4096
-// blocks gain nothing more, and their partial sums cost more.  More than 8
-// only while a full level's partials stay within kSplitBytes, the memory of
-// the allocation-free entry point.  The split depends on the level, the order
-// and the chunk count alone, so that a problem always sums in the same order
-// (up to 256 chunks, as a Laplace level 4 has, not on the count either).
-constexpr size_t kSplitBytes = ((size_t)62 << 20) - ((size_t)16 << 10);
-static inline int m2l_nsplit(int level, unsigned nchunks, size_t bytes_per_box) {
-  if (nchunks >= 1024) return 1;
-  unsigned most = 8;
-  if (level <= 3) {
-    const size_t fit = kSplitBytes / (bytes_per_box << (3 * level));
-    most = fit < 8 ? 8 : fit < 25 ? (unsigned)fit : 25;
-  }
-  return (int)(2048 / nchunks < most ? 2048 / nchunks : most);
-}
 
 // mpr[cls[i]] += sum over the splits (in split order) of the partials of
 // target i

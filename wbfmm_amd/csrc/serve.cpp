@@ -28,6 +28,8 @@
 
 #include "wbfmm_serve.h"
 
+#include "m2l_split.h"
+
 // the host layer's recovery point (wbfmm_api.c): runs fn(arg); a failure
 // that the drop-in API would turn into an abort returns its status here
 // instead (message in msg), with the library's locks released
@@ -179,8 +181,8 @@ int choose_precision(const wbfmm_serve_request_t &r, int lap_order) {
 //    the engine's field buffer; the check's copies;
 //  - the largest transient of one pass: the M2L occupancy bits and class
 //    list of a level, the partial expansions of a level whose offsets are
-//    split (fewer than 1024 chunks of 16 targets: up to 8 copies of at most
-//    16384 targets' expansions), and the radix sort's temporaries;
+//    split (m2l_split.h; at least 8 copies of at most 16384 targets'
+//    expansions), and the radix sort's temporaries;
 //  - the operator tables a worker builds for this order (rotation and
 //    coaxial tiles; kept by the worker and reused by later requests)
 // tables: rotation tiles of the order (49 angles, one 64-double tile per
@@ -205,9 +207,16 @@ size_t footprint(const wbfmm_serve_request_t &r, const Plan &p) {
     const double ka = r.k * 0.5 * std::sqrt(3.0) * p.D / (double)(1u << l);
     const size_t es = p.precision == 32 && (cplx == 1 || ka <= 2.0) ? 4 : 8;
     b += nb * (2 * C * es * cplx + 24);
-    const size_t split_targets = std::min<size_t>(nb, 16384);
-    const size_t level_tr = nb / 8 + 4 * nb + 8 * split_targets * C * es * cplx;
-    transient = std::max(transient, level_tr);
+    const size_t one = C * es * cplx;
+    size_t part = 8 * std::min<size_t>(nb, 16384) * one;
+    if (l >= 2) {
+      part = std::max(part, wbfmm::m2l_split_boxes(l, one) * one);
+      if (cplx == 2) {  // (FP64 at any precision)
+        part = std::max(part, wbfmm::wide_split_boxes(l) * C * 16);
+        part = std::max(part, wbfmm::wide_m2m_boxes(l) * C * 16);
+      }
+    }
+    transient = std::max(transient, nb / 8 + 4 * nb + part);
   }
   const size_t nt = r.xt ? r.ntgt : r.nsrc;
   b += (size_t)r.nsrc * (2 * 32 + 12 + 16 * cplx + (r.normals ? 32 : 0));
