@@ -422,6 +422,20 @@ int wbfmm_hip_lap_field(const double *xt, const uint32_t *tid, unsigned n,
                         const double *nrm, const double *dip,
                         unsigned level, const double *x0, double D, int N,
                         const double *mpr, int field, double *f, int fstr);
+/* the same with coefficients of either precision (f32: mpr as
+   wbfmm_hip_lap_field_f32 has it) and the number of leaf boxes that the
+   targets lie in, by which the lanes per target are chosen (the entries
+   without it count every box of the level) */
+int wbfmm_hip_lap_field_leaves(const double *xt, const uint32_t *tid, unsigned n,
+                               unsigned nleaf, const uint32_t *start,
+                               const uint32_t *end, const double *xyz,
+                               const double *q, const double *nrm,
+                               const double *dip, unsigned level,
+                               const double *x0, double D, int N, int f32,
+                               const void *mpr, int field, double *f, int fstr);
+/* lanes per target that it takes for n targets in nleaf boxes (1, 2, 4, 8
+   or 16; no device needed) */
+int wbfmm_hip_lap_field_lanes(unsigned n, unsigned nleaf);
 /* vector sources, nq components (src/local-laplace.c:333-1336, the curl
    and curl-gradient of :632-1291): L2P + near field for n staged targets
    (rows tid[i] of f, fstr doubles apart).  Component q's local expansions

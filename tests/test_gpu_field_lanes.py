@@ -13,8 +13,6 @@ import pytest
 
 from conftest import fit_box
 
-pytestmark = pytest.mark.gpu
-
 SIZES = [131073, 131072, 131071, 65536, 32769, 16384, 8193, 300, 1]
 TOL = 1e-12
 
@@ -39,6 +37,39 @@ def check(eval_at, xt, tol=TOL):
         assert d < tol, (m, d)
 
 
+@pytest.mark.parametrize("n,nleaf,lanes", [
+    # by the number of targets
+    (1, 1, 16), (16383, 64, 16), (16384, 64, 8), (32767, 64, 8), (32768, 64, 4), (65536, 64, 2),
+    (131072, 64, 1), (1 << 27, 1 << 30, 1),
+    # four where the occupied leaves hold fewer than two each: 1e6 in a cube
+    # and on a sphere at depth 7, 3e5 on a sphere at depths 6 and 7
+    (1000000, 794000, 4), (1000000, 68200, 1), (300000, 17300, 1), (300000, 61700, 1),
+    (300000, 178000, 4), (200000, 100000, 1), (200000, 100001, 4)])
+def test_lanes_by_occupied_leaves(wb, n, nleaf, lanes):
+    assert wb.lib().wbfmm_hip_lap_field_lanes(n, nleaf) == lanes
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("precision", [64, 32])
+def test_empty_leaves_do_not_count(wb, precision):
+    """140000 targets in few of the 262144 leaves of depth 6 take one lane
+    each: the same bits as when each is asked for four times over, where the
+    targets are more than twice all the leaves"""
+    rng = np.random.default_rng(8)
+    x = rng.normal(size=(140000, 3)) * 0.02 + 0.5
+    xs, q = np.ascontiguousarray(x[::70]), rng.normal(size=2000)
+    S = wb.LaplaceSolver(xs, np.zeros(3), 1.0, 6, [4] * 17, [4] * 17, precision=precision,
+                         host_mirror=False)
+    S.build_tree()
+    S.passes(q)
+    f, f4 = np.zeros((len(x), 4)), np.zeros((4 * len(x), 4))
+    S.field_points(x, q, f)
+    S.field_points(np.tile(x, (4, 1)), q, f4)
+    S.close()
+    assert np.abs(f).max() > 0 and np.array_equal(np.tile(f, (4, 1)), f4)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("precision,p,depth,dip", [(64, 1, 2, False), (64, 7, 3, True),
                                                    (64, 20, 2, False), (32, 9, 3, False)])
 def test_laplace(wb, precision, p, depth, dip):
@@ -61,6 +92,7 @@ def test_laplace(wb, precision, p, depth, dip):
     S.close()
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("field,width", [(6, 12), (4, 3), (3, 12)])
 def test_vector_sources(wb, field, width):
     rng, xs, _ = points(31, 3000)
@@ -80,6 +112,7 @@ def test_vector_sources(wb, field, width):
     S.close()
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("precision,p", [(64, 11), (32, 11), (64, 29)])
 def test_helmholtz(wb, precision, p):
     # a third of the sources without a monopole, a third without a dipole

@@ -1180,7 +1180,7 @@ static int lap_field(const char *name, const double *xt, const uint32_t *tid, un
                      const uint32_t *start, const uint32_t *end, const double *xyz,
                      const double *q, const double *nrm, const double *dip, unsigned level,
                      const double *x0, double D, int N, double rs, const T *mpr, int field,
-                     double *f, int fstr) {
+                     double *f, int fstr, unsigned nleaf) {
   if (N < 0 || N > kMaxN) return WBFMM_HIP_ERR_ORDER;
   if (n == 0) return 0;
   const LapTab *tab = nullptr;
@@ -1192,13 +1192,7 @@ static int lap_field(const char *name, const double *xt, const uint32_t *tid, un
                  tid, n, start, end, xyz, q, nrm, dip, (int)level, x0[0], x0[1], x0[2], D, N, \
                  rs, mpr, field, f, fstr, tab);                                               \
     return 0;
-  // leaves of fewer than two targets: mostly expansion steps, whose
-  // scattered coefficient reads four lanes of a target share (1e6 targets
-  // at depth 7, order 12: 2.40 ms with one lane, 1.80 with two, 1.57 with
-  // four)
-  int g = field_lanes(n);
-  if (g < 4 && n >> 1 < (uint64_t)1 << (3 * level)) g = 4;
-  switch (n > (1u << 26) ? 1 : g) {
+  switch (wbfmm_hip_lap_field_lanes(n, nleaf)) {
     LAP_FIELD(1)
     LAP_FIELD(2)
     LAP_FIELD(4)
@@ -1373,14 +1367,43 @@ int wbfmm_hip_lap_l2l(const uint32_t *parents, unsigned npar,
   return 0;
 }
 
+// Occupied leaves of fewer than two targets on average: mostly expansion
+// steps, whose scattered coefficient reads four lanes of a target share.
+// Measured with one lane, two and four, orders 12 (FP64) and 9 (FP32), ms,
+// at targets per occupied leaf: 1.26 (1e6 in a cube, depth 7) 2.41 1.80 1.58
+// and 1.08 0.77 0.73; 1.68 (3e5, depth 6) 0.55 0.41 0.39 and 0.27 0.24 0.23;
+// 1.96 0.65 0.48 0.47 and 0.37 0.31 0.29; 2.56 (6e5, depth 6) 0.80 0.67 0.75
+// and 0.46 0.47 0.48; 4.9 (3e5 on a sphere, depth 7) 0.31 0.34 0.41 and 0.27
+// 0.28 0.30; 14.7 (1e6 on a sphere, depth 7) 1.22 1.58 1.97 and 1.05 1.40
+// 1.63.  The empty boxes of a level do not count: over all boxes the last
+// two have 0.14 and 0.48 targets a leaf.
+int wbfmm_hip_lap_field_lanes(unsigned n, unsigned nleaf) {
+  if (n > (1u << 26)) return 1;
+  const int g = field_lanes(n);
+  return g < 4 && n >> 1 < nleaf ? 4 : g;
+}
+
+int wbfmm_hip_lap_field_leaves(const double *xt, const uint32_t *tid, unsigned n, unsigned nleaf,
+                               const uint32_t *start, const uint32_t *end, const double *xyz,
+                               const double *q, const double *nrm, const double *dip,
+                               unsigned level, const double *x0, double D, int N, int f32,
+                               const void *mpr, int field, double *f, int fstr) {
+  const double w = D / (double)(1u << level);
+  if (f32)
+    return lap_field<float>("lap_l2p_p2p_f32", xt, tid, n, start, end, xyz, q, nrm, dip, level, x0,
+                            D, N, 1.0 / w, (const float *)mpr, field, f, fstr, nleaf);
+  return lap_field<double>("lap_l2p_p2p", xt, tid, n, start, end, xyz, q, nrm, dip, level, x0, D, N,
+                           1.0, (const double *)mpr, field, f, fstr, nleaf);
+}
+
 int wbfmm_hip_lap_field(const double *xt, const uint32_t *tid, unsigned n,
                         const uint32_t *start, const uint32_t *end,
                         const double *xyz, const double *q, const double *nrm,
                         const double *dip, unsigned level, const double *x0,
                         double D, int N, const double *mpr, int field,
                         double *f, int fstr) {
-  return lap_field<double>("lap_l2p_p2p", xt, tid, n, start, end, xyz, q, nrm, dip, level, x0, D, N,
-                           1.0, mpr, field, f, fstr);
+  return wbfmm_hip_lap_field_leaves(xt, tid, n, 1u << (3 * level), start, end, xyz, q, nrm, dip,
+                                    level, x0, D, N, 0, mpr, field, f, fstr);
 }
 
 int wbfmm_hip_lap_field_f32(const double *xt, const uint32_t *tid, unsigned n,
@@ -1389,9 +1412,8 @@ int wbfmm_hip_lap_field_f32(const double *xt, const uint32_t *tid, unsigned n,
                             const double *dip, unsigned level, const double *x0,
                             double D, int N, const float *mpr, int field,
                             double *f, int fstr) {
-  const double w = D / (double)(1u << level);
-  return lap_field<float>("lap_l2p_p2p_f32", xt, tid, n, start, end, xyz, q, nrm, dip, level, x0, D,
-                          N, 1.0 / w, mpr, field, f, fstr);
+  return wbfmm_hip_lap_field_leaves(xt, tid, n, 1u << (3 * level), start, end, xyz, q, nrm, dip,
+                                    level, x0, D, N, 1, mpr, field, f, fstr);
 }
 
 int wbfmm_hip_to_f32(const double *in, float *out, size_t n) {

@@ -1760,16 +1760,13 @@ static void lap_field_run(tree_dev *td, const double *dxt,
   dp = gather_strengths(td, d, dstr, 1);
   nelem = nf_rows ? (nf_rows - 1) * (size_t)fstr + ((field & 1) ? 1 : 0) + ((field & 2) ? 3 : 0) : 0;
   df = field_begin(f, nelem, &staged);
-  if (td->prec32)
-    HIPOK(wbfmm_hip_lap_field_f32(dxt, dtid, n, td->d_start[lv], td->d_end[lv],
-                                  td->d_xyz, q, dp ? td->d_nrm : NULL, dp, lv,
-                                  ORIGIN(t), t->D, t->order_r[lv],
-                                  (const float *)t->mpr[lv], field, df, fstr));
-  else
-    HIPOK(wbfmm_hip_lap_field(dxt, dtid, n, td->d_start[lv], td->d_end[lv],
-                              td->d_xyz, q, dp ? td->d_nrm : NULL, dp, lv,
-                              ORIGIN(t), t->D, t->order_r[lv],
-                              (double *)t->mpr[lv], field, df, fstr));
+  /* leaves that the targets lie in: those of the registered list, with the
+     sources'; without one the sources', as far as is known */
+  tree_counts(td);
+  HIPOK(wbfmm_hip_lap_field_leaves(
+      dxt, dtid, n, td->have_targets && lv < td->tgt_levels ? td->nact[lv] : td->nocc[lv],
+      td->d_start[lv], td->d_end[lv], td->d_xyz, q, dp ? td->d_nrm : NULL, dp, lv, ORIGIN(t),
+      t->D, t->order_r[lv], td->prec32, t->mpr[lv], field, df, fstr));
   field_finish(f, df, nelem, staged);
 }
 
