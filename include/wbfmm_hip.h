@@ -552,6 +552,8 @@ int wbfmm_hip_hel_shift_mfma(int mode, const uint32_t *parents, unsigned npar,
    the unit n(n+1)/2 + nu), -1 for an unused row; s1: slots of a unit as
    the input of stage 1. */
 #define WBFMM_HEL_WIDE_MAXN 40
+/* the highest order of the per-order kernels (equal orders) */
+#define WBFMM_HEL_M2L_MAXN 27
 #define WBFMM_HEL_WIDE_MAXT 80
 #define WBFMM_HEL_WIDE_MAXU 861
 typedef struct {
@@ -573,6 +575,21 @@ int wbfmm_hip_hel_wide_rot(const wbfmm_hel_wide_plan_t *plan, int nth, const dou
                            double *A);
 int wbfmm_hip_hel_wide_coax(const wbfmm_hel_wide_plan_t *plan, int L, int nr, const double *E,
                             double *A2);
+/* 1 where the M2L of a level with these orders is the run-time-order kernel's
+   (no device needed): all orders above WBFMM_HEL_M2L_MAXN; equal ones are the
+   per-order kernels' up to there; of different orders those at levels 2
+   and 3, and deeper where the highest is 14 (level 4) or 15, or 12 where
+   three of four boxes hold sources (nsrc: their number).  Below that the
+   vector kernel is faster: it visits the occupied pairs alone, where a block
+   here takes the offsets of 8 targets together and has the LDS of order 24 to
+   itself.  Vector and this kernel, ms, orders (N, N-1): level 5 of 1e5 points
+   in a cube 14.9 and 44.8 at N = 8, 40.4 and 49.9 at 11, 56.7 and 51.9 at 12,
+   123 and 59 at 15; of 2e4 (46 % of the boxes) 4.0 and 21.9, 14.1 and 24.5 at
+   12, 30.1 and 28.1 at 15; of 1e5 on a sphere 0.90 and 4.7, 2.2 and 5.1, 5.9 and 6.1; level 4 of 3000 in
+   a cube 1.1 and 4.2 at 8, 5.3 and 5.2 at 14; level 3 full 1.6 and 0.84 at 8,
+   2 of 1000 points 0.23 and 0.09 at 2 (few targets: the vector kernel's
+   wavefronts leave the chip idle). */
+int wbfmm_hip_hel_wide_m2l_serves(int Ns, int Nr, unsigned level, unsigned nsrc);
 /* M2L (as wbfmm_hip_hel_m2l_mfma; CS: 343 x (N+1) x 2, cos and sin of m
    chi) and M2M / L2L (as wbfmm_hip_hel_shift_mfma; CS: 8 x (N+1) x 2) */
 int wbfmm_hip_hel_wide_m2l(const uint32_t *cls, const unsigned *cstart, const unsigned *ccount,

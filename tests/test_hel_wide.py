@@ -196,3 +196,43 @@ def test_solve_matches_oracle(wb, oracle, name):
         d = np.abs(fs[0][:, c] - fo[:, c]).max() / np.abs(fo[:, c]).max()
         assert d < 1e-10, (name, c, d)
     assert np.array_equal(fs[0], fs[1])
+
+
+@pytest.mark.parametrize("Ns,Nr,level,nsrc,wide", [
+    (28, 28, 5, 9, 1), (40, 28, 2, 9, 1), (27, 28, 7, 9, 1), (41, 41, 3, 9, 0), (1, 1, 3, 9, 0),
+    (41, 20, 3, 9, 0),
+    (27, 27, 3, 512, 0), (9, 9, 2, 64, 0),                       # equal: the per-order kernels
+    (2, 1, 2, 9, 1), (9, 8, 3, 512, 1), (8, 9, 3, 9, 1),         # few targets
+    (13, 12, 4, 3071, 0), (12, 13, 4, 9, 0), (14, 13, 4, 9, 1), (14, 13, 5, 9, 0),
+    (15, 14, 5, 9, 1), (2, 15, 7, 9, 1),
+    (11, 10, 4, 4096, 0), (12, 11, 4, 3072, 1), (11, 12, 10, 1 << 30, 1)])  # nearly full
+def test_m2l_rule(wb, Ns, Nr, level, nsrc, wide):
+    assert wb.lib().wbfmm_hip_hel_wide_m2l_serves(Ns, Nr, level, nsrc) == wide
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("Ns,Nr,wide", [(5, 4, [1, 1, 0]), (4, 5, [1, 1, 0]), (14, 13, [1, 1, 1])])
+def test_m2l_of_low_different_orders(wb, oracle, Ns, Nr, wide):
+    """levels 2, 3 and 4 each on the kernel of the rule (the run-time-order one
+    alone makes an occupancy bitmap), and the solve against the oracle FMM"""
+    rng = np.random.default_rng(900)
+    n, k, depth = 700, 2.0, 4
+    xs, q = rng.uniform(-1, 1, (n, 3)), rng.normal(size=n) + 1j * rng.normal(size=n)
+    x0, D = fit_box(xs)
+    so, ro = [Ns] * 17, [Nr] * 17
+    S = wb.HelmholtzSolver(xs, x0, D, depth, so, ro, k)
+    S.build_tree()
+    T = wb.Timing
+    T.enable(True)
+    T.reset()
+    S.passes(c2(q))
+    wb.sync()
+    maps = T.query("m2l_occ_bits")[0]
+    T.enable(False)
+    assert maps == sum(wide)
+    f = np.zeros((n, 8))
+    S.field(xs, c2(q), f)
+    S.close()
+    fo, _, _ = oracle.fmm(2, xs, xs, x0, D, depth, so, ro, q=c2(q), k=k, field=3, nthreads=8)
+    # parity 1e-10 of each column's largest value, as above
+    assert (np.abs(f - fo).max(0) < 1e-10 * np.abs(fo).max(0)).all()

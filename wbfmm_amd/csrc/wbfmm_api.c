@@ -262,7 +262,7 @@ typedef struct {
 #define M2L_MFMA_MIN 2
 #define M2L_MFMA_MAX 24
 /* orders served by the Helmholtz matrix-core M2L, M2M and L2L */
-#define HEL_MFMA_MAX 27
+#define HEL_MFMA_MAX WBFMM_HEL_M2L_MAXN
 /* orders served by the FP32 passes (the FP64 matrix-core M2M / L2L serve
    M2L_MFMA_MIN..M2L_MFMA_MAX) */
 #define SHIFT_MFMA_MAX 15
@@ -2631,13 +2631,14 @@ static int hel_shift_mfma(ops_dev *od, guint Nc, guint Np)
   return Nc == Np && (int)Nc >= M2L_MFMA_MIN && (int)Nc <= HEL_MFMA_MAX && hel_mfma_enabled();
 }
 
-/* orders Na, Nb of the two sides of a translation that the run-time-order
-   matrix-core passes take: different orders, and equal ones above those of
-   the per-order kernels, which serve equal orders better where they fit
-   (M2L of a 1e5-point sphere at orders 25/23: 7.7 against 16.8 ms).  The
-   vector kernels they replace: 3e4-point cube, order 30, M2L 63.8 -> 3.6,
-   M2M 2.0 -> 0.06, L2L 2.0 -> 0.07 ms; M2M 23 -> 25 and L2L 25 -> 23 on
-   the sphere 1.05 -> 0.30 and 1.08 -> 0.36 ms */
+/* orders Na, Nb of the two sides of an M2M or L2L that the run-time-order
+   matrix-core kernels take (M2L: wbfmm_hip_hel_wide_m2l_serves): different
+   orders, and equal ones above those of the per-order kernels, which serve
+   equal orders better where they fit (M2L of a 1e5-point sphere at orders
+   25/23: 7.7 against 16.8 ms).  The vector kernels they replace: 3e4-point
+   cube, order 30, M2L 63.8 -> 3.6, M2M 2.0 -> 0.06, L2L 2.0 -> 0.07 ms; M2M
+   23 -> 25 and L2L 25 -> 23 on the sphere 1.05 -> 0.30 and 1.08 -> 0.36 ms;
+   of orders 2..5 at depth 4 M2M 0.09 -> 0.04, L2L 0.08 -> 0.04 */
 static int hel_wide_serves(guint Na, guint Nb)
 {
   const guint N = Na > Nb ? Na : Nb;
@@ -2775,7 +2776,8 @@ static void hel_m2l64(wbfmm_tree_t *t, ops_dev *od, guint level, const uint32_t 
                                  level, N, (double *)t->mps[level], (double *)t->mpr[level],
                                  od->m2l_plan_dev[N], od->hel_A[N], od->hel_A2[level],
                                  od->m2l_CS[N], od->m2l_plan[N]));
-  } else if (hel_wide_serves(Ns, Nr) && level <= M2L_MFMA_MAX_LEVEL) {
+  } else if (wbfmm_hip_hel_wide_m2l_serves((int)Ns, (int)Nr, level, td->nocc[level]) &&
+             hel_mfma_enabled() && level <= M2L_MFMA_MAX_LEVEL) {
     int N = (int)(Ns > Nr ? Ns : Nr);
     unsigned cstart[8], ccount[8];
     const uint32_t *cls;

@@ -1235,6 +1235,17 @@ int wbfmm_hip_hel_wide_plan(int N, wbfmm_hel_wide_plan_t *P)
   return wbfmm_hip_offset_geometry(ths, &P->NTH, P->th, P->chi, P->rr, &P->NR, P->rix);
 }
 
+int wbfmm_hip_hel_wide_m2l_serves(int Ns, int Nr, unsigned level, unsigned nsrc)
+{
+  const int N = Ns > Nr ? Ns : Nr;
+  if (N < 2 || N > WBFMM_HEL_WIDE_MAXN) return 0;
+  if (N > WBFMM_HEL_M2L_MAXN) return 1;
+  if (Ns == Nr) return 0;
+  if (level <= 3) return 1;
+  if (4 * (uint64_t)nsrc >= 3ull << (3 * level)) return N >= 12;
+  return N >= (level == 4 ? 14 : 15);
+}
+
 /* the tiles of part pt with entry val(ctx, pt, size, row, column) */
 typedef double (*wide_entry)(const void *ctx, int pt, int sz, int row, int col);
 static void wide_fill(const wbfmm_hel_wide_plan_t *Q, wide_entry val, const void *ctx, double *A)
