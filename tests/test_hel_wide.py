@@ -9,6 +9,9 @@ kernel's ranges of orders (..24, ..31, ..40) and with unequal orders.
 
 import ctypes
 import math
+import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -236,3 +239,60 @@ def test_m2l_of_low_different_orders(wb, oracle, Ns, Nr, wide):
     fo, _, _ = oracle.fmm(2, xs, xs, x0, D, depth, so, ro, q=c2(q), k=k, field=3, nthreads=8)
     # parity 1e-10 of each column's largest value, as above
     assert (np.abs(f - fo).max(0) < 1e-10 * np.abs(fo).max(0)).all()
+
+
+# counts the tables made, in front of the library's function
+COUNT_C = r"""
+#define _GNU_SOURCE
+#include <dlfcn.h>
+#include <stdlib.h>
+int made;
+int wbfmm_hip_hel_wide_coax(const void *P, int L, int nr, const double *E, double *A2)
+{
+  int (*f)(const void *, int, int, const double *, double *);
+  *(void **)&f = dlsym(dlopen(getenv("WBFMM_LIB"), RTLD_NOW | RTLD_NOLOAD), "wbfmm_hip_hel_wide_coax");
+  made++;
+  return f(P, L, nr, E, A2);
+}
+"""
+COUNT_PY = r"""
+import ctypes, os, sys
+shim = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+import numpy as np
+import wbfmm_amd as wb
+os.environ["WBFMM_LIB"] = wb.LIB_PATH
+ctypes.CDLL(None).setenv(b"WBFMM_LIB", wb.LIB_PATH.encode(), 1)
+rng = np.random.default_rng(1)
+xs, q = rng.uniform(-1, 1, (300, 3)), rng.normal(size=(300, 2))
+so, ro = [9, 9, 9, 8, 7] + [7] * 12, [6, 6, 6, 5, 4] + [4] * 12
+S = wb.HelmholtzSolver(xs, np.full(3, -1.01), 2.02, 4, so, ro, 1.5)
+made, fs = [], []
+for rep in range(3):
+    S.build_tree()
+    S.passes(q)
+    f = np.zeros((300, 8))
+    S.field(xs, q, f)
+    made.append(ctypes.c_int.in_dll(shim, "made").value)
+    fs.append(f)
+S.close()
+assert np.array_equal(fs[0], fs[1]) and np.array_equal(fs[0], fs[2])
+print("made", *made)
+"""
+
+
+@pytest.mark.gpu
+def test_tables_are_made_once(tmp_path):
+    """source and receiver orders differ, and between levels too: M2M and L2L
+    ask for tables of different orders at each level, made by the first solve
+    and kept for the next ones"""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    src, so = tmp_path / "count.c", tmp_path / "count.so"
+    src.write_text(COUNT_C)
+    r = subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(so), str(src), "-ldl"],
+                       capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
+    r = subprocess.run([sys.executable, "-u", "-c", COUNT_PY, str(so)], cwd=root,
+                       capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stdout + r.stderr
+    first, second, third = (int(a) for a in r.stdout.split()[-3:])
+    assert first > 0 and second == third == first, r.stdout

@@ -233,15 +233,17 @@ typedef struct {
   int hel_SS2_N[WBFMM_TREE_MAX_DEPTH + 1];
   /* Helmholtz passes with run-time orders (wbfmm_hip_hel_wide_*): plan,
      rotation tiles of the offset and child angles and phases per order
-     (shared by the process), coaxial tiles per level with the order they
-     were made for */
+     (shared by the process), coaxial tiles per level: of the M2L with the
+     order they were made for, of the shifts per order (M2M and L2L of a level
+     ask for two where source and receiver orders differ) */
   wbfmm_hel_wide_plan_t *wide_plan[WBFMM_HIP_MAX_ORDER + 1];
   void *wide_plan_dev[WBFMM_HIP_MAX_ORDER + 1];
   double *wide_A[WBFMM_HIP_MAX_ORDER + 1], *wide_shA[WBFMM_HIP_MAX_ORDER + 1];
   double *wide_CS[WBFMM_HIP_MAX_ORDER + 1], *wide_CSup[WBFMM_HIP_MAX_ORDER + 1],
       *wide_CSdn[WBFMM_HIP_MAX_ORDER + 1];
-  double *wide_SR[WBFMM_TREE_MAX_DEPTH + 1], *wide_SS[WBFMM_TREE_MAX_DEPTH + 1];
-  int wide_SR_N[WBFMM_TREE_MAX_DEPTH + 1], wide_SS_N[WBFMM_TREE_MAX_DEPTH + 1];
+  double *wide_SR[WBFMM_TREE_MAX_DEPTH + 1];
+  double *wide_SS[WBFMM_TREE_MAX_DEPTH + 1][WBFMM_HIP_MAX_ORDER + 1];
+  int wide_SR_N[WBFMM_TREE_MAX_DEPTH + 1];
   /* mixed-precision Helmholtz: FP32 rotation tiles and phases per order,
      and per level the scaled FP32 coaxial tiles of the M2L and of the
      M2M into / L2L from the level above, with the order and wavenumber
@@ -1124,6 +1126,16 @@ static void ensure_lap_coax(ops_dev *od)
   mu_unlock(&g_tab_mu);
 }
 
+/* the coaxial tiles of a level's shifts, of every order */
+static void wide_shifts_free(ops_dev *od, unsigned level)
+{
+  int N;
+  for (N = 0; N <= WBFMM_HIP_MAX_ORDER; N++) {
+    wbfmm_hip_free(od->wide_SS[level][N]);
+    od->wide_SS[level][N] = NULL;
+  }
+}
+
 gint wbfmm_shift_operators_free(wbfmm_shift_operators_t *op)
 {
   ops_dev *od = (ops_dev *)op;
@@ -1139,7 +1151,7 @@ gint wbfmm_shift_operators_free(wbfmm_shift_operators_t *op)
     wbfmm_hip_free(od->hel_SS2[n]);
     free(od->ss_host[n]);
     wbfmm_hip_free(od->wide_SR[n]);
-    wbfmm_hip_free(od->wide_SS[n]);
+    wide_shifts_free(od, n);
     wbfmm_hip_free(od->f_hA2[n]);
     wbfmm_hip_free(od->f_hUp[n]);
     wbfmm_hip_free(od->f_hDn[n]);
@@ -2359,8 +2371,7 @@ gint wbfmm_shift_operators_coaxial_SS_init(wbfmm_shift_operators_t *w, gdouble D
   od->ss_host[level] = h;
   wbfmm_hip_free(od->hel_SS2[level]);
   od->hel_SS2[level] = NULL;
-  wbfmm_hip_free(od->wide_SS[level]);
-  od->wide_SS[level] = NULL;
+  wide_shifts_free(od, level);
   od->ss_L[level] = L;
   return 0;
 }
@@ -2388,8 +2399,8 @@ gint wbfmm_shift_operators_coaxial_reset(wbfmm_shift_operators_t *w)
     wbfmm_hip_free(od->f_hDn[n]);
     od->f_hA2[n] = od->f_hUp[n] = od->f_hDn[n] = NULL;
     wbfmm_hip_free(od->wide_SR[n]);
-    wbfmm_hip_free(od->wide_SS[n]);
-    od->wide_SR[n] = od->wide_SS[n] = NULL;
+    od->wide_SR[n] = NULL;
+    wide_shifts_free(od, n);
   }
   od->hel_k_set = 0;
   return 0;
@@ -2732,12 +2743,12 @@ static void ensure_wide_rot(ops_dev *od, int N)
 static const double *wide_coax(ops_dev *od, guint level, int N, int shift)
 {
   const wbfmm_hel_wide_plan_t *P = od->wide_plan[N];
-  double **slot = shift ? &od->wide_SS[level] : &od->wide_SR[level], *h;
-  int *have = shift ? &od->wide_SS_N[level] : &od->wide_SR_N[level], i;
+  double **slot = shift ? &od->wide_SS[level][N] : &od->wide_SR[level], *h;
+  int i;
   const double *E = shift ? od->ss_host[level] : od->sr_host[level];
   const int nr = shift ? 1 : P->NR;
   const size_t n = (size_t)nr * 2 * P->KT * 64;
-  if (*slot && *have == N) return *slot;
+  if (*slot && (shift || od->wide_SR_N[level] == N)) return *slot;
   if (!E) WBFMM_FATAL("coaxial operators not initialised at level %u", level);
   if (!shift) {
     /* both follow wbfmm_hip_offset_geometry */
@@ -2751,7 +2762,7 @@ static const double *wide_coax(ops_dev *od, guint level, int N, int shift)
   wbfmm_hip_free(*slot);
   *slot = NULL;
   *slot = dev_copy(h, sizeof(double) * n);
-  *have = N;
+  if (!shift) od->wide_SR_N[level] = N;
   free(h);
   return *slot;
 }
