@@ -46,7 +46,7 @@ def test_powers(N, kind):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("w", [1.0, 0.3, 1.7e-3])
+@pytest.mark.parametrize("w", [1.0, 0.3, 1.7e-3, 4.92e-7])
 @pytest.mark.parametrize("kind", [0, 1, 2])
 @pytest.mark.parametrize("N", ORDERS)
 def test_scaled(wb, N, kind, w):
@@ -60,6 +60,9 @@ def test_scaled(wb, N, kind, w):
     assert lib.wbfmm_hip_lap_coax_scale(_vp(d1.ptr), _vp(de.ptr), sz(one.size), sz(e.size),
                                         ctypes.c_double(w), _vp(do.ptr)) == 0
     got = do.download(np.zeros_like(one))
+    # (4.92e-7: the last entries of order 24 are near the largest double, and
+    # w^-49 is beyond it)
+    assert np.isfinite(want).all()
     # the host's rounding of r w, taken to a power of up to 2 N + 1, and one
-    # rounding each of the powers and the products
+    # rounding each of two powers and two products
     assert np.all(np.abs(got - want) <= (2 * N + 6) * 2 ** -53 * np.abs(want))

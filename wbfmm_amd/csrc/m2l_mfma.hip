@@ -110,14 +110,18 @@ __global__ void k_class_count(const uint32_t *list, unsigned n,
 
 
 // out[i] = unit[i] w^e[i mod period]: the coaxial tables of a box width from
-// those of width 1, with the powers -100..100 of w as an argument
+// those of width 1, with the powers -100..100 of w as an argument.  The power
+// is applied in two halves: by itself w^e leaves the range of a double for
+// boxes some 5 % wider than the entry does (order 24: 5.2e-7 and 4.9e-7).
 struct WidthPowers {
   double v[201];
 };
 __global__ void k_coax_scale(const double *unit, const signed char *e, size_t n, size_t period,
                              WidthPowers pw, double *out) {
   const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) out[i] = unit[i] * pw.v[e[i % period] + 100];
+  if (i >= n) return;
+  const int k = e[i % period], h = k / 2;
+  out[i] = unit[i] * pw.v[h + 100] * pw.v[k - h + 100];
 }
 
 // the zero expansion (its bytes are zero for either precision, real or
