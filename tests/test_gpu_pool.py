@@ -62,6 +62,18 @@ def test_bounded(wb, lib):
     assert lib.wbfmm_hip_pool_release() == 0 and lib.wbfmm_hip_pool_bytes() == 0
 
 
+def test_bounded_in_number(wb, lib):
+    """an allocation looks through the kept blocks: there are few of them,
+    however small they are"""
+    ps = [take(lib, 4096) for _ in range(5000)]
+    for p in ps:
+        lib.wbfmm_hip_free(p)
+    assert 0 < lib.wbfmm_hip_pool_bytes() <= 2048 * 4096
+    a = take(lib, 4096)
+    assert a in ps[-2048:]
+    lib.wbfmm_hip_free(a)
+
+
 def runtime():
     """the HIP runtime that the library has loaded"""
     path = next(l.split()[-1] for l in open("/proc/self/maps") if "libamdhip64" in l)
