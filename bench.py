@@ -580,9 +580,9 @@ def field_errors(f, fd):
     return err_pot, err_grad, maxd
 
 
-KERNEL_NAMES = ("lap_m2l", "lap_m2m", "lap_l2l", "lap_p2m", "lap_l2p_p2p", "tree_sort",
-                "tree_morton", "tree_box_ranges", "tree_box_flags", "tree_box_scatter",
-                "tree_mark_boxes", "gather4", "gather_strength", "stage4")
+KERNEL_NAMES = ("lap_m2l", "m2l_occ_bits", "m2l_reduce", "lap_m2m", "lap_l2l", "lap_p2m",
+                "lap_l2p_p2p", "tree_sort", "tree_morton", "tree_box_ranges", "tree_box_flags",
+                "tree_box_scan", "tree_box_lists", "clear_rows", "gather4", "gather_strength")
 
 
 def laplace_timed(W, L, d_xs, d_q, d_f, x0, D, n, depth, p, steps, warmup):

@@ -144,11 +144,10 @@ int wbfmm_hip_tree_targets(const uint64_t *tcodes, unsigned n, unsigned hi,
                            uint32_t *const *act, uint32_t *const *cls, uint32_t *tot);
 /* every box of a level >= 1 grouped by child digit (8^(level-1) each) */
 int wbfmm_hip_all_classes(unsigned level, uint32_t *out);
-/* compact list of the boxes with end>start (or flag!=0 when flag is not
-   NULL) in Morton order; *count (host) gets the list length */
+/* compact list of the boxes with end>start in Morton order; *count (host)
+   gets the list length */
 int wbfmm_hip_compact_boxes(const uint32_t *start, const uint32_t *end,
-                            const uint32_t *flag, unsigned level,
-                            uint32_t *list, unsigned *count);
+                            unsigned level, uint32_t *list, unsigned *count);
 /* coordinate bounds of n points (host or device, byte stride pstr) into
    host lo[3], hi[3]; returns after the reduction */
 int wbfmm_hip_bounds(const void *pts, size_t pstr, unsigned n, double *lo,
@@ -156,9 +155,6 @@ int wbfmm_hip_bounds(const void *pts, size_t pstr, unsigned n, double *lo,
 /* dst[i*dstr + c] += src[i*sstr + c], c < ncomp, i < n (device arrays) */
 int wbfmm_hip_accumulate(double *dst, int dstr, const double *src, int sstr,
                          int ncomp, unsigned n);
-/* flag[b] |= 1 for every box at `level` holding one of the n codes */
-int wbfmm_hip_mark_boxes(const uint64_t *codes, unsigned n, unsigned level,
-                         uint32_t *flag);
 
 /* ---- operator tables --------------------------------------------------- */
 /* Real rotation matrices of every list-4 offset (343 slots), of the 8
@@ -362,7 +358,9 @@ int wbfmm_hip_hel_coax_tiles_scaled(const wbfmm_m2l_plan_t *plan, int L, int nr,
 /* out[i] = (float)in[i] on the device */
 int wbfmm_hip_to_f32(const double *in, float *out, size_t n);
 /* sort a box list by Morton child digit (stable); returns the per-class
-   starts and counts on the host */
+   starts and counts on the host.  For callers of the M2L entries below with
+   lists of their own (the passes take their class lists from
+   wbfmm_hip_tree_targets and wbfmm_hip_all_classes). */
 int wbfmm_hip_split_classes(const uint32_t *list, unsigned n, uint32_t *out,
                             unsigned *cstart, unsigned *ccount);
 

@@ -25,45 +25,10 @@ using T2t = typename MF<T>::t2;
 template <typename T>
 using V4t = typename MF<T>::v4;
 
-// stage 2: complex coaxial tiles ar + i ai.  The imaginary product reads
-// the partner column, so that column 2t receives Ar Zr - Ai Zi and column
-// 2t+1 receives Ar Zi + Ai Zr.
-template <typename T, int N, int W, int WI>
-__device__ __forceinline__ void stage_cx(const T *__restrict__ ar,
-                                         const T *__restrict__ ai, const T *R,
-                                         int lane, int grp, int col, V4t<T> *y) {
-  constexpr Bins BN = M2LShape<N>::BN;
-  constexpr WaveSeq WS = make_seq(BN, W, WI);
-  constexpr int AD = WS.n < 8 ? (WS.n > 0 ? WS.n : 1) : 8;
-  T avr[AD], avi[AD];
-#pragma unroll
-  for (int s = 0; s < AD && s < WS.n; s++) {
-    avr[s] = ar[WS.t[s] * 64 + lane];
-    avi[s] = ai[WS.t[s] * 64 + lane];
-  }
-  const T sg = (col & 1) ? T(1) : T(-1);
-  const int pc = col ^ 1;
-#pragma unroll
-  for (int lb = 0; lb < WS.nb; lb++) {
-    const int b = WI + W * lb;
-    V4t<T> r4 = {T(0), T(0), T(0), T(0)}, i4 = {T(0), T(0), T(0), T(0)};
-#pragma unroll
-    for (int j = 0; j < BN.nk[b]; j++) {
-      const int s = WS.start[lb] + j;
-      const int row = (BN.kbase[b] + 4 * j + grp) * 16;
-      r4 = MF<T>::mma(avr[s % AD], R[row + col], r4);
-      i4 = MF<T>::mma(avi[s % AD], R[row + pc], i4);
-      if (s + AD < WS.n) {
-        avr[s % AD] = ar[WS.t[s + AD] * 64 + lane];
-        avi[s % AD] = ai[WS.t[s + AD] * 64 + lane];
-      }
-    }
-    y[lb] = r4 + sg * i4;
-  }
-}
-
-// stage 2 of the T-buffered form: as stage_cx, results stored per bin
-// into the other buffer
+// stage 2 of the T-buffered form: complex coaxial tiles ar + i ai, results
+// stored per bin into the other buffer.  The imaginary product reads the
+// partner column, so that column 2t receives Ar Zr - Ai Zi and column 2t+1
+// receives Ar Zi + Ai Zr.
 template <typename T, int N, int W, int WI>
 __device__ __forceinline__ void stage_cx_wo(const T *__restrict__ ar,
                                             const T *__restrict__ ai, const T *Rin,
@@ -109,7 +74,7 @@ __device__ __forceinline__ void stage_cx_wo(const T *__restrict__ ar,
 // loads run while the stage before is exchanged: op holds the first 16
 // k-steps of a rotation, or the first 8 of a complex coaxial stage (real
 // parts, then imaginary parts); the later ones follow through the same ring
-// as in stage_w and stage_cx.  1e5-point sphere, FP64, orders 25/23: M2L 7.7
+// as in stage_w.  1e5-point sphere, FP64, orders 25/23: M2L 7.7
 // -> 7.1 ms (sixteen wavefronts instead of eight: 596 to 1624 registers
 // spilled); 1e6-point sphere, FP32, order 23: 30.6 -> 29.5 ms.
 template <int N, int W, int WI>

@@ -15,13 +15,14 @@
 // The inverse rotation swaps phi and chi.
 //
 // Kernel shapes (first version, one wavefront per box, vectors in LDS):
-//   P2M      one wave per leaf box; per point the regular functions
-//            R_n^m = j_n(kr) Pbar_n^|m| e^{i m phi} go to LDS (lane m
-//            computes column m) and lane m accumulates orders +-m
+//   P2M      one block per leaf box; per batch of points the regular
+//            functions R_n^m = j_n(kr) Pbar_n^|m| e^{i m phi} go to LDS (a
+//            thread per point and column m), and every thread sums the
+//            points' moments with the R_n^m it owns
 //   M2M/L2L  one wave per parent, the 8 children in turn
 //   M2L      one wave per target box, its list-4 sources in turn, the
 //            local expansion accumulated in LDS
-//   L2P+P2P  one thread per target, regular functions streamed by order
+//   L2P+P2P  1 to 16 lanes per target, regular functions streamed by order
 //            with the gradient in the re-indexed form of G&D (2004) eq 3.7
 
 #include <algorithm>
@@ -113,12 +114,6 @@ __device__ __forceinline__ void sph(double dx, double dy, double dz, double &r,
   }
 }
 
-// Pbar_m^m (G&D normalisation, no Condon-Shortley phase)
-__device__ __forceinline__ double pbar_mm(int m, double S) {
-  double p = 1.0 / sqrt(4.0 * kPi);
-  for (int i = 1; i <= m; i++) p *= sqrt((2.0 * i + 1) / (2.0 * i)) * S;
-  return p;
-}
 // Pbar_{n+1}^m from Pbar_n^m, Pbar_{n-1}^m (src/util.c:81-115)
 __device__ __forceinline__ double pbar_up(int n, int m, double C, double pn, double pnm1) {
   const double v = C * sqrt(2.0 * n + 1) * pn - sqrt((double)(n * n - m * m) / (2 * n - 1)) * pnm1;
@@ -298,9 +293,9 @@ constexpr int kP2MSlots = (p2m_slots(WBFMM_HIP_MAX_ORDER) + kP2MThreads - 1) / k
 // O: double2 (FP64 coefficients) or float2 (FP32 coefficients, each degree
 // n divided by sc[n] in FP64 before rounding; sc NULL: no scaling)
 // NS: slots per thread, ceil((N+2)(N+3)/2 / 256); DIP: with dipoles; three
-// blocks per CU (the LDS of a batch and of two weights' moments is at most
-// 60 KiB), two with the dipoles' moments of three or four slots (above
-// order 29)
+// blocks per CU up to order 26 (their LDS, a batch's and two weights' moments,
+// is at most 60 KiB a block; above, 160 KiB hold two), two with the dipoles'
+// moments of three or four slots (above order 29)
 template <typename O, int NS, bool DIP>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(
     DIP && NS > 2 ? 2 : 3))) void k_hel_p2m(
@@ -621,7 +616,7 @@ __device__ __forceinline__ const double *hel_field_bessel(const RecTab *__restri
 
 // ---------------------------------------------------------------------
 // L2P + near field (src/local.c:32-310, src/expansions.c:275-344,
-// src/gradient.c:282-399), one thread per target.  With
+// src/gradient.c:282-399), G lanes per target.  With
 // R_n^m = j_n(kr) Pbar_n^|m| e^{i m phi} and the G&D eq 3.7 derivatives
 // re-indexed so that every R_n^m (n <= N+1) is used once:
 //   dz f = k sum R_n^m [a_n^m L_{n+1}^m - a_{n-1}^m L_{n-1}^m]
@@ -957,7 +952,7 @@ __global__ __launch_bounds__(64) void k_hel_field_box(
 }
 
 // ---------------------------------------------------------------------
-// Mixed precision with one thread per target (the form of k_hel_field):
+// Mixed precision with G lanes per target (the form of k_hel_field):
 // the local expansion holds L_n^m s_n in FP32 (sc: the level's scales
 // s_n, divided out in FP64 through 1/s_n in LDS), the regular functions
 // and the L2P sums are FP64, and the near-field kernel runs in FP32 with

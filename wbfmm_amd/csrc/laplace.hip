@@ -15,7 +15,7 @@
 //   M2L   one wave per target box, list-4 sources streamed through LDS,
 //         accumulators in registers (rows lane, lane+64, ...)
 //   L2L   one wave per parent, its local expansion staged in LDS
-//   L2P+P2P one thread per target
+//   L2P+P2P 1 to 16 lanes per target
 
 #include <hip/hip_runtime.h>
 

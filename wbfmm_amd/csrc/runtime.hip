@@ -192,11 +192,10 @@ __global__ void k_box_ranges(const uint64_t *codes, unsigned n, int shift,
 }
 
 __global__ void k_box_flags(const uint32_t *start, const uint32_t *end,
-                            const uint32_t *flag, unsigned nb,
-                            uint32_t *out) {
+                            unsigned nb, uint32_t *out) {
   unsigned b = blockIdx.x * blockDim.x + threadIdx.x;
   if (b >= nb) return;
-  out[b] = flag ? (flag[b] != 0) : (end[b] > start[b]);
+  out[b] = end[b] > start[b];
 }
 
 __global__ void k_box_scatter(const uint32_t *flags, const uint32_t *pos,
@@ -204,13 +203,6 @@ __global__ void k_box_scatter(const uint32_t *flags, const uint32_t *pos,
   unsigned b = blockIdx.x * blockDim.x + threadIdx.x;
   if (b >= nb) return;
   if (flags[b]) list[pos[b]] = b;
-}
-
-__global__ void k_mark_boxes(const uint64_t *codes, unsigned n, int shift,
-                             uint32_t *flag) {
-  unsigned i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  flag[codes[i] >> shift] = 1u;
 }
 
 // ---- box ranges and box lists of all levels of a tree at once ----------------
@@ -990,8 +982,7 @@ int wbfmm_hip_box_ranges(const uint64_t *codes, unsigned n, unsigned level,
 }
 
 int wbfmm_hip_compact_boxes(const uint32_t *start, const uint32_t *end,
-                            const uint32_t *flag, unsigned level,
-                            uint32_t *list, unsigned *count) {
+                            unsigned level, uint32_t *list, unsigned *count) {
   unsigned nb = 1u << (3 * level);
   uint32_t *flags = nullptr, *pos = nullptr;
   void *tmp = nullptr;
@@ -999,7 +990,7 @@ int wbfmm_hip_compact_boxes(const uint32_t *start, const uint32_t *end,
       dmalloc((void **)&pos, sizeof(uint32_t) * nb))
     return WBFMM_HIP_ERR_NOMEM;
   WBFMM_LAUNCH("tree_box_flags", k_box_flags, dim3(nblk(nb, 256)), dim3(256),
-               0, start, end, flag, nb, flags);
+               0, start, end, nb, flags);
   size_t bytes = 0;
   WBFMM_CHECK(rocprim::exclusive_scan(nullptr, bytes, flags, pos, 0u, nb,
                                       rocprim::plus<uint32_t>(), stream()));
@@ -1171,14 +1162,6 @@ int wbfmm_hip_accumulate(double *dst, int dstr, const double *src, int sstr,
   if (dstr < ncomp || sstr < ncomp) return WBFMM_HIP_ERR_ARG;
   WBFMM_LAUNCH("accumulate", k_accumulate, dim3(nblk(n, 256)), dim3(256), 0,
                dst, dstr, src, sstr, ncomp, n);
-  return 0;
-}
-
-int wbfmm_hip_mark_boxes(const uint64_t *codes, unsigned n, unsigned level,
-                         uint32_t *flag) {
-  if (n == 0) return 0;
-  WBFMM_LAUNCH("tree_mark_boxes", k_mark_boxes, dim3(nblk(n, 256)),
-               dim3(256), 0, codes, n, (int)(3 * (20 - level)), flag);
   return 0;
 }
 

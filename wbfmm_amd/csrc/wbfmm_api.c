@@ -1693,8 +1693,8 @@ static void stage_targets(const void *xt, size_t tstr, unsigned n,
                           const double *x0, double D, int depth, int sort_them)
 {
   unsigned nbad = 0;
-  double *raw;
-  HIPOK(wbfmm_hip_malloc((void **)&raw, sizeof(double) * 4 * (n ? n : 1)));
+  double *raw = NULL;
+  if (sort_them) HIPOK(wbfmm_hip_malloc((void **)&raw, sizeof(double) * 4 * (n ? n : 1)));
   HIPOK(wbfmm_hip_malloc((void **)dx, sizeof(double) * 4 * (n ? n : 1)));
   HIPOK(wbfmm_hip_malloc((void **)did, sizeof(uint32_t) * (n ? n : 1)));
   HIPOK(wbfmm_hip_malloc((void **)dcodes, sizeof(uint64_t) * (n ? n : 1)));
@@ -3126,7 +3126,7 @@ gint wbfmm_downward_pass_avx(wbfmm_tree_t *t, wbfmm_shift_operators_t *op,
   return hel_downward(t, op, level);
 }
 
-/* the field kernels: one thread per target (FP64 or mixed), or one
+/* the field kernels: 1 to 16 lanes per target (FP64 or mixed), or one
    wavefront per target box (WBFMM_HEL_FIELD=box, kept for comparison:
    slower on leaves of a few tens of targets) */
 static int hel_field_box64(void)
@@ -3164,7 +3164,7 @@ static void hel_field_run(tree_dev *td, double k, const double *dxt,
   nelem = nf_rows ? (nf_rows - 1) * (size_t)fstr + ((fl & 1) ? 2 : 0) + ((fl & 2) ? 6 : 0) : 0;
   df = field_begin(f, nelem, &staged);
   if (f32 && !hel_field_box64()) {
-    /* mixed precision, one thread per target */
+    /* mixed precision, 1 to 16 lanes per target */
     HIPOK(wbfmm_hip_hel_field_f32(dxt, dtid, n, td->d_start[lv], td->d_end[lv], td->d_xyz, q,
                                   dp ? td->d_nrm : NULL, dp, lv, ORIGIN(t), t->D,
                                   t->order_r[lv], k, (const float *)t->mpr[lv], td->d_hsc[lv],
@@ -3178,7 +3178,7 @@ static void hel_field_run(tree_dev *td, double k, const double *dxt,
     HIPOK(wbfmm_hip_malloc((void **)&te, sizeof(uint32_t) * nb));
     HIPOK(wbfmm_hip_malloc((void **)&tb, sizeof(uint32_t) * nb));
     HIPOK(wbfmm_hip_box_ranges(dcodes, n, lv, ts, te));
-    HIPOK(wbfmm_hip_compact_boxes(ts, te, NULL, lv, tb, &ntb));
+    HIPOK(wbfmm_hip_compact_boxes(ts, te, lv, tb, &ntb));
     HIPOK(wbfmm_hip_hel_field_box(tb, ntb, ts, te, dxt, dtid, td->d_start[lv], td->d_end[lv],
                                   td->d_xyz, q, dp ? td->d_nrm : NULL, dp, lv, ORIGIN(t), t->D,
                                   t->order_r[lv], k, f32 ? 32 : 64, t->mpr[lv],
