@@ -163,23 +163,27 @@ def test_address_that_comes_back_with_another_size(wb, lib, foreign):
     s, pool = _vp(), _vp()
     assert hip.hipStreamCreate(ctypes.byref(s)) == 0
     assert hip.hipDeviceGetDefaultMemPool(ctypes.byref(pool), 0) == 0
-    hip.hipMemPoolTrimTo(pool, ctypes.c_size_t(0))
-    a = take(lib, 2 * MIB)
-    wb.sync()
-    assert hip.hipFree(_vp(a)) == 0
-    hip.hipMemPoolTrimTo(pool, ctypes.c_size_t(0))
-    lib.wbfmm_hip_set_stream(s if foreign else None, None)
-    ps = [take(lib, MIB) for _ in range(8)]
-    lib.wbfmm_hip_set_stream(None, None)
-    assert hip.hipStreamSynchronize(s) == 0
-    back = a in ps
-    if back:
-        lib.wbfmm_hip_free(a)
-        assert lib.wbfmm_hip_pool_bytes() == (0 if foreign else MIB)
-    for p in ps:
-        if p != a:
-            lib.wbfmm_hip_free(p)
-    wb.sync()
+    back = False
+    for size in (2 * MIB, 16 * MIB, MIB // 4, 6 * MIB, 48 * MIB, MIB):
+        hip.hipMemPoolTrimTo(pool, ctypes.c_size_t(0))
+        a = take(lib, size)
+        wb.sync()
+        assert hip.hipFree(_vp(a)) == 0
+        hip.hipMemPoolTrimTo(pool, ctypes.c_size_t(0))
+        lib.wbfmm_hip_set_stream(s if foreign else None, None)
+        ps = [take(lib, size // 2) for _ in range(8)]
+        lib.wbfmm_hip_set_stream(None, None)
+        assert hip.hipStreamSynchronize(s) == 0
+        if a in ps:
+            back = True
+            lib.wbfmm_hip_free(a)
+            assert lib.wbfmm_hip_pool_bytes() == (0 if foreign else size // 2)
+        for p in ps:
+            if p != a:
+                lib.wbfmm_hip_free(p)
+        wb.sync()
+        lib.wbfmm_hip_pool_release()
+        wb.sync()
     assert hip.hipStreamDestroy(s) == 0
     if not back:
         pytest.skip("the runtime gave the address to no later block")
