@@ -54,7 +54,7 @@ void *wbfmm_hip_get_stream(void);
      hold targets): 0 chunks of targets running every offset, 1 tiles of
      one offset (Laplace FP64; Helmholtz: as 2), 2 tiles of one offset
      class (the default);
-   - WBFMM_VARIANT_FIELD (Helmholtz L2P + P2P): 0 one thread per target
+   - WBFMM_VARIANT_FIELD (Helmholtz L2P + P2P): 0 lanes per target
      (the default), 1 one wavefront per target box with the neighbours'
      sources staged through LDS. */
 #define WBFMM_VARIANT_M2L 0
@@ -642,7 +642,7 @@ int wbfmm_hip_hel_shift_mfma_f32(int mode, const uint32_t *parents, unsigned npa
                                  const uint32_t *cflag, int N, const float *in, float *out,
                                  const void *plan_dev, const float *A, const float *A2,
                                  const float *CS, const wbfmm_m2l_plan_t *plan_host);
-/* mixed-precision L2P + near field with one thread per target (the form
+/* mixed-precision L2P + near field with 1 to 16 lanes per target (the form
    of wbfmm_hip_hel_field): FP32 local expansions holding L_n^m s_n
    (scale: the level's s_n, FP64), FP64 regular functions and L2P sums,
    FP32 near-field kernel with compensated sums (src/local.c:32-310) */

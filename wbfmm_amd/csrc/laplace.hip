@@ -1396,13 +1396,16 @@ int wbfmm_hip_lap_field_leaves(const double *xt, const uint32_t *tid, unsigned n
                            1.0, (const double *)mpr, field, f, fstr, nleaf);
 }
 
+// boxes of a level, as many as the type holds
+static unsigned level_boxes(unsigned level) { return level <= 10 ? 1u << (3 * level) : ~0u; }
+
 int wbfmm_hip_lap_field(const double *xt, const uint32_t *tid, unsigned n,
                         const uint32_t *start, const uint32_t *end,
                         const double *xyz, const double *q, const double *nrm,
                         const double *dip, unsigned level, const double *x0,
                         double D, int N, const double *mpr, int field,
                         double *f, int fstr) {
-  return wbfmm_hip_lap_field_leaves(xt, tid, n, 1u << (3 * level), start, end, xyz, q, nrm, dip,
+  return wbfmm_hip_lap_field_leaves(xt, tid, n, level_boxes(level), start, end, xyz, q, nrm, dip,
                                     level, x0, D, N, 0, mpr, field, f, fstr);
 }
 
@@ -1412,7 +1415,7 @@ int wbfmm_hip_lap_field_f32(const double *xt, const uint32_t *tid, unsigned n,
                             const double *dip, unsigned level, const double *x0,
                             double D, int N, const float *mpr, int field,
                             double *f, int fstr) {
-  return wbfmm_hip_lap_field_leaves(xt, tid, n, 1u << (3 * level), start, end, xyz, q, nrm, dip,
+  return wbfmm_hip_lap_field_leaves(xt, tid, n, level_boxes(level), start, end, xyz, q, nrm, dip,
                                     level, x0, D, N, 1, mpr, field, f, fstr);
 }
 
