@@ -63,14 +63,30 @@ def test_bounded(wb, lib):
 
 
 def test_bounded_in_number(wb, lib):
-    """an allocation looks through the kept blocks: there are few of them,
-    however small they are"""
-    ps = [take(lib, 4096) for _ in range(5000)]
+    """however small they are, at most 16384 blocks are kept, the last freed"""
+    ps = [take(lib, 4096) for _ in range(20000)]
     for p in ps:
         lib.wbfmm_hip_free(p)
-    assert 0 < lib.wbfmm_hip_pool_bytes() <= 2048 * 4096
+    assert lib.wbfmm_hip_pool_bytes() == 16384 * 4096
     a = take(lib, 4096)
-    assert a in ps[-2048:]
+    assert a in ps[-16384:]
+    lib.wbfmm_hip_free(a)
+
+
+def test_smallest_that_fits(wb, lib):
+    """of the kept blocks the smallest that holds the request, no more than a
+    quarter and a page larger, whatever the order they were freed in"""
+    sizes = [40, 10, 24, 12, 30, 11]
+    ps = {m: take(lib, m * MIB) for m in sizes}
+    for p in ps.values():
+        lib.wbfmm_hip_free(p)
+    for want, got in ((11, 11), (11, 12), (20, 24), (25, 30), (35, 40), (9, 10)):
+        assert take(lib, want * MIB) == ps[got]
+    assert lib.wbfmm_hip_pool_bytes() == 0
+    for p in ps.values():
+        lib.wbfmm_hip_free(p)
+    a = take(lib, 15 * MIB)                                # 24 is too large
+    assert a not in ps.values()
     lib.wbfmm_hip_free(a)
 
 
